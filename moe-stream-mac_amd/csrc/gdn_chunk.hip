@@ -1217,6 +1217,17 @@ __global__ __launch_bounds__(NTB) void ck_bwd_local_bf16_kernel(Args a) {
 // ahead (ck_prep wrote them as bf16 tiles); LDS only carries what the waves exchange each chunk: h as the
 // operand [i][j] (hi / lo) and Delta as [i][r] (hi / lo).  Two barriers per chunk.
 
+// Reading ahead (slices narrower than 64).  The D / VS workgroups of a head ask for the same tiles at the same time,
+// so a line that is not in L2 yet is missed by each of them, and the loads of the next chunk, issued one step ahead,
+// come back late: with tiles that outgrow the Infinity Cache a step took 3.0 us against 1.7 us within it.  Each slice
+// therefore reads one 4-byte word of its own share (1 / (D / VS)) of the shared lines of the chunk kReadAhead steps on
+// (at most one load per thread and step), so each line leaves memory once and the fragment loads hit L2.  At B = 1,
+// T = 4001, Hv = 32: ck_fwd_bf16 188 -> 166 us, ck_bwd_seq_bf16 170 -> 152 us; at B = 2, T = 2048: 148 -> 129 and
+// 135 -> 125 us; three, four and six steps ahead gain less (170, 179, 184 us forward at B = 1).  At 64-wide slices the
+// kernels have no register to spare for it (forward at B = 4: 346 -> 373 us).  Args::read_ahead says whether the
+// launch's tiles outgrow the cache.
+constexpr int kReadAhead = 2, kLine = 128;  // bytes of an L2 line
+
 template <int DN>
 struct FwdFrags {
     bf8 W[4], Q[4], P[4], K[2];  // P[0..1] hi, P[2..3] lo
@@ -1295,6 +1306,28 @@ __global__ __launch_bounds__(NTS) void ck_fwd_bf16_kernel(Args a) {
         if constexpr (VG) f.gc = *reinterpret_cast<const float4 *>(a.w.Gv + (ci * C + C - 1) * D + 16 * w + 4 * lg);
         else f.g = tid < C ? a.w.G[ci * C + tid] : 0.0;
     };
+    uint32_t ahead = 0;
+    auto read_ahead = [&](int c) {
+        // threads below LPS: this slice's share of the 512 lines of W, (K diag(gamma_C / gamma))^T, P and Q; threads
+        // 256..: the slice's own blocks of U (accumulator order: VS / 16 blocks of 1 KiB per 16-row strip)
+        constexpr int S = D / VS, LPS = 4 * kLine / S, ULN = VS / 2;
+        const size_t ci = head * a.NC + c;
+        const char *p = nullptr;
+        if (tid < LPS) {
+            const int i = sb.slice * LPS + tid, tile = i / kLine, ln = i % kLine;  // each tile is 128 lines
+            if (tile == 0) p = reinterpret_cast<const char *>(a.w.Wb + ci * C * D) + kLine * ln;
+            else if (tile == 1) p = reinterpret_cast<const char *>(a.w.KTb + ci * D * C) + kLine * ln;
+            else if (tile == 2) p = reinterpret_cast<const char *>(a.w.Pb + ci * 2 * C * C) + kLine * ln;
+            else if (VG) p = reinterpret_cast<const char *>(a.w.QGb + ci * C * D) + kLine * ln;
+            else p = reinterpret_cast<const char *>(static_cast<const bfr *>(a.q) +
+                                                    (((size_t)b * a.Ts + min(c * C + ln / 2, T - 1)) * a.Hk + hk) * D) +
+                     kLine * (ln & 1);
+        } else if (tid >= 256 && tid < 256 + 4 * ULN) {
+            const int i = tid - 256, m = i / ULN;
+            p = reinterpret_cast<const char *>(a.w.U + ci * C * D + acc_off(16 * m, i0)) + kLine * (i - m * ULN);
+        }
+        if (p) ahead = *reinterpret_cast<const uint32_t *>(p);
+    };
     // The chunk loop is unrolled by two over ping-pong fragment buffers: no register copy of the prefetched
     // fragments, so the wait for them sits at their first use, one chunk step after the loads were issued.
     auto step = [&](const int c, FwdFrags<DN> &cur, FwdFrags<DN> &nxt) {
@@ -1315,7 +1348,9 @@ __global__ __launch_bounds__(NTS) void ck_fwd_bf16_kernel(Args a) {
         float *const sGam = sGamBuf[c & 1];
         if (!VG && tid < C) sGam[tid] = __builtin_amdgcn_exp2f((float)(cur.g * 1.4426950408889634));  // v_exp_f32 on log2 units
         __syncthreads();
+        if constexpr (VS < 64) asm volatile("" ::"v"(ahead));  // the previous step's read
         if (c + 1 < ce) fetch(nxt, c + 1);
+        if (VS < 64 && a.read_ahead && c + kReadAhead < ce) read_ahead(c + kReadAhead);
         // Delta = U - W h ; Yi = Q h
         f4 yi[DN];
 #pragma unroll
@@ -1771,6 +1806,31 @@ __global__ __launch_bounds__(NTS) void ck_bwd_seq_bf16_kernel(Args a) {
             }
         }
     };
+    uint32_t ahead = 0;
+    auto read_ahead = [&](int c) {
+        // threads below LPS: this slice's share of the 640 lines of P^T, Q^T, -W^T, T^T and K; threads 384..447: dY's
+        // rows of the slice
+        constexpr int S = D / VS, LPS = 5 * kLine / S;
+        static_assert(VS >= 64 || LPS <= 384, "the two groups of threads are apart");
+        const size_t ci = head * a.NC + c;
+        const char *p = nullptr;
+        if (tid < LPS) {
+            const int i = sb.slice * LPS + tid, tile = i / kLine, ln = i % kLine;  // each tile is 128 lines
+            if (tile == 0) p = reinterpret_cast<const char *>(a.w.PTb + ci * 2 * C * C) + kLine * ln;
+            else if (tile == 1)
+                p = reinterpret_cast<const char *>(a.w.QTb + (VG ? ci : ((size_t)b * a.Hk + hk) * a.NC + c) * D * C) + kLine * ln;
+            else if (tile == 2) p = reinterpret_cast<const char *>(a.w.nWTb + ci * D * C) + kLine * ln;
+            else if (tile == 3) p = reinterpret_cast<const char *>(reinterpret_cast<const bfr *>(a.w.T) + ci * 2 * C * C) + kLine * ln;
+            else if (VG) p = reinterpret_cast<const char *>(a.w.KDb + ci * C * D) + kLine * ln;
+            else p = reinterpret_cast<const char *>(static_cast<const bfr *>(a.k) +
+                                                    (((size_t)b * a.Ts + min(c * C + ln / 2, T - 1)) * a.Hk + hk) * D) +
+                     kLine * (ln & 1);
+        } else if (tid >= 384 && tid < 384 + C) {
+            const size_t off = (((size_t)b * a.Ts + min(c * C + tid - 384, T - 1)) * a.Hv + hv) * D + i0;
+            p = static_cast<const char *>(a.dy) + off * (DYF32 ? 4 : 2);
+        }
+        if (p) ahead = *reinterpret_cast<const uint32_t *>(p);
+    };
     // unrolled by two over ping-pong fragment buffers, as in ck_fwd_bf16_kernel; both steps of a pair are
     // unconditional (a prefetch used only under a branch is sunk to its use by the compiler)
     YRaw yr[8];
@@ -1830,7 +1890,9 @@ __global__ __launch_bounds__(NTS) void ck_bwd_seq_bf16_kernel(Args a) {
         // first barrier of this one); the next chunk's pieces are loaded after the second barrier
         reinterpret_cast<uint4 *>(sTT)[tid] = ttr0;
         reinterpret_cast<uint4 *>(sTT)[tid + NTS] = ttr1;
+        if constexpr (VS < 64) asm volatile("" ::"v"(ahead));  // the previous step's read
         if (c > 0) fetch(nxt, yr, c - 1);
+        if (VS < 64 && a.read_ahead && c >= kReadAhead) read_ahead(c - kReadAhead);
         // dDelta = diag(rc) K dh' + P^T dY
         if (cwave) {
             f4 kd[DN], pd[DN];
@@ -1956,6 +2018,12 @@ ChunkSizes chunk_sizes(int B, int T, int Hk, int Hv, bool bf16, bool bwd, int vg
     return s;
 }
 
+// The tile set of a launch from which the sequential kernels read ahead (kReadAhead): tiles that ck_prep has just left
+// in the 256 MiB Infinity Cache come fast enough without, and the extra loads cost.  Whole passes with / without, at
+// Hv = 32: tile set 150 MiB (T = 1536) 200 / 201 us, 175 MiB (T = 1792) 234 / 249 us, 200 MiB (T = 2048) 262 / 286 us;
+// a forward-only group (161 MiB) 178 / 172 us at B = 1.
+constexpr size_t kReadAheadBytes = (size_t)168 << 20;
+
 static ck::Args make_args(const ChunkCall &cc) {
     ck::Args a{};
     a.q = cc.q; a.k = cc.k; a.v = cc.v; a.g = cc.g; a.beta = cc.beta; a.state0 = cc.state0;
@@ -1992,6 +2060,7 @@ static ck::Args make_args(const ChunkCall &cc) {
     a.B = cc.B; a.T = cc.T; a.Ts = cc.Ts; a.Hk = cc.Hk; a.Hv = cc.Hv; a.NC = (cc.T + CK_C - 1) / CK_C;
     a.in_dt = cc.in_dt; a.out_dt = cc.out_dt; a.dy_dt = cc.dy_dt; a.grad_dt = cc.grad_dt; a.gate = cc.gate;
     a.snap = cc.snap; a.wc = cc.wc; a.win0 = cc.win0; a.recompute = cc.recompute; a.fwd_only = cc.fwd_only;
+    a.read_ahead = s.saved >= kReadAheadBytes;
     return a;
 }
 

@@ -297,6 +297,7 @@ struct Args {
     float *snap;
     int wc, win0, recompute;
     int fwd_only;  // forward-only: ck_prep writes only the tiles the sequential forward reads
+    int read_ahead;  // the launch's tiles outgrow the Infinity Cache: the sequential kernels read them ahead into L2
 };
 
 __device__ __forceinline__ size_t chunk_index(const Args &a, int b, int hv, int c) {
