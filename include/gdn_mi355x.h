@@ -54,8 +54,8 @@ enum gdn_gate {
 enum gdn_form {
     GDN_FORM_AUTO = 0,       /* the chunked form when eligible, else the recurrent form */
     GDN_FORM_RECURRENT = 1,  /* token-sequential recurrence, state rows resident in VGPRs; any shape */
-    GDN_FORM_CHUNK = 2       /* chunked WY/UT form on MFMA (64-token tiles); Dk = Dv = 128, scalar gate; a mask runs
-                                two chunked passes (see below) */
+    GDN_FORM_CHUNK = 2       /* chunked WY/UT form on MFMA (64-token tiles); Dk = Dv = 128, scalar gate; masks:
+                                see below */
 };
 
 /* Library version, (major << 16) | minor. */
@@ -100,10 +100,9 @@ int gdn_select_form(int Hv, int Dk, int Dv, int has_mask, int gate_kind, int for
  * minimum. */
 
 /* Masks on the chunked form.  A masked step keeps the state but its output reads the candidate state.  The chunked
- * form runs the recurrence with decay 1 and beta 0 at masked tokens (the same states), once with q and once with k as
- * the query, and rewrites y at masked tokens as decay y' + beta (k . q) (v - decay z) from the two outputs; the
- * backward runs both passes' backwards and the rewrite's VJP.  Needs Hv <= 256; the saved buffer holds both passes
- * (checkpointing: pass 1's snapshots serve both) plus fp32 [B][T][Hv][Dv] copies of the two outputs. */
+ * form runs the recurrence once, with decay 1 and beta 0 at masked tokens (the same states); a masked token's query is
+ * decay (q - beta (k . q) k), one per value head, and beta (k . q) v is added to its y.  Needs Hv <= 256; the saved
+ * buffer also holds the effective gates and those queries (4 bytes per (token, value head, key channel)). */
 
 /* Size of the buffer gdn_fwd fills for gdn_bwd (the "saved" activations) for inputs of in_dtype. */
 size_t gdn_saved_bytes(int B, int T, int Hk, int Hv, int Dk, int Dv, int chunk, int gate_kind, int has_mask,

@@ -104,8 +104,7 @@ static int check_shape(int B, int T, int Hk, int Hv, int Dk, int Dv, int chunk, 
     return GDN_OK;
 }
 
-// Masked calls run the chunked form as two passes (gdn_mask.hip), whose fix-up kernels hold per-head values of one
-// token in LDS: Hv <= mask_max_heads().  Per-channel gates run on the chunked form with bf16 inputs and no mask
+// Masked calls run on the chunked form (gdn_mask.hip) up to mask_max_heads() value heads.  Per-channel gates run on the chunked form with bf16 inputs and no mask
 // (gdn_chunk_vg.hip).
 static bool chunk_eligible(int Hv, int Dk, int Dv, int has_mask, int gate, int in_dt) {
     if (Dk != 128 || Dv != 128) return false;
@@ -182,17 +181,22 @@ struct CkShape {
     int B, T, Hk, Hv;
     bool bf16;
     int vg;  // vg_kind of the gate: 0 one decay per head, 1 per-channel log decays, 2 per-channel decays
+    bool masked;
 };
+
+static ChunkSizes ck_sizes(const CkShape &s, int T, bool bwd) {
+    return chunk_sizes(s.B, T, s.Hk, s.Hv, s.bf16, bwd, s.vg, s.masked);
+}
 
 // Forward group workspace: the forward tile set of Tg tokens, plus two carried states between groups when no
 // snapshots carry them.
 static size_t ck_fwd_group_bytes(const CkShape &s, int Tg, bool ckpt) {
-    return chunk_sizes(s.B, Tg, s.Hk, s.Hv, s.bf16, false, s.vg).saved + (ckpt ? 0 : 2 * align256(ck_state_bytes(s.B, s.Hv)));
+    return ck_sizes(s, Tg, false).saved + (ckpt ? 0 : 2 * align256(ck_state_bytes(s.B, s.Hv)));
 }
 
 // Backward group workspace: two carried state adjoints, the whole tile set and the backward buffers of Tg tokens.
 static size_t ck_bwd_group_bytes(const CkShape &s, int Tg) {
-    const ChunkSizes cs = chunk_sizes(s.B, Tg, s.Hk, s.Hv, s.bf16, true, s.vg);
+    const ChunkSizes cs = ck_sizes(s, Tg, true);
     return 2 * align256(ck_state_bytes(s.B, s.Hv)) + align256(cs.saved) + cs.work;
 }
 
@@ -219,56 +223,35 @@ static size_t ck_bwd_target_bytes(const CkShape &s, int W) {
     return ck_bwd_group_bytes(s, std::min(g * W, s.T));
 }
 
-// ---- masked calls on the chunked form: two chunked passes over the effective gates (gdn_mask.hip)
-//
-// saved (training): pass 1's saved buffer (tiles or snapshots), pass 2's tiles (chunk <= 64 only: checkpointing
-// rebuilds pass 2 from pass 1's snapshots, the state sequences being the same), the effective gates g', beta', and
-// z and y' (fp32 [B][T][Hv][Dv], read at masked tokens).
-struct MaskSaved {
-    size_t p1, p2, g2, b2, Z, Yp, total;
+// ---- masked calls on the chunked form (gdn_mask.hip): what mask_query_kernel writes and the chunked kernels read, the
+// effective gates g', beta', the masked tokens' queries (fp32, or bf16 hi and lo planes) and value factors, and the chunk
+// flags.  A training call keeps them behind the tiles or snapshots, a forward-only call at the head of its workspace.
+struct MaskBufs {
+    size_t g2, b2, e, qm, cm, total;
 };
-static MaskSaved mask_saved(const CkShape &s, int chunk) {
-    const int W = ck_window(chunk);
-    const size_t tiles = chunk_sizes(s.B, s.T, s.Hk, s.Hv, s.bf16, true, s.vg).saved;
-    const size_t ng = (size_t)s.B * s.T * s.Hv * 4, nv = ng * kChunkD;
-    MaskSaved m{};
+static MaskBufs mask_bufs(const CkShape &s) {
+    const size_t ng = (size_t)s.B * s.T * s.Hv * 4;
+    MaskBufs m{};
     size_t off = 0;
-    m.p1 = off; off += align256(W ? ck_snap_bytes(s.B, s.T, s.Hv, W) : tiles);
-    m.p2 = off; off += align256(W ? 0 : tiles);
     m.g2 = off; off += align256(ng);
     m.b2 = off; off += align256(ng);
-    m.Z = off; off += align256(nv);
-    m.Yp = off; off += align256(nv);
+    m.e = off; off += align256(ng);
+    m.qm = off; off += align256(ng * kChunkD);
+    m.cm = off; off += align256((size_t)s.B * ((s.T + kChunkC - 1) / kChunkC));
     m.total = off;
     return m;
 }
-
-// Backward workspace: one pass's workspace (used by both passes in turn), the passes' cotangents and their fp32
-// gradients.
-struct MaskWork {
-    size_t pass, pass_bytes, dy1, dz, g1[6], g2[6], total;  // g1 / g2: dq, dk, dv, dg, dbeta, dS0
-};
-static MaskWork mask_work(const CkShape &s, int chunk) {
+static size_t mask_tiles_bytes(const CkShape &s, int chunk) {
     const int W = ck_window(chunk);
-    MaskWork m{};
-    m.pass_bytes = W ? ck_bwd_target_bytes(s, W) : chunk_sizes(s.B, s.T, s.Hk, s.Hv, s.bf16, true, s.vg).work;
-    const size_t nqk = (size_t)s.B * s.T * s.Hk * kChunkD * 4, ng = (size_t)s.B * s.T * s.Hv * 4, nv = ng * kChunkD;
-    const size_t nst = ck_state_bytes(s.B, s.Hv);
-    const size_t sizes[6] = {nqk, nqk, nv, ng, ng, nst};
-    size_t off = 0;
-    m.pass = off; off += align256(m.pass_bytes);
-    m.dy1 = off; off += align256(nv);
-    m.dz = off; off += align256(nv);
-    for (int i = 0; i < 6; ++i) { m.g1[i] = off; off += align256(sizes[i]); }
-    for (int i = 0; i < 6; ++i) { m.g2[i] = off; off += align256(sizes[i]); }
-    m.total = off;
-    return m;
+    return align256(W ? ck_snap_bytes(s.B, s.T, s.Hv, W) : ck_sizes(s, s.T, true).saved);
 }
-
-// Forward-only workspace: g', beta', z, then the group workspace.
-static size_t mask_fwd_only_head(const CkShape &s) {
-    const size_t ng = (size_t)s.B * s.T * s.Hv * 4;
-    return 2 * align256(ng) + align256(ng * kChunkD);
+// Backward workspace of the chunked stages; a masked call puts dL/dq~ (fp32 [B][T][Hv][Dk]) behind it.
+static size_t mask_stage_bytes(const CkShape &s, int chunk) {
+    const int W = ck_window(chunk);
+    return align256(W ? ck_bwd_target_bytes(s, W) : ck_sizes(s, s.T, true).work);
+}
+static size_t mask_work_bytes(const CkShape &s, int chunk) {
+    return mask_stage_bytes(s, chunk) + align256((size_t)s.B * s.T * s.Hv * kChunkD * 4);
 }
 
 static size_t dt_size(int dt) { return dt == DT_F32 ? 4 : 2; }
@@ -351,9 +334,10 @@ size_t gdn_saved_bytes(int B, int T, int Hk, int Hv, int Dk, int Dv, int chunk, 
     if (f < 0 || B == 0 || T == 0) return 0;
     if (f == GDN_FORM_CHUNK) {
         const int W = ck_window(chunk);
-        if (has_mask) return mask_saved({B, T, Hk, Hv, in_dtype == DT_BF16, false}, chunk).total;
+        const CkShape shp{B, T, Hk, Hv, in_dtype == DT_BF16, vg_kind(gate_kind), has_mask != 0};
+        if (has_mask) return mask_tiles_bytes(shp, chunk) + mask_bufs(shp).total;
         if (W) return ck_snap_bytes(B, T, Hv, W);
-        return chunk_sizes(B, T, Hk, Hv, in_dtype == DT_BF16, true, vg_kind(gate_kind)).saved;
+        return ck_sizes(shp, T, true).saved;
     }
     return rec_saved_bytes(B, T, Hv, Dk, Dv, chunk);
 }
@@ -364,29 +348,35 @@ size_t gdn_fwd_workspace_bytes(int B, int T, int Hk, int Hv, int Dk, int Dv, int
     const int f = resolve_form(Hv, Dk, Dv, has_mask, gate_kind, form, in_dtype);
     if (f != GDN_FORM_CHUNK || B == 0 || T == 0) return 0;
     const int W = ck_window(chunk);
-    const CkShape shp{B, T, Hk, Hv, in_dtype == DT_BF16, vg_kind(gate_kind)};
-    if (has_mask) {
-        // pass 2 runs forward-only when checkpointing; a forward-only call also holds g', beta' and z
-        if (with_saved) return W ? std::max(ck_fwd_target_bytes(shp, W, true), ck_fwd_target_bytes(shp, W, false)) : 0;
-        return mask_fwd_only_head(shp) + ck_fwd_target_bytes(shp, W, false);
-    }
+    const CkShape shp{B, T, Hk, Hv, in_dtype == DT_BF16, vg_kind(gate_kind), has_mask != 0};
     if (with_saved && !W) return 0;
-    return ck_fwd_target_bytes(shp, W, with_saved != 0);
+    return ck_fwd_target_bytes(shp, W, with_saved != 0) + (has_mask && !with_saved ? mask_bufs(shp).total : 0);
 }
 
 }  // extern "C"
 
 namespace gdn {
 
+// A masked call's pointers moved to token ts (a multiple of the chunk).
+static void offset_mask(ChunkCall &cc, int ts) {
+    if (!cc.mask) return;
+    const size_t th = (size_t)ts * cc.Hv;
+    cc.mask += ts;
+    cc.cm += ts / kChunkC;
+    cc.qm = tok_offset(cc.qm, th * kChunkD, cc.in_dt == DT_BF16 ? DT_BF16 : DT_F32);
+    cc.e += th;
+    if (cc.xm) cc.xm += th * kChunkD;
+}
+
 // Chunked forward (resolved form GDN_FORM_CHUNK, arguments checked).
 static int ck_forward(const ChunkCall &base, int chunk, void *saved, size_t saved_bytes, void *ws, size_t ws_bytes,
                       hipStream_t st) {
     const int B = base.B, T = base.T, Hk = base.Hk, Hv = base.Hv;
-    const CkShape shp{B, T, Hk, Hv, base.in_dt == DT_BF16, vg_kind(base.gate)};
+    const CkShape shp{B, T, Hk, Hv, base.in_dt == DT_BF16, vg_kind(base.gate), base.mask != nullptr};
     const int W = ck_window(chunk);
     int rc;
     if (saved && !W) {  // the whole tile set, kept for the backward
-        const size_t need = chunk_sizes(B, T, Hk, Hv, shp.bf16, true, shp.vg).saved;
+        const size_t need = ck_sizes(shp, T, true).saved;
         if (saved_bytes < need)
             return fail(GDN_ERR_WORKSPACE, "saved buffer of %zu bytes is smaller than the %zu bytes required",
                         saved_bytes, need);
@@ -434,6 +424,7 @@ static int ck_forward(const ChunkCall &base, int chunk, void *saved, size_t save
         cc.g = base.g + (size_t)ts * Hv * gate_width(base.gate);
         cc.beta = base.beta + (size_t)ts * Hv;
         cc.y = tok_offset(base.y, (size_t)ts * Hv * kChunkD, base.out_dt);
+        offset_mask(cc, ts);
         cc.T = Tg;
         cc.Ts = T;
         cc.tiles = w8;
@@ -467,11 +458,11 @@ static int ck_forward(const ChunkCall &base, int chunk, void *saved, size_t save
 static int ck_backward(const ChunkCall &base, int chunk, const void *saved, size_t saved_bytes, void *ws,
                        size_t ws_bytes, hipStream_t st) {
     const int B = base.B, T = base.T, Hk = base.Hk, Hv = base.Hv;
-    const CkShape shp{B, T, Hk, Hv, base.in_dt == DT_BF16, vg_kind(base.gate)};
+    const CkShape shp{B, T, Hk, Hv, base.in_dt == DT_BF16, vg_kind(base.gate), base.mask != nullptr};
     const int W = ck_window(chunk);
     int rc;
     if (!W) {
-        const ChunkSizes cs = chunk_sizes(B, T, Hk, Hv, shp.bf16, true, shp.vg);
+        const ChunkSizes cs = ck_sizes(shp, T, true);
         if (!saved || saved_bytes < cs.saved)
             return fail(GDN_ERR_INVALID, "the saved buffer written by gdn_fwd (%zu bytes) is required", cs.saved);
         if (!ws || ws_bytes < cs.work)
@@ -508,7 +499,7 @@ static int ck_backward(const ChunkCall &base, int chunk, const void *saved, size
     const size_t sb = align256(ck_state_bytes(B, Hv));
     char *w8 = static_cast<char *>(ws);
     float *carry[2] = {reinterpret_cast<float *>(w8), reinterpret_cast<float *>(w8 + sb)};
-    const ChunkSizes full = chunk_sizes(B, std::min(Gt, T), Hk, Hv, shp.bf16, true, shp.vg);
+    const ChunkSizes full = ck_sizes(shp, std::min(Gt, T), true);
     char *tiles = w8 + 2 * sb, *work = tiles + align256(full.saved);
     for (int g = ng - 1; g >= 0; --g) {
         const int ts = g * Gt, Tg = std::min(Gt, T - ts);
@@ -525,6 +516,7 @@ static int ck_backward(const ChunkCall &base, int chunk, const void *saved, size
         cc.dv = tok_offset(base.dv, vv, base.grad_dt);
         cc.dg = base.dg + (size_t)ts * Hv * gate_width(base.gate);
         cc.dbeta = base.dbeta + (size_t)ts * Hv;
+        offset_mask(cc, ts);
         cc.T = Tg;
         cc.Ts = T;
         cc.tiles = tiles;
@@ -570,141 +562,89 @@ static int ck_backward(const ChunkCall &base, int chunk, const void *saved, size
 
 static char *at_off(void *base, size_t off) { return static_cast<char *>(base) + off; }
 
+static MaskArgs mask_args(const ChunkCall &base, const uint8_t *mask) {
+    MaskArgs ma{};
+    ma.q = base.q; ma.k = base.k; ma.v = base.v; ma.dy = base.dy; ma.g = base.g; ma.beta = base.beta; ma.mask = mask;
+    ma.dq = base.dq; ma.dk = base.dk; ma.dv = base.dv; ma.dg = base.dg; ma.dbeta = base.dbeta;
+    ma.B = base.B; ma.T = base.T; ma.Hk = base.Hk; ma.Hv = base.Hv; ma.Dk = kChunkD; ma.Dv = kChunkD;
+    ma.in_dt = base.in_dt; ma.dy_dt = base.dy_dt; ma.grad_dt = base.grad_dt; ma.gate = base.gate;
+    return ma;
+}
+
+// The chunked call over the effective gates and the masked tokens' queries in bufs (mask_bufs).
+static ChunkCall masked_call(const ChunkCall &base, const uint8_t *mask, const MaskBufs &m, void *bufs) {
+    ChunkCall c = base;
+    c.g = reinterpret_cast<const float *>(at_off(bufs, m.g2));
+    c.beta = reinterpret_cast<const float *>(at_off(bufs, m.b2));
+    c.mask = mask;
+    c.e = reinterpret_cast<const float *>(at_off(bufs, m.e));
+    c.qm = at_off(bufs, m.qm);
+    c.qm_lo = (size_t)base.B * base.T * base.Hv * kChunkD;
+    c.cm = reinterpret_cast<const uint8_t *>(at_off(bufs, m.cm));
+    c.cm_stride = (base.T + kChunkC - 1) / kChunkC;
+    return c;
+}
+
 // Masked chunked forward (resolved form GDN_FORM_CHUNK, arguments checked).  base holds the caller's q, k, v, g,
 // beta, state0, y, state_T and shapes.
 static int ck_masked_forward(const ChunkCall &base, const uint8_t *mask, int chunk, void *saved, size_t saved_bytes,
                              void *ws, size_t ws_bytes, hipStream_t st) {
-    const CkShape shp{base.B, base.T, base.Hk, base.Hv, base.in_dt == DT_BF16, vg_kind(base.gate)};
-    const int W = ck_window(chunk);
-    const size_t tokens = (size_t)base.B * base.T;
-    float *g2, *b2, *Z, *Yp = nullptr;
-    void *p1 = nullptr, *p2 = nullptr;
-    size_t p1_bytes = 0, p2_bytes = 0;
-    void *gws = ws;
-    size_t gws_bytes = ws ? ws_bytes : 0;
+    const CkShape shp{base.B, base.T, base.Hk, base.Hv, base.in_dt == DT_BF16, vg_kind(base.gate), true};
+    const MaskBufs m = mask_bufs(shp);
+    size_t tiles_bytes = 0;
+    void *bufs = ws;
     if (saved) {
-        const MaskSaved m = mask_saved(shp, chunk);
-        if (saved_bytes < m.total)
+        tiles_bytes = mask_tiles_bytes(shp, chunk);
+        if (saved_bytes < tiles_bytes + m.total)
             return fail(GDN_ERR_WORKSPACE, "saved buffer of %zu bytes is smaller than the %zu bytes required",
-                        saved_bytes, m.total);
-        p1 = at_off(saved, m.p1);
-        p1_bytes = m.p2 - m.p1;
-        if (!W) {
-            p2 = at_off(saved, m.p2);
-            p2_bytes = m.g2 - m.p2;
-        }
-        g2 = reinterpret_cast<float *>(at_off(saved, m.g2));
-        b2 = reinterpret_cast<float *>(at_off(saved, m.b2));
-        Z = reinterpret_cast<float *>(at_off(saved, m.Z));
-        Yp = reinterpret_cast<float *>(at_off(saved, m.Yp));
+                        saved_bytes, tiles_bytes + m.total);
+        bufs = at_off(saved, tiles_bytes);
     } else {
-        const size_t head = mask_fwd_only_head(shp);
-        if (!ws || ws_bytes < head)
+        if (!ws || ws_bytes < m.total)
             return fail(GDN_ERR_WORKSPACE, "workspace of %zu bytes is smaller than the %zu bytes a masked call needs",
-                        ws ? ws_bytes : 0, head);
-        const size_t ng = align256(tokens * base.Hv * 4);
-        g2 = reinterpret_cast<float *>(ws);
-        b2 = reinterpret_cast<float *>(at_off(ws, ng));
-        Z = reinterpret_cast<float *>(at_off(ws, 2 * ng));
-        gws = at_off(ws, head);
-        gws_bytes = ws_bytes - head;
+                        ws ? ws_bytes : 0, m.total);
+        ws = at_off(ws, m.total);
+        ws_bytes -= m.total;
     }
-    launch_mask_gates(base.g, base.beta, mask, g2, b2, tokens, base.Hv, base.gate, st);
-    int rc = check_launch(st, "gdn_fwd(mask gates)");
-    if (rc) return rc;
-    // pass 2: k as the query, z = S' k (fp32); its tiles kept only without checkpointing
-    ChunkCall c2 = base;
-    c2.q = base.k;
-    c2.g = g2;
-    c2.beta = b2;
-    c2.y = Z;
-    c2.out_dt = DT_F32;
-    c2.state_T = nullptr;
-    if ((rc = ck_forward(c2, chunk, p2, p2_bytes, gws, gws_bytes, st))) return rc;
-    // pass 1: y' into y, or in fp32 into Yp when the backward needs it (the fix-up then writes every y)
-    ChunkCall c1 = base;
-    c1.g = g2;
-    c1.beta = b2;
-    if (Yp) {
-        c1.y = Yp;
-        c1.out_dt = DT_F32;
-    }
-    if ((rc = ck_forward(c1, chunk, p1, p1_bytes, gws, gws_bytes, st))) return rc;
-    MaskArgs ma{};
-    ma.q = base.q; ma.k = base.k; ma.v = base.v; ma.g = base.g; ma.beta = base.beta; ma.mask = mask;
-    ma.y = base.y; ma.Z = Z; ma.Yp = Yp;
-    ma.Hk = base.Hk; ma.Hv = base.Hv; ma.Dk = kChunkD; ma.Dv = kChunkD;
-    ma.in_dt = base.in_dt; ma.out_dt = base.out_dt; ma.gate = base.gate;
+    const ChunkCall c = masked_call(base, mask, m, bufs);
+    MaskArgs ma = mask_args(base, mask);
+    ma.g2 = const_cast<float *>(c.g);
+    ma.beta2 = const_cast<float *>(c.beta);
+    ma.e = const_cast<float *>(c.e);
+    ma.qm = const_cast<void *>(c.qm);
+    ma.qm_lo = c.qm_lo;
+    ma.cm = const_cast<uint8_t *>(c.cm);
     {
-        Timed tm("mask_fix_fwd", st);
-        launch_mask_fix_fwd(ma, tokens, st);
+        Timed tm("mask_query", st);
+        launch_mask_query(ma, st);
     }
-    return check_launch(st, "gdn_fwd(mask fix-up)");
+    const int rc = check_launch(st, "gdn_fwd(mask queries)");
+    if (rc) return rc;
+    return ck_forward(c, chunk, saved, tiles_bytes, ws, ws ? ws_bytes : 0, st);
 }
 
 // Masked chunked backward (resolved form GDN_FORM_CHUNK, arguments checked).
 static int ck_masked_backward(const ChunkCall &base, const uint8_t *mask, int chunk, const void *saved,
                               size_t saved_bytes, void *ws, size_t ws_bytes, hipStream_t st) {
-    const CkShape shp{base.B, base.T, base.Hk, base.Hv, base.in_dt == DT_BF16, vg_kind(base.gate)};
-    const int W = ck_window(chunk);
-    const size_t tokens = (size_t)base.B * base.T;
-    const MaskSaved m = mask_saved(shp, chunk);
-    if (!saved || saved_bytes < m.total)
-        return fail(GDN_ERR_INVALID, "the saved buffer written by gdn_fwd (%zu bytes) is required", m.total);
-    const MaskWork k = mask_work(shp, chunk);
-    if (!ws || ws_bytes < k.total)
-        return fail(GDN_ERR_WORKSPACE, "workspace of %zu bytes is smaller than the %zu bytes required", ws_bytes,
-                    k.total);
-    void *sv = const_cast<void *>(saved);
-    const float *g2 = reinterpret_cast<const float *>(at_off(sv, m.g2));
-    const float *b2 = reinterpret_cast<const float *>(at_off(sv, m.b2));
-    float *wf[2][6];
-    for (int i = 0; i < 6; ++i) {
-        wf[0][i] = reinterpret_cast<float *>(at_off(ws, k.g1[i]));
-        wf[1][i] = reinterpret_cast<float *>(at_off(ws, k.g2[i]));
-    }
-    MaskArgs ma{};
-    ma.q = base.q; ma.k = base.k; ma.v = base.v; ma.dy = base.dy; ma.g = base.g; ma.beta = base.beta;
-    ma.mask = mask;
-    ma.Z = reinterpret_cast<const float *>(at_off(sv, m.Z));
-    ma.Yp = reinterpret_cast<float *>(at_off(sv, m.Yp));
-    ma.dy1 = reinterpret_cast<float *>(at_off(ws, k.dy1));
-    ma.dz = reinterpret_cast<float *>(at_off(ws, k.dz));
-    ma.Hk = base.Hk; ma.Hv = base.Hv; ma.Dk = kChunkD; ma.Dv = kChunkD;
-    ma.in_dt = base.in_dt; ma.dy_dt = base.dy_dt; ma.grad_dt = base.grad_dt; ma.gate = base.gate;
-    {
-        Timed tm("mask_bwd_cot", st);
-        launch_mask_bwd_cot(ma, tokens, st);
-    }
-    int rc = check_launch(st, "gdn_bwd(mask cotangents)");
+    const CkShape shp{base.B, base.T, base.Hk, base.Hv, base.in_dt == DT_BF16, vg_kind(base.gate), true};
+    const MaskBufs m = mask_bufs(shp);
+    const size_t tiles_bytes = mask_tiles_bytes(shp, chunk);
+    if (!saved || saved_bytes < tiles_bytes + m.total)
+        return fail(GDN_ERR_INVALID, "the saved buffer written by gdn_fwd (%zu bytes) is required", tiles_bytes + m.total);
+    const size_t stage_bytes = mask_stage_bytes(shp, chunk), need = mask_work_bytes(shp, chunk);
+    if (!ws || ws_bytes < need)
+        return fail(GDN_ERR_WORKSPACE, "workspace of %zu bytes is smaller than the %zu bytes required", ws_bytes, need);
+    ChunkCall c = masked_call(base, mask, m, at_off(const_cast<void *>(saved), tiles_bytes));
+    c.xm = reinterpret_cast<float *>(at_off(ws, stage_bytes));
+    int rc = ck_backward(c, chunk, saved, tiles_bytes, ws, stage_bytes, st);
     if (rc) return rc;
-    const bool want_ds0 = base.dstate0 != nullptr;
-    for (int pass = 0; pass < 2; ++pass) {
-        ChunkCall c = base;
-        c.g = g2;
-        c.beta = b2;
-        c.dy = pass ? ma.dz : ma.dy1;
-        c.dy_dt = DT_F32;
-        c.grad_dt = DT_F32;
-        c.dq = wf[pass][0]; c.dk = wf[pass][1]; c.dv = wf[pass][2]; c.dg = wf[pass][3]; c.dbeta = wf[pass][4];
-        c.dstate0 = want_ds0 ? wf[pass][5] : nullptr;
-        if (pass) {
-            c.q = base.k;           // pass 2 ran with k as its query
-            c.dstate_T = nullptr;   // the final state is pass 1's
-        }
-        const void *ps = pass && !W ? at_off(sv, m.p2) : at_off(sv, m.p1);
-        const size_t ps_bytes = pass && !W ? m.g2 - m.p2 : m.p2 - m.p1;
-        if ((rc = ck_backward(c, chunk, ps, ps_bytes, at_off(ws, k.pass), k.pass_bytes, st))) return rc;
-    }
-    ma.dq1 = wf[0][0]; ma.dk1 = wf[0][1]; ma.dv1 = wf[0][2]; ma.dg1 = wf[0][3]; ma.dbeta1 = wf[0][4];
-    ma.dq2 = wf[1][0]; ma.dk2 = wf[1][1]; ma.dv2 = wf[1][2]; ma.dg2 = wf[1][3]; ma.dbeta2 = wf[1][4];
-    ma.dq = base.dq; ma.dk = base.dk; ma.dv = base.dv; ma.dg = base.dg; ma.dbeta = base.dbeta;
+    MaskArgs ma = mask_args(base, mask);
+    ma.xm = c.xm;
     {
-        Timed tm("mask_bwd_combine", st);
-        launch_mask_bwd_combine(ma, tokens, st);
-        if (want_ds0) launch_add2(base.dstate0, wf[0][5], wf[1][5], ck_state_bytes(base.B, base.Hv) / 4, st);
+        Timed tm("mask_bwd_fix", st);
+        launch_mask_bwd_fix(ma, st);
     }
-    return check_launch(st, "gdn_bwd(mask combine)");
+    return check_launch(st, "gdn_bwd(masked tokens)");
 }
 
 // Fixed device scratch of gdn_fwd_noalloc: a file-scope device array, one copy per GPU, held until the process
@@ -752,7 +692,7 @@ int gdn_fwd_noalloc(const void *q, const void *k, const void *v, const float *g,
     int rc = check_shape(B, T, Hk, Hv, Dk, Dv, kChunkC, gate_kind, form);
     if (rc) return rc;
     if (!dtype_ok(in_dtype) || !dtype_ok(out_dtype)) return fail(GDN_ERR_INVALID, "unknown dtype code");
-    // masked calls keep the recurrent form here: the chunked form's masked passes need buffers that grow with T
+    // masked calls keep the recurrent form here: the chunked form's masked queries need buffers that grow with T
     if (mask && form == GDN_FORM_CHUNK)
         return fail(GDN_ERR_UNSUPPORTED, "gdn_fwd_noalloc runs masked calls in the recurrent form only");
     if (mask) form = GDN_FORM_RECURRENT;
@@ -761,7 +701,7 @@ int gdn_fwd_noalloc(const void *q, const void *k, const void *v, const float *g,
     void *ws = nullptr;
     size_t ws_bytes = 0;
     if (f == GDN_FORM_CHUNK && B > 0 && T > 0) {
-        const CkShape shp{B, T, Hk, Hv, in_dtype == DT_BF16, vg_kind(gate_kind)};
+        const CkShape shp{B, T, Hk, Hv, in_dtype == DT_BF16, vg_kind(gate_kind), false};
         const size_t one = ck_fwd_group_bytes(shp, std::min(kChunkC, T), false);
         if (one > kNoAllocScratchBytes)
             return fail(GDN_ERR_UNSUPPORTED,
@@ -851,9 +791,10 @@ size_t gdn_bwd_workspace_bytes(int B, int T, int Hk, int Hv, int Dk, int Dv, int
     if (f == GDN_FORM_CHUNK) {
         if (B == 0 || T == 0) return 0;
         const int W = ck_window(chunk);
-        if (has_mask) return mask_work({B, T, Hk, Hv, in_dtype == DT_BF16, false}, chunk).total;
-        if (W) return ck_bwd_target_bytes({B, T, Hk, Hv, in_dtype == DT_BF16, vg_kind(gate_kind)}, W);
-        return chunk_sizes(B, T, Hk, Hv, in_dtype == DT_BF16, true, vg_kind(gate_kind)).work;
+        const CkShape shp{B, T, Hk, Hv, in_dtype == DT_BF16, vg_kind(gate_kind), has_mask != 0};
+        if (has_mask) return mask_work_bytes(shp, chunk);
+        if (W) return ck_bwd_target_bytes(shp, W);
+        return ck_sizes(shp, T, true).work;
     }
     return bwd_layout(B, T, Hv, Dk, Dv, chunk, gate_kind).total;
 }

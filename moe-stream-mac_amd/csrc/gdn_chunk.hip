@@ -31,7 +31,7 @@ namespace ck {
               k_out_dt = AF32 ? (int)DT_F32 : (args).out_dt, k_grad_dt = AF32 ? (int)DT_F32 : (args).grad_dt; \
     (void)k_in_dt; (void)k_dy_dt; (void)k_out_dt; (void)k_grad_dt
 
-template <bool AF32>
+template <bool AF32, bool MASK>
 __global__ __launch_bounds__(NTP) void ck_prep_kernel(Args a) {
     DTYPES_OF(a);
     __shared__ __align__(16) float sK[C * LD];
@@ -53,6 +53,7 @@ __global__ __launch_bounds__(NTP) void ck_prep_kernel(Args a) {
     tile_fetch(rV, elem_ptr(a.v, v0, k_in_dt), v_row, n, k_in_dt);
     load_tile<C, D, NTP>(sK, LD, elem_ptr(a.k, qk0, k_in_dt), qk_row, n, k_in_dt);
     load_tile<C, D, NTP>(sX, LD, elem_ptr(a.q, qk0, k_in_dt), qk_row, n, k_in_dt);
+    if (MASK && flag_set(chunk_flag(a, b, c))) load_queries<NTP>(sX, LD, a, b, hv, t0, n, k_in_dt, tid);
     if (tid < C) {
         // inclusive prefix sum of the log decays in fp64 across wave 0
         float bt = 0.f, gl = 0.f;
@@ -130,7 +131,7 @@ struct RcScale {
     __device__ float operator()(int r) const { return expf((float)(G[C - 1] - G[r])); }
 };
 
-template <int VS, int MODE, bool AF32>
+template <int VS, int MODE, bool AF32, bool MASK>
 __global__ __launch_bounds__(NTS) void ck_fwd_kernel(Args a) {
     DTYPES_OF(a);
     constexpr bool kTiles = MODE != FWD_ONLY, kOut = MODE != FWD_RECOMPUTE;
@@ -183,6 +184,8 @@ __global__ __launch_bounds__(NTS) void ck_fwd_kernel(Args a) {
         tile_fetch(rP, a.w.P + ci * C * C, C, C, DT_F32);
         tile_fetch(rK, elem_ptr(a.k, qk0, k_in_dt), qk_row, n, k_in_dt);
     };
+    ChunkFlags<MASK> flags;
+    flags.start(a, b, cb, 1, ce);
     fetchA(cb);
     fetchB(cb);
     for (int c = cb; c < ce; ++c) {
@@ -197,6 +200,8 @@ __global__ __launch_bounds__(NTS) void ck_fwd_kernel(Args a) {
         tile_store(sW, LD, rW, DT_F32, NoScale{});
         tile_store(sU, LV, rU, DT_F32, NoScale{});
         tile_store(sQ, LD, rQ, k_in_dt, NoScale{});
+        flags.enter(a, b, c, 1, ce);
+        if (flags.cur) load_queries<NTS>(sQ, LD, a, b, hv, t0, n, k_in_dt, tid);
         if (tid < C) sG[tid] = rG;
         __syncthreads();
         if (c + 1 < ce) fetchA(c + 1);
@@ -230,6 +235,11 @@ __global__ __launch_bounds__(NTS) void ck_fwd_kernel(Args a) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) yi[t][e] *= expf((float)sG[mrow + 4 * lg + e]);
             mma_strip<C, DN>(yi, sW + mrow * LDC, LDC, 1, sD + 16 * nt0, LV, 1, 16);
+            if (flags.cur) {
+                ValueTerms<DN> vt;
+                vt.load(a, b, hv, t0, n, mrow, i0 + 16 * nt0, k_in_dt);
+                vt.add(yi);
+            }
 #pragma unroll
             for (int t = 0; t < DN; ++t)
 #pragma unroll
@@ -251,7 +261,7 @@ __global__ __launch_bounds__(NTS) void ck_fwd_kernel(Args a) {
 
 // ---------------------------------------------------------------------------------------------- ck_bwd_seq
 
-template <int VS, bool AF32>
+template <int VS, bool AF32, bool MASK>
 __global__ __launch_bounds__(NTS) void ck_bwd_seq_kernel(Args a) {
     DTYPES_OF(a);
     constexpr int LV = VS + 4;
@@ -307,6 +317,8 @@ __global__ __launch_bounds__(NTS) void ck_bwd_seq_kernel(Args a) {
         tile_fetch(rQ, elem_ptr(a.q, qk0, k_in_dt), qk_row, n, k_in_dt);
         tile_fetch(rT, a.w.T + ci * C * C, C, C, DT_F32);
     };
+    ChunkFlags<MASK> flags;
+    flags.start(a, b, a.NC - 1, -1, -1);
     fetchA(a.NC - 1);
     fetchB(a.NC - 1);
     for (int c = a.NC - 1; c >= 0; --c) {
@@ -342,6 +354,8 @@ __global__ __launch_bounds__(NTS) void ck_bwd_seq_kernel(Args a) {
         __syncthreads();
         tile_store(sW, LD, rW, DT_F32, NoScale{});
         tile_store(sQ, LD, rQ, k_in_dt, NoScale{});
+        flags.enter(a, b, c, -1, -1);
+        if (flags.cur) load_queries<NTS>(sQ, LD, a, b, hv, c * C, min(C, T - c * C), k_in_dt, tid);
         tile_store(sT, LDC, rT, DT_F32, NoScale{});  // over dh', read before the barrier above
         __syncthreads();
         if (c > 0) fetchB(c - 1);
@@ -470,7 +484,7 @@ __device__ __forceinline__ void chunk_dg_dbeta(float *sE, const float (*sRow)[2]
 // and the last value head writes dq and dk in the gradient dtype.  T and dDelta enter only through TdD = T^T dDelta
 // (saved by ck_bwd_seq_kernel): dv = diag(beta) TdD, dK -= diag(beta gamma) Y2 (Y2 = TdD h^T), dA = -TdD Delta^T
 // below the diagonal, dbeta += rowsum(V * TdD) - gamma s4 and dG -= beta gamma s4 (s4 = rowsum(K * Y2)).
-template <bool AF32>
+template <bool AF32, bool MASK>
 __device__ __forceinline__ void bwd_local_f32_head(const Args &a, int c, int hk, int b, int rr, int rep) {
     DTYPES_OF(a);
     __shared__ __align__(16) float R1[D * LD];       // h, then dh' ([j][i]); then K at R1, Q at R1 + C*LD
@@ -651,6 +665,8 @@ __device__ __forceinline__ void bwd_local_f32_head(const Args &a, int c, int hk,
     // ---- phase 3: dQ += dPG K ; dK += dPG^T Q ; K K^T
     load_tile<C, D, NTB>(sKm, LD, elem_ptr(a.k, qk0, k_in_dt), qk_row, n, k_in_dt, nullptr, tid);
     load_tile<C, D, NTB>(sQm, LD, elem_ptr(a.q, qk0, k_in_dt), qk_row, n, k_in_dt, nullptr, tid);
+    const bool mk = MASK && flag_set(chunk_flag(a, b, c));
+    if (mk) load_queries<NTB>(sQm, LD, a, b, hv, t0, n, k_in_dt, tid);
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -751,6 +767,8 @@ __device__ __forceinline__ void bwd_local_f32_head(const Args &a, int c, int hk,
             const int i = l + 64 * p, rr2 = i >> 4, r = r0 + rr2, c4 = 64 * ch + 4 * (i & 15);
             float4 v = *reinterpret_cast<const float4 *>(stg + rr2 * LQ + 4 * (i & 15));
             if (r >= n) continue;
+            if (MASK && half == 0 && mk)
+                *reinterpret_cast<float4 *>(a.xm + query_row(a, b, t0 + r, hv) + c4) = v;  // dL/dq~ of this value head
             if (!first) v = make_float4(prev[p].x + v.x, prev[p].y + v.y, prev[p].z + v.z, prev[p].w + v.w);
             const size_t o = qk_out + (size_t)r * a.Hk * D + c4;
             if (!last) {
@@ -771,7 +789,7 @@ __device__ __forceinline__ void bwd_local_f32_head(const Args &a, int c, int hk,
 }
 
 // One workgroup of 8 waves per (chunk, key head), walking the key head's value heads in order.
-template <bool AF32>
+template <bool AF32, bool MASK>
 __global__ __launch_bounds__(NTB) void ck_bwd_local_kernel(Args a) {
     typedef const __attribute__((address_space(4))) Args *KArgs;  // the kernel arguments (constant memory)
     const int rep = a.Hv / a.Hk;
@@ -779,7 +797,7 @@ __global__ __launch_bounds__(NTB) void ck_bwd_local_kernel(Args a) {
         // the arguments are read anew for each value head instead of being held in scalar registers across it
         KArgs ap = (KArgs)__builtin_amdgcn_kernarg_segment_ptr();
         asm volatile("" : "+s"(ap));
-        bwd_local_f32_head<AF32>(*(const Args *)ap, blockIdx.x, blockIdx.y, blockIdx.z, rr, rep);
+        bwd_local_f32_head<AF32, MASK>(*(const Args *)ap, blockIdx.x, blockIdx.y, blockIdx.z, rr, rep);
     }
 }
 
@@ -823,7 +841,7 @@ constexpr int NQR = 4;  // dq row pieces per thread whose running sum stays in r
 // in order (rr = 0, 1, ...) at the 16-byte row pieces each thread writes out: dk (ck) and the first NQR dq pieces
 // (cq) in registers, any other dq pieces in the part rows of the key head (each thread reading back only the
 // elements it wrote itself); the last value head writes dq and dk in the gradient dtype.
-template <bool DYF32>
+template <bool DYF32, bool MASK>
 __device__ __forceinline__ void bwd_local_bf16_head(const Args &a, int c, int hk, int b, int rr, int rep,
                                                     float4 (&ck)[4], float4 (&cq)[NQR]) {
     __shared__ __align__(16) unsigned char arena[ARENA];
@@ -860,6 +878,7 @@ __device__ __forceinline__ void bwd_local_bf16_head(const Args &a, int c, int hk
     // the tile loads, or a branch on the dtype among them, made the compiler wait for the loads in flight and split
     // the phase's loads into serial batches.  dv = diag(beta) TdD leaves from the fp32 TdD loads, and
     // rowsum(V * TdD) goes to sVT.
+    const bool mk = MASK && flag_set(chunk_flag(a, b, c));
     double gch = 0.0;
     float bch = 0.f;
     if (tid < C) {
@@ -976,6 +995,7 @@ __device__ __forceinline__ void bwd_local_bf16_head(const Args &a, int c, int hk
     const bool isk = tid >= NBQ;
     Blk84 bk;
     bk.load(isk ? ksrc : qsrc, qk_row, isk ? tid - NBQ : tid, D, n);
+    if (mk && !isk) bk.load(static_cast<const bfr *>(a.qm) + query_row(a, b, t0, hv), (size_t)a.Hv * D, tid, D, n);  // q~ (hi)
     float bnd[4] = {0.f, 0.f, 0.f, 0.f}, rowB[4] = {0.f, 0.f, 0.f, 0.f}, tl[4] = {0.f, 0.f, 0.f, 0.f};
     f4 dQ[4], dK[4], Y2[4], dPG[2], Ep[2], dA[2];
 #pragma unroll
@@ -1081,9 +1101,31 @@ __device__ __forceinline__ void bwd_local_bf16_head(const Args &a, int c, int hk
                 bnd[e] -= bg * s4;
                 dK[t][e] -= bg * Y2[t][e];
             }
+        if (mk) {  // the lo part of q~ in the boundary terms: four rows of one column are 8 contiguous bytes
+            const bfr *ql = a.w.QMb + ci * 2 * D * C + D * C;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const uint2 x = *reinterpret_cast<const uint2 *>(ql + frag_off<C>(64 * ch + 16 * t + li, r0 + 4 * lg));
+                bnd[0] += bf2f(x.x & 0xffffu) * dQ[t][0];
+                bnd[1] += bf2f(x.x >> 16) * dQ[t][1];
+                bnd[2] += bf2f(x.y & 0xffffu) * dQ[t][2];
+                bnd[3] += bf2f(x.y >> 16) * dQ[t][3];
+            }
+        }
     }
     mmab<C, 4, true>(dQ, T16(O_PNH), T16(O_PNL), LB, r0, T16(O_KT), nullptr, LB, 64 * ch, l);
     mmab<C, 4, true>(dK, T16(O_PTH), T16(O_PTL), LB, r0, T16(O_QT), nullptr, LB, 64 * ch, l);
+    if (mk) {
+        // the lo part of q~: dK += dPG^T Q~lo, fragments straight from ck_prep's tile
+        const bfr *ql = a.w.QMb + ci * 2 * D * C + D * C;
+#pragma unroll
+        for (int k0 = 0; k0 < C; k0 += 32) {
+            const bf8 x = frag(T16(O_PTH), LB, r0, k0, l);
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                dK[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, ld_frag(ql + frag_off<C>(64 * ch + 16 * t, k0) + 8 * l), dK[t], 0, 0, 0);
+        }
+    }
     // dQ is complete: it goes out now (to the running sum, or as dq from the last value head) instead of staying
     // live
 #pragma unroll
@@ -1095,6 +1137,8 @@ __device__ __forceinline__ void bwd_local_bf16_head(const Args &a, int c, int hk
         const int i = l + 64 * p, rr2 = i >> 4, r = r0 + rr2, c4 = 64 * ch + 4 * (i & 15);
         float4 v = *reinterpret_cast<const float4 *>(stq + rr2 * LQ + 4 * (i & 15));
         if (r >= n) continue;
+        if (mk)
+            *reinterpret_cast<float4 *>(a.xm + query_row(a, b, t0 + r, hv) + c4) = v;  // dL/dq~ of this value head
         if (!first) {
             const float4 s = p < NQR ? cq[p < NQR ? p : 0] : prevq[p];
             v = make_float4(s.x + v.x, s.y + v.y, s.z + v.z, s.w + v.w);
@@ -1196,7 +1240,7 @@ __device__ __forceinline__ void bwd_local_bf16_head(const Args &a, int c, int hk
 }
 
 // One workgroup of 8 waves per (chunk, key head), walking the key head's value heads in order.
-template <bool DYF32>
+template <bool DYF32, bool MASK>
 __global__ __launch_bounds__(NTB) void ck_bwd_local_bf16_kernel(Args a) {
     typedef const __attribute__((address_space(4))) Args *KArgs;  // the kernel arguments (constant memory)
     const int rep = a.Hv / a.Hk;
@@ -1206,7 +1250,7 @@ __global__ __launch_bounds__(NTB) void ck_bwd_local_bf16_kernel(Args a) {
         // the arguments are read anew for each value head instead of being held in scalar registers across it
         KArgs ap = (KArgs)__builtin_amdgcn_kernarg_segment_ptr();
         asm volatile("" : "+s"(ap));
-        bwd_local_bf16_head<DYF32>(*(const Args *)ap, blockIdx.x, blockIdx.y, blockIdx.z, rr, rep, ck, cq);
+        bwd_local_bf16_head<DYF32, MASK>(*(const Args *)ap, blockIdx.x, blockIdx.y, blockIdx.z, rr, rep, ck, cq);
     }
 }
 
@@ -1238,7 +1282,7 @@ struct FwdFrags {
 
 // VG: one decay per key channel (gdn_chunk_vg.hip wrote the tiles): Y = (Q * exp(G)) h + P Delta with the Q * exp(G)
 // tile as the A operand, and h' = diag(exp(G_C)) h + (K * exp(G_C - G))^T Delta, a decay per state row.
-template <int VS, int MODE, bool VG = false>
+template <int VS, int MODE, bool VG, bool MASK>
 __global__ __launch_bounds__(NTS) void ck_fwd_bf16_kernel(Args a) {
     constexpr bool kTiles = MODE != FWD_ONLY, kOut = MODE != FWD_RECOMPUTE;
     constexpr int NTN = VS / 16, DN = NTN >= 2 ? NTN / 2 : 1;
@@ -1269,13 +1313,21 @@ __global__ __launch_bounds__(NTS) void ck_fwd_bf16_kernel(Args a) {
             const int j = 16 * w + 4 * lg + e, i = i0 + 16 * t + li;
             h[t][e] = sr.s0 ? sr.s0[(head * D + i) * D + j] : 0.f;
         }
+    ChunkFlags<MASK> flags;
     auto fetch = [&](FwdFrags<DN> &f, int c) {
         const size_t ci = head * a.NC + c;
         const int t0 = c * C, n = min(C, T - t0), r = mrow + li;
         const bfr *wb = a.w.Wb + ci * C * D + frag_off<D>(mrow, 0) + 8 * l;
         const bfr *pb = a.w.Pb + ci * 2 * C * C + frag_off<C>(mrow, 0) + 8 * l;
         const bfr *kt = a.w.KTb + ci * D * C + frag_off<C>(16 * w, 0) + 8 * l;
-        const bfr *qb = static_cast<const bfr *>(a.q) + (((size_t)b * a.Ts + t0 + r) * a.Hk + hk) * D + 8 * lg;
+        // q, or a masked chunk's query rows (hi): a scalar choice of the tile's first row and of the row stride
+        const bfr *q0 = static_cast<const bfr *>(a.q) + (((size_t)b * a.Ts + t0) * a.Hk + hk) * D;
+        int q_row = a.Hk * D;
+        if (flags.nxt) {
+            q0 = static_cast<const bfr *>(a.qm) + query_row(a, b, t0, hv);
+            q_row = a.Hv * D;
+        }
+        const bfr *qb = q0 + (size_t)r * q_row + 8 * lg;
         const bfr *qg = VG ? a.w.QGb + ci * C * D + frag_off<D>(mrow, 0) + 8 * l : nullptr;
         // W and U in the waves that form Delta, Q and P in the waves that form y
         if (dwave) {
@@ -1334,6 +1386,7 @@ __global__ __launch_bounds__(NTS) void ck_fwd_bf16_kernel(Args a) {
         const int t0 = c * C, n = min(C, T - t0);
         const size_t ci = head * a.NC + c;
         if (float *sp = snap_at<MODE>(a, c)) store_state_acc<NTN>(sp, h, head, i0, w, lg, li);
+        flags.enter(a, b, c, 1, ce);
         // h -> LDS as the operand [i][j]; the chunk-entry state -> saved H ([j][i], bf16)
 #pragma unroll
         for (int t = 0; t < NTN; ++t) {
@@ -1360,6 +1413,17 @@ __global__ __launch_bounds__(NTS) void ck_fwd_bf16_kernel(Args a) {
         for (int t = 0; t < DN; ++t) wh[t] = zero4();
         if (dwave) mmar<D, DN>(wh, cur.W, nullptr, sHh, nullptr, LH, 16 * nt0);
         if (ywave) mmar<D, DN, false, true>(yi, cur.Q, nullptr, sHh, sHl, LH, 16 * nt0);
+        // a masked chunk's own loads, the lo part of its queries and its value terms, go out here, where the registers of
+        // W, Q and U fall free (64-wide slices have none to spare before), and arrive during Delta's conversion
+        ValueTerms<DN> vt;
+        bf8 ql[MASK ? 4 : 1];
+        if (MASK && flags.cur && ywave) {
+            const int x = opaque(l), r = min(mrow + (x & 15), n - 1);
+            const bfr *p = static_cast<const bfr *>(a.qm) + a.qm_lo + query_row(a, b, t0, hv) + (size_t)r * a.Hv * D + 8 * (x >> 4);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) ql[MASK ? k : 0] = ld_frag(p + 32 * k);
+            vt.load(a, b, hv, t0, n, mrow, i0 + 16 * nt0, DT_BF16);
+        }
         if (dwave) {
 #pragma unroll
             for (int t = 0; t < DN; ++t) {
@@ -1374,6 +1438,14 @@ __global__ __launch_bounds__(NTS) void ck_fwd_bf16_kernel(Args a) {
                 }
             }
         }
+        if (MASK && flags.cur && ywave) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int t = 0; t < DN; ++t)
+                    yi[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mrow + li < n ? ql[MASK ? k : 0] : zero_frag(),
+                                                                    frag(sHh, LH, 16 * (nt0 + t), 32 * k), yi[t], 0, 0, 0);
+        }
         __syncthreads();
         if (ywave && kOut) {
             // Y = diag(gamma) Q h + P Delta  (per-channel gates: the decays are inside the Q * exp(G) tile)
@@ -1384,6 +1456,7 @@ __global__ __launch_bounds__(NTS) void ck_fwd_bf16_kernel(Args a) {
                     for (int e = 0; e < 4; ++e) yi[t][e] *= sGam[mrow + 4 * lg + e];
             }
             mmar<C, DN, true, true>(yi, cur.P, cur.P + 2, sDh, sDl, LDd, 16 * nt0);
+            if (MASK && flags.cur) vt.add(yi);
             // the output dtype is tested once for the whole tile, not at every element
             auto store_y = [&](auto dtag) {
                 using E = decltype(dtag);
@@ -1420,6 +1493,7 @@ __global__ __launch_bounds__(NTS) void ck_fwd_bf16_kernel(Args a) {
         mmar<C, NTN>(h, cur.K, nullptr, sDh, nullptr, LDd, 0);
     };
     FwdFrags<DN> fa, fb;
+    flags.start(a, b, cb, 1, ce);
     fetch(fa, cb);
     for (int c = cb; c < ce; c += 2) {
         step(c, fa, fb);
@@ -1448,6 +1522,7 @@ constexpr int LU = D + 4;
 static_assert(C * LDC * 4 <= D * LT * 2, "A fits its region");
 static_assert(C * LU * 4 + C * LK * 2 <= PR_T, "U and W staging below T");
 
+template <bool MASK>
 __global__ __launch_bounds__(NTP, 2) void ck_prep_bf16_kernel(Args a) {
     __shared__ __align__(16) unsigned char pa[PR_END];
     __shared__ float scratch[3 * 256];
@@ -1467,6 +1542,7 @@ __global__ __launch_bounds__(NTP, 2) void ck_prep_bf16_kernel(Args a) {
     const size_t qk0 = (((size_t)b * a.Ts + t0) * a.Hk + hk) * D, qk_row = (size_t)a.Hk * D;
     const size_t v0 = (((size_t)b * a.Ts + t0) * a.Hv + hv) * D, v_row = (size_t)a.Hv * D;
 
+    const int flag = MASK ? chunk_flag(a, b, c) : 0;
     // V as 8-token x 2-channel blocks (one per thread) for the transposed tile, kept in registers until Q is dead
     static_assert((C / 8) * (D / 2) == NTP, "one V block per thread");
     const int vb = tid / (D / 2), vc = 2 * (tid - vb * (D / 2));
@@ -1491,6 +1567,15 @@ __global__ __launch_bounds__(NTP, 2) void ck_prep_bf16_kernel(Args a) {
         const uint4 xq = *reinterpret_cast<const uint4 *>(static_cast<const bfr *>(a.q) + o);
         kr[p] = r < n ? xk : make_uint4(0u, 0u, 0u, 0u);
         qr[p] = r < n ? xq : make_uint4(0u, 0u, 0u, 0u);
+    }
+    const bool mk = MASK && flag_set(flag);
+    if (mk) {  // q~ (hi) in the place of q
+#pragma unroll
+        for (int p = 0; p < KPER; ++p) {
+            const int pc = tid + p * NTP, r = pc / (D / 8), c8 = (pc - r * (D / 8)) * 8;
+            const uint4 x = *reinterpret_cast<const uint4 *>(static_cast<const bfr *>(a.qm) + query_row(a, b, t0 + min(r, n - 1), hv) + c8);
+            qr[p] = r < n ? x : make_uint4(0u, 0u, 0u, 0u);
+        }
     }
     const size_t gi = ((size_t)b * a.Ts + t0 + min(tid, n - 1)) * a.Hv + hv;
     const float b_ld = a.beta[gi], g_ld = a.g[gi];
@@ -1528,10 +1613,28 @@ __global__ __launch_bounds__(NTP, 2) void ck_prep_bf16_kernel(Args a) {
             v[rr][0] = bf2f(x.x & 0xffffu) * sc; v[rr][1] = bf2f(x.x >> 16) * sc;
             v[rr][2] = bf2f(x.y & 0xffffu) * sc; v[rr][3] = bf2f(x.y >> 16) * sc;
         }
-        // Q^T depends on the key head only: the first value head of each key head writes it
+        // Q^T depends on the key head only, and the first value head of each key head writes it; in a chunk that holds
+        // masked tokens it is Q~^T, per value head
         const int rep = a.Hv / a.Hk;
-        bfr *dst = isq ? a.w.QTb + (((size_t)b * a.Hk + hk) * a.NC + c) * D * C : a.w.KTb + ci * D * C;
-        if (!isq || (hv % rep == 0 && !a.fwd_only)) {
+        bfr *dst = !isq ? a.w.KTb + ci * D * C
+                   : mk ? a.w.QMb + ci * 2 * D * C
+                        : a.w.QTb + (((size_t)b * a.Hk + hk) * a.NC + c) * D * C;
+        if (mk && isq && !a.fwd_only) {  // Q~^T lo
+            uint2 x[8];
+#pragma unroll
+            for (int rr = 0; rr < 8; ++rr) {
+                const int r = rb * 8 + rr;
+                const uint2 y = *reinterpret_cast<const uint2 *>(static_cast<const bfr *>(a.qm) + a.qm_lo + query_row(a, b, t0 + min(r, n - 1), hv) + j0);
+                x[rr] = r < n ? y : make_uint2(0u, 0u);
+            }
+            auto e16 = [&](int rr, int cc) { const uint32_t wd = cc < 2 ? x[rr].x : x[rr].y; return cc & 1 ? wd >> 16 : wd & 0xffffu; };
+#pragma unroll
+            for (int cc = 0; cc < 4; ++cc)
+                *reinterpret_cast<uint4 *>(dst + D * C + frag_off<C>(j0 + cc, rb * 8)) =
+                    make_uint4(e16(0, cc) | (e16(1, cc) << 16), e16(2, cc) | (e16(3, cc) << 16),
+                               e16(4, cc) | (e16(5, cc) << 16), e16(6, cc) | (e16(7, cc) << 16));
+        }
+        if (!isq || ((mk || hv % rep == 0) && !a.fwd_only)) {
 #pragma unroll
             for (int cc = 0; cc < 4; ++cc)
                 *reinterpret_cast<uint4 *>(dst + frag_off<C>(j0 + cc, rb * 8)) =
@@ -1550,6 +1653,18 @@ __global__ __launch_bounds__(NTP, 2) void ck_prep_bf16_kernel(Args a) {
 #pragma unroll
         for (int t = 0; t < 4; ++t) acc[t] = zero4();
         mmab<D, 4>(acc, isq ? sQ : sK, nullptr, LK, r0, sK, nullptr, LK, 0);
+        if (mk && isq) {  // the lo part of q~, as fragments straight from its rows
+            const int r = r0 + li;
+            const bfr *ql = static_cast<const bfr *>(a.qm) + a.qm_lo + query_row(a, b, t0 + min(r, n - 1), hv) + 8 * lg;
+            bf8 x[D / 32];
+#pragma unroll
+            for (int k = 0; k < D / 32; ++k) x[k] = ld_frag(ql + 32 * k);
+#pragma unroll
+            for (int k = 0; k < D / 32; ++k)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(r < n ? x[k] : zero_frag(), frag(sK, LK, 16 * t, 32 * k), acc[t], 0, 0, 0);
+        }
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             uint32_t ph[4], pl[4];
@@ -1717,7 +1832,7 @@ struct BwdFrags {
 
 // VG: one decay per key channel (gdn_chunk_vg.hip wrote the tiles): dDelta = (K * exp(G_C - G)) dh' + P^T dY with that
 // tile as the A operand, and dh = diag(exp(G_C)) dh' + (Q * exp(G))^T dY - W^T dDelta, (Q * exp(G))^T per value head.
-template <int VS, bool DYF32, bool VG = false>
+template <int VS, bool DYF32, bool VG, bool MASK>
 __global__ __launch_bounds__(NTS) void ck_bwd_seq_bf16_kernel(Args a) {
     constexpr int NTN = VS / 16, DN = NTN >= 2 ? NTN / 2 : 1;
     constexpr int LH = D + 8, LDd = C + 8;
@@ -1765,13 +1880,16 @@ __global__ __launch_bounds__(NTS) void ck_bwd_seq_bf16_kernel(Args a) {
         ttr1 = src[tid + NTS];
     };
     using YRaw = typename std::conditional<DYF32, float2, uint32_t>::type;
+    ChunkFlags<MASK> flags;
     auto fetch = [&](BwdFrags &f, YRaw (&y)[8], int c) {
         const size_t ci = head * a.NC + c;
         const int t0 = c * C, n = min(C, T - t0), r = mrow + li;
         const bfr *kb = static_cast<const bfr *>(a.k) + (((size_t)b * a.Ts + t0 + r) * a.Hk + hk) * D + 8 * lg;
         const bfr *kd = VG ? a.w.KDb + ci * C * D + frag_off<D>(mrow, 0) + 8 * l : nullptr;
         const bfr *pt = a.w.PTb + ci * 2 * C * C + frag_off<C>(mrow, 0) + 8 * l;
-        const bfr *qt = a.w.QTb + (VG ? ci : ((size_t)b * a.Hk + hk) * a.NC + c) * D * C + frag_off<C>(16 * w, 0) + 8 * l;
+        const bfr *qt0 = a.w.QTb + (VG ? ci : ((size_t)b * a.Hk + hk) * a.NC + c) * D * C;
+        if (flags.nxt) qt0 = a.w.QMb + ci * 2 * D * C;  // Q~^T (hi)
+        const bfr *qt = qt0 + frag_off<C>(16 * w, 0) + 8 * l;
         const bfr *wt = a.w.nWTb + ci * D * C + frag_off<C>(16 * w, 0) + 8 * l;
         // K and P^T only in the waves that form dDelta (all of them when NTN >= 2)
         if (cwave) {
@@ -1836,6 +1954,7 @@ __global__ __launch_bounds__(NTS) void ck_bwd_seq_bf16_kernel(Args a) {
     YRaw yr[8];
     auto step = [&](const int c, BwdFrags &cur, BwdFrags &nxt) {
         const size_t ci = head * a.NC + c;
+        flags.enter(a, b, c, -1, -1);
         // dh' -> LDS as the operand [i][j] (hi / lo) and -> the saved dH ([j][i], fp32)
 #pragma unroll
         for (int t = 0; t < NTN; ++t) {
@@ -1933,6 +2052,12 @@ __global__ __launch_bounds__(NTS) void ck_bwd_seq_bf16_kernel(Args a) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) td[(size_t)(mrow + 4 * lg + e) * D + i0 + 16 * (nt0 + t) + li] = tdd[t][e];
         }
+        bf8 ql[MASK ? 2 : 1];
+        if (MASK && flags.cur) {
+            const bfr *p = a.w.QMb + ci * 2 * D * C + D * C + frag_off<C>(16 * w, 0) + 8 * opaque(l);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) ql[MASK ? k : 0] = ld_frag(p + FRAG_BLOCK * k);
+        }
         // dh = gamma_C dh' + Q^T diag(gamma) dY + (-W^T) dDelta  (per-channel gates: row j decays by exp(G_C,j))
         if constexpr (VG) {
             const float gcr[4] = {cur.gc.x, cur.gc.y, cur.gc.z, cur.gc.w};
@@ -1948,8 +2073,16 @@ __global__ __launch_bounds__(NTS) void ck_bwd_seq_bf16_kernel(Args a) {
         }
         mmar<C, NTN, false, true>(dh, cur.QT, nullptr, sYgh, sYgl, LDd, 0);
         mmar<C, NTN>(dh, cur.WT, nullptr, sDd, nullptr, LDd, 0);
+        if (MASK && flags.cur) {  // the lo part of q~
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+#pragma unroll
+                for (int t = 0; t < NTN; ++t)
+                    dh[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ql[MASK ? k : 0], frag(sYgh, LDd, 16 * t, 32 * k), dh[t], 0, 0, 0);
+        }
     };
     BwdFrags fa, fb;
+    flags.start(a, b, a.NC - 1, -1, -1);
     fetch(fa, yr, a.NC - 1);
     fetch_tt(a.NC - 1);
     int c = a.NC - 1;
@@ -1978,7 +2111,7 @@ constexpr int CK_D = ck::D;
 
 static size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-ChunkSizes chunk_sizes(int B, int T, int Hk, int Hv, bool bf16, bool bwd, int vgk) {
+ChunkSizes chunk_sizes(int B, int T, int Hk, int Hv, bool bf16, bool bwd, int vgk, bool masked) {
     static_assert(CK_C == kChunkC && CK_D == kChunkD, "chunk geometry");
     ChunkSizes s{};
     const size_t NC = (size_t)(T + CK_C - 1) / CK_C;
@@ -2007,6 +2140,7 @@ ChunkSizes chunk_sizes(int B, int T, int Hk, int Hv, bool bf16, bool bwd, int vg
     put(s.Gv, vg ? n * cd * 4 : 0);
     put(s.QGb, vg ? n * cd * 2 : 0);
     put(s.KDb, vg && bwd ? n * cd * 2 : 0);
+    put(s.QMb, bf16 && bwd && masked ? n * 2 * cd * 2 : 0);
     s.saved = off;
     off = 0;
     put(s.dH, n * dd * (bf16 ? 2 : 4));
@@ -2031,7 +2165,7 @@ static ck::Args make_args(const ChunkCall &cc) {
     a.state_T = cc.state_T;
     a.dg = cc.dg; a.dbeta = cc.dbeta; a.dstate0 = cc.dstate0;
     const bool bf16 = cc.in_dt == DT_BF16;
-    const ChunkSizes s = chunk_sizes(cc.B, cc.T, cc.Hk, cc.Hv, bf16, !cc.fwd_only, vg_kind(cc.gate));
+    const ChunkSizes s = chunk_sizes(cc.B, cc.T, cc.Hk, cc.Hv, bf16, !cc.fwd_only, vg_kind(cc.gate), cc.mask != nullptr);
     char *sv = static_cast<char *>(cc.tiles);
     auto at = [&](const ChunkSizes::Buf &bf) -> void * { return bf.size ? sv + bf.off : nullptr; };
     a.w.H = static_cast<float *>(at(s.H));
@@ -2050,6 +2184,7 @@ static ck::Args make_args(const ChunkCall &cc) {
     a.w.Gv = static_cast<float *>(at(s.Gv));
     a.w.QGb = static_cast<unsigned short *>(at(s.QGb));
     a.w.KDb = static_cast<unsigned short *>(at(s.KDb));
+    a.w.QMb = static_cast<unsigned short *>(at(s.QMb));
     if (cc.work) {
         char *wk = static_cast<char *>(cc.work);
         a.w.dH = reinterpret_cast<float *>(wk + s.dH.off);
@@ -2060,6 +2195,7 @@ static ck::Args make_args(const ChunkCall &cc) {
     a.B = cc.B; a.T = cc.T; a.Ts = cc.Ts; a.Hk = cc.Hk; a.Hv = cc.Hv; a.NC = (cc.T + CK_C - 1) / CK_C;
     a.in_dt = cc.in_dt; a.out_dt = cc.out_dt; a.dy_dt = cc.dy_dt; a.grad_dt = cc.grad_dt; a.gate = cc.gate;
     a.snap = cc.snap; a.wc = cc.wc; a.win0 = cc.win0; a.recompute = cc.recompute; a.fwd_only = cc.fwd_only;
+    a.mask = cc.mask; a.cm = cc.cm; a.qm = cc.qm; a.qm_lo = cc.qm_lo; a.e = cc.e; a.xm = cc.xm; a.cm_stride = cc.cm_stride;
     a.read_ahead = s.saved >= kReadAheadBytes;
     return a;
 }
@@ -2076,13 +2212,30 @@ static bool all_f32(const ck::Args &a) {
     return a.in_dt == DT_F32 && a.dy_dt == DT_F32 && a.out_dt == DT_F32 && a.grad_dt == DT_F32;
 }
 
-// MT: the kernel set, 0 fp32 (fp32 / fp16 inputs), 1 bf16, 2 bf16 with one decay per key channel
+// f(std::integral_constant<bool, x>): a runtime flag as a template argument
+template <class F>
+static void with_flag(bool x, F f) {
+    if (x) f(std::true_type{});
+    else f(std::false_type{});
+}
+
+// MT: the kernel set, 0 fp32 (fp32 / fp16 inputs), 1 bf16, 2 bf16 with one decay per key channel (never masked)
 template <int MT, int VS, int MODE>
 static void fwd_launch(const ck::Args &a, hipStream_t st, dim3 grid) {
-    if constexpr (MT == 2) hipLaunchKernelGGL((ck::ck_fwd_bf16_kernel<VS, MODE, true>), grid, dim3(ck::NTS), 0, st, a);
-    else if constexpr (MT == 1) hipLaunchKernelGGL((ck::ck_fwd_bf16_kernel<VS, MODE>), grid, dim3(ck::NTS), 0, st, a);
-    else if (all_f32(a)) hipLaunchKernelGGL((ck::ck_fwd_kernel<VS, MODE, true>), grid, dim3(ck::NTS), 0, st, a);
-    else hipLaunchKernelGGL((ck::ck_fwd_kernel<VS, MODE, false>), grid, dim3(ck::NTS), 0, st, a);
+    if constexpr (MT == 2) {
+        hipLaunchKernelGGL((ck::ck_fwd_bf16_kernel<VS, MODE, true, false>), grid, dim3(ck::NTS), 0, st, a);
+    } else {
+        // recomputed windows write no y: they need no query
+        with_flag(MODE != ck::FWD_RECOMPUTE && a.mask != nullptr, [&](auto mask) {
+            constexpr bool MASK = MODE != ck::FWD_RECOMPUTE && decltype(mask)::value;
+            if constexpr (MT == 1)
+                hipLaunchKernelGGL((ck::ck_fwd_bf16_kernel<VS, MODE, false, MASK>), grid, dim3(ck::NTS), 0, st, a);
+            else if (all_f32(a))
+                hipLaunchKernelGGL((ck::ck_fwd_kernel<VS, MODE, true, MASK>), grid, dim3(ck::NTS), 0, st, a);
+            else
+                hipLaunchKernelGGL((ck::ck_fwd_kernel<VS, MODE, false, MASK>), grid, dim3(ck::NTS), 0, st, a);
+        });
+    }
 }
 
 template <int MT, int VS>
@@ -2092,16 +2245,18 @@ static void seq_launch(const ck::Args &a, hipStream_t st, bool fwd) {
         if (a.recompute) fwd_launch<MT, VS, ck::FWD_RECOMPUTE>(a, st, grid);
         else if (a.fwd_only) fwd_launch<MT, VS, ck::FWD_ONLY>(a, st, grid);
         else fwd_launch<MT, VS, ck::FWD_TRAIN>(a, st, grid);
-    } else if constexpr (MT >= 1) {
-        constexpr bool VG = MT == 2;
-        if (a.dy_dt == DT_F32)
-            hipLaunchKernelGGL((ck::ck_bwd_seq_bf16_kernel<VS, true, VG>), grid, dim3(ck::NTS), 0, st, a);
-        else
-            hipLaunchKernelGGL((ck::ck_bwd_seq_bf16_kernel<VS, false, VG>), grid, dim3(ck::NTS), 0, st, a);
-    } else {
-        if (all_f32(a)) hipLaunchKernelGGL((ck::ck_bwd_seq_kernel<VS, true>), grid, dim3(ck::NTS), 0, st, a);
-        else hipLaunchKernelGGL((ck::ck_bwd_seq_kernel<VS, false>), grid, dim3(ck::NTS), 0, st, a);
+        return;
     }
+    with_flag(MT != 2 && a.mask != nullptr, [&](auto mask) {
+        constexpr bool MASK = MT != 2 && decltype(mask)::value;
+        with_flag(MT == 0 ? all_f32(a) : a.dy_dt == DT_F32, [&](auto f32) {
+            constexpr bool F32 = decltype(f32)::value;
+            if constexpr (MT >= 1)
+                hipLaunchKernelGGL((ck::ck_bwd_seq_bf16_kernel<VS, F32, MT == 2, MASK>), grid, dim3(ck::NTS), 0, st, a);
+            else
+                hipLaunchKernelGGL((ck::ck_bwd_seq_kernel<VS, F32, MASK>), grid, dim3(ck::NTS), 0, st, a);
+        });
+    });
 }
 
 template <int MT>
@@ -2115,36 +2270,39 @@ static void seq_dispatch(const ck::Args &a, hipStream_t st, bool fwd) {
 
 template <int MT>
 static void ck_fwd_launch(const ck::Args &a, hipStream_t st, const char *stage) {
-    if (stage[0] == 'p' && MT == 2)
-        ck::launch_vg_prep(a, st);
-    else if (stage[0] == 'p' && MT == 1)
-        hipLaunchKernelGGL(ck::ck_prep_bf16_kernel, dim3(a.NC, a.Hv, a.B), dim3(ck::NTP), 0, st, a);
-    else if (stage[0] == 'p' && all_f32(a))
-        hipLaunchKernelGGL(ck::ck_prep_kernel<true>, dim3(a.NC, a.Hv, a.B), dim3(ck::NTP), 0, st, a);
-    else if (stage[0] == 'p')
-        hipLaunchKernelGGL(ck::ck_prep_kernel<false>, dim3(a.NC, a.Hv, a.B), dim3(ck::NTP), 0, st, a);
-    else
+    if (stage[0] != 'p') {
         seq_dispatch<MT>(a, st, true);
+    } else if constexpr (MT == 2) {
+        ck::launch_vg_prep(a, st);
+    } else {
+        const dim3 grid(a.NC, a.Hv, a.B);
+        with_flag(a.mask != nullptr, [&](auto mask) {
+            constexpr bool MASK = decltype(mask)::value;
+            if constexpr (MT == 1) hipLaunchKernelGGL(ck::ck_prep_bf16_kernel<MASK>, grid, dim3(ck::NTP), 0, st, a);
+            else if (all_f32(a)) hipLaunchKernelGGL((ck::ck_prep_kernel<true, MASK>), grid, dim3(ck::NTP), 0, st, a);
+            else hipLaunchKernelGGL((ck::ck_prep_kernel<false, MASK>), grid, dim3(ck::NTP), 0, st, a);
+        });
+    }
 }
 
 template <int MT>
 static void ck_bwd_launch(const ck::Args &a, hipStream_t st, const char *stage) {
     if (stage[0] == 's') {
         seq_dispatch<MT>(a, st, false);
-    } else if (stage[0] == 'd') {
-        if constexpr (MT == 2) ck::launch_vg_dg(a, st);
     } else if constexpr (MT == 2) {
-        ck::launch_vg_local(a, st);
-    } else if constexpr (MT == 1) {
-        if (a.dy_dt == DT_F32)
-            hipLaunchKernelGGL(ck::ck_bwd_local_bf16_kernel<true>, dim3(a.NC, a.Hk, a.B), dim3(ck::NTB), 0, st, a);
-        else
-            hipLaunchKernelGGL(ck::ck_bwd_local_bf16_kernel<false>, dim3(a.NC, a.Hk, a.B), dim3(ck::NTB), 0, st, a);
+        if (stage[0] == 'd') ck::launch_vg_dg(a, st);
+        else ck::launch_vg_local(a, st);
+    } else {
+        const dim3 grid(a.NC, a.Hk, a.B);
+        with_flag(a.mask != nullptr, [&](auto mask) {
+            constexpr bool MASK = decltype(mask)::value;
+            with_flag(MT == 0 ? all_f32(a) : a.dy_dt == DT_F32, [&](auto f32) {
+                constexpr bool F32 = decltype(f32)::value;
+                if constexpr (MT == 1) hipLaunchKernelGGL((ck::ck_bwd_local_bf16_kernel<F32, MASK>), grid, dim3(ck::NTB), 0, st, a);
+                else hipLaunchKernelGGL((ck::ck_bwd_local_kernel<F32, MASK>), grid, dim3(ck::NTB), 0, st, a);
+            });
+        });
     }
-    else if (all_f32(a))
-        hipLaunchKernelGGL(ck::ck_bwd_local_kernel<true>, dim3(a.NC, a.Hk, a.B), dim3(ck::NTB), 0, st, a);
-    else
-        hipLaunchKernelGGL(ck::ck_bwd_local_kernel<false>, dim3(a.NC, a.Hk, a.B), dim3(ck::NTB), 0, st, a);
 }
 
 static int kernel_set(int in_dt, int gate) { return in_dt == DT_BF16 ? (gate_vec(gate) ? 2 : 1) : 0; }

@@ -259,6 +259,8 @@ struct Bufs {
     float *Gv;            // [B][Hv][NC][C][D]     G_rj log2(e), G_rj = sum_{u<=r} log d_uj within the chunk; row C-1: G_C
     unsigned short *QGb;  // [B][Hv][NC][C][D]     Q * exp(G), fragment order (the forward's A operand of Y)
     unsigned short *KDb;  // [B][Hv][NC][C][D]     K * exp(G_C - G), fragment order (ck_bwd_seq's A operand of dDelta)
+    // masked calls: the chunks that hold a masked token keep the transposed queries per value head, hi and lo
+    unsigned short *QMb;  // [B][Hv][NC][2][D][C]  Q~^T hi, lo (fragment order; in the place of Q^T)
     // per-channel decays (not log decays): what ck_bwd_local_vg leaves for ck_vg_dg, VGD_FLOATS per chunk-head
     float *vgd;
 };
@@ -297,12 +299,104 @@ struct Args {
     float *snap;
     int wc, win0, recompute;
     int fwd_only;  // forward-only: ck_prep writes only the tiles the sequential forward reads
+    // A masked call (gdn_mask.hip; NULL without a mask): cm [B][cm_stride] says which of the launch's chunks hold a
+    // masked token; there the query rows qm stand in the place of q (fp32 [tok][Hv][D], or bf16 with the lo plane qm_lo
+    // elements on), e v is added to the masked tokens' y (e [tok][Hv]), and the queries' gradient goes to xm (fp32
+    // [tok][Hv][D]).  mask, qm, e and xm have the token stride Ts of the inputs.
+    const uint8_t *mask, *cm;
+    const void *qm;
+    size_t qm_lo;
+    const float *e;
+    float *xm;
+    int cm_stride;
     int read_ahead;  // the launch's tiles outgrow the Infinity Cache: the sequential kernels read them ahead into L2
 };
 
 __device__ __forceinline__ size_t chunk_index(const Args &a, int b, int hv, int c) {
     return ((size_t)b * a.Hv + hv) * a.NC + c;
 }
+
+// Whether chunk c of a masked launch holds a masked token: the same for the whole workgroup, in a scalar register.
+__device__ __forceinline__ int chunk_flag(const Args &a, int b, int c) { return a.cm[(size_t)b * a.cm_stride + c]; }
+__device__ __forceinline__ bool flag_set(int flag) { return __builtin_amdgcn_readfirstlane(flag) != 0; }
+// Offset of a token's query row (elements of qm and of xm).
+__device__ __forceinline__ size_t query_row(const Args &a, int b, int t, int hv) {
+    return (((size_t)b * a.Ts + t) * a.Hv + hv) * D;
+}
+
+// The flags of a sequential kernel's chunks, each loaded a step before its first use: cur of the chunk being worked on,
+// nxt of the one being prefetched.
+template <bool MASK>
+struct ChunkFlags {
+    bool cur = false, nxt = false;
+    int ahead = 0;
+    __device__ __forceinline__ void start(const Args &a, int b, int c, int step, int end) {
+        if constexpr (MASK) {
+            nxt = flag_set(chunk_flag(a, b, c));
+            if (c + step != end) ahead = chunk_flag(a, b, c + step);
+        }
+    }
+    // entering chunk c (of those up to end, exclusive, by step)
+    __device__ __forceinline__ void enter(const Args &a, int b, int c, int step, int end) {
+        if constexpr (MASK) {
+            cur = nxt;
+            nxt = flag_set(ahead);
+            if (c + step != end && c + 2 * step != end) ahead = chunk_flag(a, b, c + 2 * step);
+        }
+    }
+};
+
+// fp32 set: the [C][D] query tile of a chunk with masked tokens, over the one just written to LDS from q (row stride
+// lds_stride, by load_tile or tile_store from inputs of dtype dt).  Each thread writes the pieces it wrote there, so no
+// barrier is needed between.
+template <int NTH>
+__device__ __forceinline__ void load_queries(float *dst, int lds_stride, const Args &a, int b, int hv, int t0, int n,
+                                             int dt, int tid) {
+    const int epq = dt == DT_F32 ? 4 : 8, vpr = D / epq;
+    for (int v = tid; v < C * vpr; v += NTH) {
+        const int r = v / vpr, c0 = (v - r * vpr) * epq;
+        if (r >= n) continue;
+        const float *src = static_cast<const float *>(a.qm) + query_row(a, b, t0 + r, hv) + c0;
+        for (int i = 0; i < epq; i += 4) {
+            const float4 x = *reinterpret_cast<const float4 *>(src + i);
+            float *d = dst + r * lds_stride + c0 + i;
+            d[0] = x.x; d[1] = x.y; d[2] = x.z; d[3] = x.w;
+        }
+    }
+}
+
+// x, unknown to the compiler from here on: addresses that only a masked chunk needs are formed from it in place instead
+// of being hoisted out of the chunk loop and held in registers by every step.
+__device__ __forceinline__ int opaque(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
+// The terms e v of a masked token's y, for an accumulator strip of rows m0.. and value tiles from column c0: loaded with
+// no branch (clamped rows) before they are used.
+template <int NTL>
+struct ValueTerms {
+    float e[4], v[NTL][4];
+    bool m[4];
+    __device__ __forceinline__ void load(const Args &a, int b, int hv, int t0, int n, int m0, int c0, int dt) {
+        const int l = opaque(threadIdx.x & 63);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = m0 + 4 * (l >> 4) + i, t = t0 + min(r, n - 1);
+            const size_t gi = ((size_t)b * a.Ts + t) * a.Hv + hv;
+            m[i] = r < n && a.mask[(size_t)b * a.Ts + t] == 0;
+            e[i] = a.e[gi];
+#pragma unroll
+            for (int x = 0; x < NTL; ++x) v[x][i] = load_as_f32(a.v, gi * D + c0 + 16 * x + (l & 15), dt);
+        }
+    }
+    __device__ __forceinline__ void add(f4 (&y)[NTL]) const {
+#pragma unroll
+        for (int x = 0; x < NTL; ++x)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) y[x][i] = m[i] ? y[x][i] + e[i] * v[x][i] : y[x][i];
+    }
+};
 
 // What a sequential forward launch writes.  FWD_TRAIN: y, the final state and the tiles the backward reads (H,
 // Delta); FWD_ONLY: y, the final state and the window snapshots (when Args::snap is set); FWD_RECOMPUTE: the windows

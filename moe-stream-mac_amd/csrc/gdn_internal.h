@@ -49,12 +49,13 @@ struct ChunkSizes {
     Buf H, G, T, P, W, U, Dl;         // tile set
     Buf Wb, KTb, Pb, PTb, QTb, nWTb;  // bf16 operand tiles of the bf16 set
     Buf Gv, QGb, KDb;                 // per-channel gates (bf16 set)
+    Buf QMb;                          // masked calls (bf16 set)
     size_t saved;                     // size of the tile set
     Buf dH, dDl, part, vgd;           // backward workspace
     size_t work;                      // its size
 };
-// vg: the per-channel gate kind (vg_kind), bf16 set only.
-ChunkSizes chunk_sizes(int B, int T, int Hk, int Hv, bool bf16, bool bwd, int vg = 0);
+// vg: the per-channel gate kind (vg_kind), bf16 set only; masked: a call with a mask.
+ChunkSizes chunk_sizes(int B, int T, int Hk, int Hv, bool bf16, bool bwd, int vg, bool masked);
 // The per-channel gate kind of a gate: 0 one decay per head, 1 per-channel log decays, 2 per-channel decays (whose
 // backward also keeps the pieces ck_vg_dg forms d/d(decay) from, in the vgd buffer).
 inline int vg_kind(int gate) { return gate == GATE_LOG_VEC ? 1 : gate == GATE_DECAY_VEC ? 2 : 0; }
@@ -71,6 +72,14 @@ struct ChunkCall {
     float *state_T, *dg, *dbeta, *dstate0;
     void *tiles, *work;
     float *snap;        // window snapshots (see ck::Args)
+    // masked calls (MaskArgs; mask NULL without one): g and beta are the effective gates; mask, qm, e and xm point at
+    // the launch's first token, cm at its first chunk
+    const uint8_t *mask, *cm;
+    const void *qm;
+    size_t qm_lo;
+    const float *e;
+    float *xm;
+    int cm_stride;  // chunks of a whole sequence
     int wc, win0, recompute, fwd_only;
     int B, T, Ts, Hk, Hv, in_dt, out_dt, dy_dt, grad_dt, gate;
 };
@@ -80,28 +89,27 @@ void launch_chunk_stage(const ChunkCall &cc, const char *stage, hipStream_t st);
 // The chunked form takes per-channel gates (GATE_DECAY_VEC, GATE_LOG_VEC) for bf16 inputs (gdn_chunk_vg.hip).
 bool chunk_vg_supported(int in_dt);
 
-// Masked steps on the chunked form (gdn_mask.hip): tensors of B*T tokens, contiguous; q, k [tok][Hk][Dk], v, y, dy
-// [tok][Hv][Dv], g, beta [tok][Hv] (the raw gates), mask [tok]; Z, Yp, dy1, dz and the passes' parts fp32.
+// Masked steps on the chunked form (gdn_mask.hip): tensors of B*T tokens, contiguous; q, k [tok][Hk][Dk], v, dy
+// [tok][Hv][Dv], g, beta [tok][Hv] (the raw gates), mask [tok].
 struct MaskArgs {
     const void *q, *k, *v, *dy;
     const float *g, *beta;
     const uint8_t *mask;
-    void *y;          // forward: holds y' on entry, y on exit
-    const float *Z;   // second pass output S' k
-    float *Yp;        // the first pass's fp32 output y' (read at masked tokens by the backward), or NULL
-    float *dy1, *dz;  // cotangents of the two passes
-    const float *dq1, *dk1, *dv1, *dg1, *dbeta1, *dq2, *dk2, *dv2, *dg2, *dbeta2;
+    // forward: the effective gates [tok][Hv]; the chunks that hold a masked token [B][ceil(T / 64)]; the queries
+    // [tok][Hv][Dk] of those chunks (fp32, or bf16 with the lo plane qm_lo elements on); the masked tokens' value
+    // factors e [tok][Hv]
+    float *g2, *beta2, *e;
+    void *qm;
+    size_t qm_lo;
+    uint8_t *cm;
+    const float *xm;  // backward: the queries' gradient [tok][Hv][Dk] in those chunks
     void *dq, *dk, *dv;
     float *dg, *dbeta;
-    int Hk, Hv, Dk, Dv, in_dt, out_dt, dy_dt, grad_dt, gate;
+    int B, T, Hk, Hv, Dk, Dv, in_dt, dy_dt, grad_dt, gate;
 };
 int mask_max_heads();
-void launch_mask_gates(const float *g, const float *beta, const uint8_t *mask, float *g2, float *beta2,
-                       size_t tokens, int Hv, int gate, hipStream_t st);
-void launch_mask_fix_fwd(const MaskArgs &a, size_t tokens, hipStream_t st);
-void launch_mask_bwd_cot(const MaskArgs &a, size_t tokens, hipStream_t st);
-void launch_mask_bwd_combine(const MaskArgs &a, size_t tokens, hipStream_t st);
-void launch_add2(float *dst, const float *x, const float *y, size_t n, hipStream_t st);
+void launch_mask_query(const MaskArgs &a, hipStream_t st);
+void launch_mask_bwd_fix(const MaskArgs &a, hipStream_t st);
 
 int pick_lane_width(int Dk);
 int rec_num_row_blocks(int Dv);

@@ -1,17 +1,24 @@
-// Masked steps on the chunked form: the elementwise pieces around two chunked passes.
+// Masked steps on the chunked form: what makes a masked call one chunked pass.
 //
 // A step with mask m_t = 0 keeps the state (S_t = S_{t-1}) but its output reads the candidate state
 // (tools/gdn_vjp.py:3-6, _step_parts :238-256):
-//   y_t = S~_t q_t = d_t S_{t-1} q_t + beta_t (k_t . q_t) (v_t - d_t S_{t-1} k_t)          (d_t the decay).
+//   y_t = S~_t q_t = d_t S_{t-1} q_t + beta_t c_t (v_t - d_t S_{t-1} k_t),   c_t = k_t . q_t      (d_t the decay).
 // The chunked form runs the effective recurrence with d'_t = m_t ? d_t : 1 and beta'_t = m_t beta_t, whose state
-// equals the masked recurrence's state at every token.  Its output y'_t = S'_t q_t is y_t where m_t = 1 and
-// S_{t-1} q_t where m_t = 0; a second pass with k as the query gives z_t = S'_t k_t = S_{t-1} k_t there.  Then at
-// masked tokens, with c = k_t . q_t (the value head's key head) and u = v_t - d_t z_t:
-//   y_t = d_t y'_t + beta_t c u
-// and the VJP of that expression feeds the two passes' backwards:
-//   dy'_t = d_t dy_t,  dz_t = -beta_t c d_t dy_t,  dv_t += beta_t c dy_t,  dbeta_t = c (u . dy_t),
-//   dd_t = (y'_t - beta_t c z_t) . dy_t,  dq_t += beta_t (u . dy_t) k_t,  dk_t += beta_t (u . dy_t) q_t
-// (dq / dk summed over the value heads of a key head).  Unmasked tokens pass dy through to the first pass.
+// equals the masked recurrence's state at every token.  y_t is linear in that state, so a masked token needs no pass of
+// its own, only another query (one per value head, as d and beta are) and a term that the state does not enter:
+//   y_t = S'_t q~_t + e_t v_t,   q~_t = d_t (q_t - beta_t c_t k_t),   e_t = beta_t c_t.
+// mask_query_kernel writes the effective gates, q~ and e of the masked tokens and which 64-token chunks hold one; the
+// chunked kernels read q~ in the place of q in those chunks (hi / lo planes in the bf16 set, whose q is exact where q~ is
+// not) and add e v to y.  The backward's only special output is X_t = dL/dq~_t: a masked token's k
+// and v enter nothing else (Delta_t = 0, beta'_t = 0), so all of its gradients follow from X_t and dy_t
+// (mask_bwd_fix_kernel):
+//   dv = e dy,   dc = beta (v . dy - d k . X),   dbeta = c (v . dy - d k . X),   dd = q . X - beta c k . X,
+//   dq = sum over the key head's value heads of d X + dc k,   dk = ... of dc q - d beta c X.
+//
+// The first form of this path ran the recurrence twice, the second time with k as the query, around fp32 copies of
+// every output, cotangent and gradient: at B = 4, T = 4096, Hv = 32, bf16, a fifth of the tokens masked, 3.78 ms per
+// forward + VJP, with the query rows 1.94 ms (1.56 ms without a mask).  Both kernels here are bound by the rows of the
+// masked tokens: 45 us (forward) and 82 us (backward) of that.
 #include "gdn_common.h"
 #include "gdn_internal.h"
 
@@ -19,15 +26,7 @@ namespace gdn {
 
 constexpr int MK_THREADS = 256;
 constexpr int MK_MAX_HEADS = 256;
-
-__global__ __launch_bounds__(256) void mask_gates_kernel(const float *g, const float *beta, const uint8_t *mask,
-                                                         float *g2, float *beta2, size_t n, int Hv, int gate) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const bool keep = mask[i / Hv] != 0;
-    g2[i] = keep ? g[i] : (gate == GATE_LOG ? 0.f : 1.f);
-    beta2[i] = keep ? beta[i] : 0.f;
-}
+static_assert(MK_MAX_HEADS <= MK_THREADS, "one thread per value head's gates");
 
 // Sum over the wave, the same bits in every lane: DPP row sums, then the lane swaps across rows and halves.
 __device__ __forceinline__ float wave_sum(float x) {
@@ -36,196 +35,138 @@ __device__ __forceinline__ float wave_sum(float x) {
     return x + lane_xor32(x);
 }
 
-// Four consecutive elements (i % 4 == 0) of a tensor of dtype dt, as fp32 / from fp32.
-__device__ __forceinline__ float4 load4(const void *p, size_t i, int dt) {
-    if (dt == DT_F32) return *reinterpret_cast<const float4 *>(static_cast<const float *>(p) + i);
-    if (dt == DT_BF16) {
-        const uint2 w = *reinterpret_cast<const uint2 *>(static_cast<const uint16_t *>(p) + i);
-        return make_float4(__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xffff0000u), __uint_as_float(w.y << 16),
-                           __uint_as_float(w.y & 0xffff0000u));
-    }
-    return make_float4(load_as_f32(p, i, dt), load_as_f32(p, i + 1, dt), load_as_f32(p, i + 2, dt),
-                       load_as_f32(p, i + 3, dt));
-}
-__device__ __forceinline__ void store4(void *p, size_t i, float4 x, int dt) {
-    if (dt == DT_F32) {
-        *reinterpret_cast<float4 *>(static_cast<float *>(p) + i) = x;
-    } else if (dt == DT_BF16) {
-        const uint32_t a = f32_to_bf16_cvt(x.x) | ((uint32_t)f32_to_bf16_cvt(x.y) << 16);
-        const uint32_t b = f32_to_bf16_cvt(x.z) | ((uint32_t)f32_to_bf16_cvt(x.w) << 16);
-        *reinterpret_cast<uint2 *>(static_cast<uint16_t *>(p) + i) = make_uint2(a, b);
-    } else {
-        store_from_f32(p, i, x.x, dt);
-        store_from_f32(p, i + 1, x.y, dt);
-        store_from_f32(p, i + 2, x.z, dt);
-        store_from_f32(p, i + 3, x.w, dt);
-    }
-}
-__device__ __forceinline__ float4 ld4f(const float *p, size_t i) { return *reinterpret_cast<const float4 *>(p + i); }
-__device__ __forceinline__ float4 add4(float4 a, float4 b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
-__device__ __forceinline__ float4 fma4(float s, float4 a, float4 b) {
-    return make_float4(fmaf(s, a.x, b.x), fmaf(s, a.y, b.y), fmaf(s, a.z, b.z), fmaf(s, a.w, b.w));
-}
-
 __device__ __forceinline__ float decay_of(const float *g, size_t gi, int gate) {
     return gate == GATE_LOG ? expf(g[gi]) : g[gi];
 }
 
-// c[hk] = k_t . q_t for every key head of token tok, one wave per key head (ends with a barrier).
-__device__ __forceinline__ void key_dots(const MaskArgs &a, size_t tok, float *c) {
-    const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
+// A row of D <= 128 elements (even) over a wave: lane l holds elements 2 l and 2 l + 1.
+__device__ __forceinline__ float2 load_row(const void *p, size_t base, int D, int l, int dt) {
+    const size_t i = base + 2 * l;
+    if (2 * l >= D) return make_float2(0.f, 0.f);
+    if (dt == DT_F32) return *reinterpret_cast<const float2 *>(static_cast<const float *>(p) + i);
+    const uint32_t w = *reinterpret_cast<const uint32_t *>(static_cast<const uint16_t *>(p) + i);
+    if (dt == DT_BF16) return make_float2(__uint_as_float(w << 16), __uint_as_float(w & 0xffff0000u));
+    return make_float2(__half2float(__ushort_as_half((unsigned short)(w & 0xffffu))),
+                       __half2float(__ushort_as_half((unsigned short)(w >> 16))));
+}
+__device__ __forceinline__ void store_row(void *p, size_t base, int D, int l, float2 x, int dt) {
+    const size_t i = base + 2 * l;
+    if (2 * l >= D) return;
+    if (dt == DT_F32) {
+        *reinterpret_cast<float2 *>(static_cast<float *>(p) + i) = x;
+    } else if (dt == DT_BF16) {
+        *reinterpret_cast<uint32_t *>(static_cast<uint16_t *>(p) + i) =
+            f32_to_bf16_cvt(x.x) | ((uint32_t)f32_to_bf16_cvt(x.y) << 16);
+    } else {
+        store_from_f32(p, i, x.x, dt);
+        store_from_f32(p, i + 1, x.y, dt);
+    }
+}
+__device__ __forceinline__ float dot_row(float2 x, float2 y) { return wave_sum(fmaf(x.x, y.x, x.y * y.y)); }
+
+// One workgroup per token, a wave per key head in turn: the effective gates, and in a chunk that holds a masked token the
+// query rows of the value heads (an unmasked token's is q, so that the chunked kernels pick q or qm by the chunk alone)
+// and e.  The workgroup of a chunk's first token writes the chunk's flag.
+__global__ __launch_bounds__(MK_THREADS) void mask_query_kernel(MaskArgs a) {
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+    const size_t tok = blockIdx.x;
+    const int b = (int)(tok / a.T), t = (int)(tok - (size_t)b * a.T), t0 = t - t % kChunkC;
+    const bool keep = a.mask[tok] != 0;
+    const bool any = __ballot(t0 + l < a.T && a.mask[(size_t)b * a.T + min(t0 + l, a.T - 1)] == 0) != 0;
+    if (t == t0 && threadIdx.x == 0) a.cm[(size_t)b * ((a.T + kChunkC - 1) / kChunkC) + t / kChunkC] = any;
+    if ((int)threadIdx.x < a.Hv) {  // Hv <= MK_MAX_HEADS
+        const size_t gi = tok * a.Hv + threadIdx.x;
+        a.g2[gi] = keep ? a.g[gi] : (a.gate == GATE_LOG ? 0.f : 1.f);
+        a.beta2[gi] = keep ? a.beta[gi] : 0.f;
+    }
+    if (!any) return;
+    const int rep = a.Hv / a.Hk;
+    if (w >= a.Hk) return;
+    const size_t row0 = (tok * a.Hk + w) * a.Dk;
+    float2 qn = load_row(a.q, row0, a.Dk, l, a.in_dt), kn = load_row(a.k, row0, a.Dk, l, a.in_dt);
     for (int hk = w; hk < a.Hk; hk += MK_THREADS / 64) {
-        const size_t base = (tok * a.Hk + hk) * a.Dk;
-        float s = 0.f;
-        for (int j = l; j < a.Dk; j += 64) s += load_as_f32(a.q, base + j, a.in_dt) * load_as_f32(a.k, base + j, a.in_dt);
-        s = wave_sum(s);
-        if (l == 0) c[hk] = s;
-    }
-    __syncthreads();
-}
-
-// Forward fix-up: y <- d y' + beta c (v - d z) at masked tokens, y' elsewhere.  With Yp set, y' is the first pass's
-// fp32 output there (kept for the backward) and every token's y is written; without, y holds y' in its own dtype
-// and only masked tokens are rewritten.
-__global__ __launch_bounds__(MK_THREADS) void mask_fix_fwd_kernel(MaskArgs a) {
-    const size_t tok = blockIdx.x;
-    const bool keep = a.mask[tok] != 0;
-    if (keep && !a.Yp) return;
-    __shared__ float c[MK_MAX_HEADS];
-    if (!keep) key_dots(a, tok, c);
-    const int rep = a.Hv / a.Hk;
-    // four consecutive elements per thread and step (Dv % 4 == 0)
-    for (int e = 4 * threadIdx.x; e < a.Hv * a.Dv; e += 4 * MK_THREADS) {
-        const size_t vi = tok * a.Hv * a.Dv + e;
-        float4 y = a.Yp ? ld4f(a.Yp, vi) : load4(a.y, vi, a.out_dt);
-        if (!keep) {
-            const int hv = e / a.Dv;
-            const size_t gi = tok * a.Hv + hv;
-            const float d = decay_of(a.g, gi, a.gate), bc = a.beta[gi] * c[hv / rep];
-            const float4 v = load4(a.v, vi, a.in_dt), z = ld4f(a.Z, vi);
-            y = make_float4(d * y.x + bc * (v.x - d * z.x), d * y.y + bc * (v.y - d * z.y), d * y.z + bc * (v.z - d * z.z),
-                            d * y.w + bc * (v.w - d * z.w));
+        const float2 q = qn, k = kn;
+        if (hk + MK_THREADS / 64 < a.Hk) {  // the wave's next key head, in flight during this one
+            const size_t row = (tok * a.Hk + hk + MK_THREADS / 64) * a.Dk;
+            qn = load_row(a.q, row, a.Dk, l, a.in_dt);
+            kn = load_row(a.k, row, a.Dk, l, a.in_dt);
         }
-        store4(a.y, vi, y, a.out_dt);
+        const float c = dot_row(q, k);
+        for (int hv = hk * rep; hv < (hk + 1) * rep; ++hv) {
+            const size_t gi = tok * a.Hv + hv, base = gi * a.Dk;
+            float2 x = q;
+            if (!keep) {
+                const float d = decay_of(a.g, gi, a.gate), e = a.beta[gi] * c;
+                if (l == 0) a.e[gi] = e;
+                x = make_float2(d * (q.x - e * k.x), d * (q.y - e * k.y));
+            }
+            if (a.in_dt == DT_BF16) {
+                store_row(a.qm, base, a.Dk, l, x, DT_BF16);
+                const float2 lo = make_float2(x.x - bf16_to_f32(f32_to_bf16_cvt(x.x)), x.y - bf16_to_f32(f32_to_bf16_cvt(x.y)));
+                store_row(a.qm, a.qm_lo + base, a.Dk, l, lo, DT_BF16);
+            } else {
+                store_row(a.qm, base, a.Dk, l, x, DT_F32);
+            }
+        }
     }
 }
 
-// Cotangents of the two passes: dy1 = (masked ? d dy : dy), dz = (masked ? -beta c d dy : 0), both fp32; four
-// consecutive elements per thread and step (Dv % 4 == 0).
-__global__ __launch_bounds__(MK_THREADS) void mask_bwd_cot_kernel(MaskArgs a) {
+// Every gradient of the masked tokens from X = dL/dq~ and dy: one workgroup per token, a wave per key head in turn, the
+// next value head's rows in flight.
+__global__ __launch_bounds__(MK_THREADS) void mask_bwd_fix_kernel(MaskArgs a) {
     const size_t tok = blockIdx.x;
-    const bool keep = a.mask[tok] != 0;
-    __shared__ float c[MK_MAX_HEADS];
-    if (!keep) key_dots(a, tok, c);
-    const int rep = a.Hv / a.Hk;
-    for (int e = 4 * threadIdx.x; e < a.Hv * a.Dv; e += 4 * MK_THREADS) {
-        const size_t vi = tok * a.Hv * a.Dv + e;
-        const float4 dy = load4(a.dy, vi, a.dy_dt);
-        float s1 = 1.f, sz = 0.f;
-        if (!keep) {
-            const int hv = e / a.Dv;
-            const size_t gi = tok * a.Hv + hv;
-            s1 = decay_of(a.g, gi, a.gate);
-            sz = -a.beta[gi] * c[hv / rep] * s1;
-        }
-        *reinterpret_cast<float4 *>(a.dy1 + vi) = make_float4(s1 * dy.x, s1 * dy.y, s1 * dy.z, s1 * dy.w);
-        *reinterpret_cast<float4 *>(a.dz + vi) = make_float4(sz * dy.x, sz * dy.y, sz * dy.z, sz * dy.w);
-    }
-}
-
-// Gradients: the two passes' fp32 parts summed (pass 2 ran with k as its query, so its dq adds to dk), the
-// chunked gate gradients kept where m = 1, and the fix-up's terms added where m = 0.
-__global__ __launch_bounds__(MK_THREADS) void mask_bwd_combine_kernel(MaskArgs a) {
-    const size_t tok = blockIdx.x;
-    const bool keep = a.mask[tok] != 0;
-    const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, rep = a.Hv / a.Hk;
-    __shared__ float c[MK_MAX_HEADS], su[MK_MAX_HEADS], sd[MK_MAX_HEADS];
-    if (!keep) {
-        key_dots(a, tok, c);
-        for (int hv = w; hv < a.Hv; hv += MK_THREADS / 64) {
-            const size_t gi = tok * a.Hv + hv, base = gi * a.Dv;
-            const float d = decay_of(a.g, gi, a.gate), bc = a.beta[gi] * c[hv / rep];
-            float s = 0.f, dd = 0.f;
-            for (int i = l; i < a.Dv; i += 64) {
-                const float dy = load_as_f32(a.dy, base + i, a.dy_dt), z = a.Z[base + i];
-                s += (load_as_f32(a.v, base + i, a.in_dt) - d * z) * dy;
-                dd += (a.Yp[base + i] - bc * z) * dy;
-            }
-            s = wave_sum(s);
-            dd = wave_sum(dd);
-            if (l == 0) {
-                su[hv] = s;
-                sd[hv] = dd;
-            }
-        }
-        __syncthreads();
-    }
-    // four consecutive elements per thread and step (Dk, Dv % 4 == 0)
-    for (int e = 4 * tid; e < a.Hk * a.Dk; e += 4 * MK_THREADS) {
-        const int hk = e / a.Dk;
-        const size_t i = tok * a.Hk * a.Dk + e;
-        float4 dq = ld4f(a.dq1, i), dk = add4(add4(ld4f(a.dk1, i), ld4f(a.dk2, i)), ld4f(a.dq2, i));
-        if (!keep) {
-            float f = 0.f;
-            for (int r = 0; r < rep; ++r) {
-                const int hv = hk * rep + r;
-                f += a.beta[tok * a.Hv + hv] * su[hv];
-            }
-            dq = fma4(f, load4(a.k, i, a.in_dt), dq);
-            dk = fma4(f, load4(a.q, i, a.in_dt), dk);
-        }
-        store4(a.dq, i, dq, a.grad_dt);
-        store4(a.dk, i, dk, a.grad_dt);
-    }
-    for (int e = 4 * tid; e < a.Hv * a.Dv; e += 4 * MK_THREADS) {
-        const size_t i = tok * a.Hv * a.Dv + e;
-        float4 dv = add4(ld4f(a.dv1, i), ld4f(a.dv2, i));
-        if (!keep) {
-            const int hv = e / a.Dv;
-            dv = fma4(a.beta[tok * a.Hv + hv] * c[hv / rep], load4(a.dy, i, a.dy_dt), dv);
-        }
-        store4(a.dv, i, dv, a.grad_dt);
-    }
-    for (int hv = tid; hv < a.Hv; hv += MK_THREADS) {
+    if (a.mask[tok] != 0) return;
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63, rep = a.Hv / a.Hk;
+    struct Rows {
+        float2 X, v, dy;
+        float g, beta;
+    };
+    auto load = [&](int hv) {
         const size_t gi = tok * a.Hv + hv;
-        if (keep) {
-            a.dg[gi] = a.dg1[gi] + a.dg2[gi];
-            a.dbeta[gi] = a.dbeta1[gi] + a.dbeta2[gi];
-        } else {
-            a.dg[gi] = a.gate == GATE_LOG ? decay_of(a.g, gi, a.gate) * sd[hv] : sd[hv];
-            a.dbeta[gi] = c[hv / rep] * su[hv];
+        return Rows{load_row(a.xm, gi * a.Dk, a.Dk, l, DT_F32), load_row(a.v, gi * a.Dv, a.Dv, l, a.in_dt),
+                    load_row(a.dy, gi * a.Dv, a.Dv, l, a.dy_dt), a.g[gi], a.beta[gi]};
+    };
+    if (w >= a.Hk) return;
+    Rows nx = load(w * rep);
+    for (int hk = w; hk < a.Hk; hk += MK_THREADS / 64) {
+        const size_t qb = (tok * a.Hk + hk) * a.Dk;
+        const float2 q = load_row(a.q, qb, a.Dk, l, a.in_dt), k = load_row(a.k, qb, a.Dk, l, a.in_dt);
+        const float c = dot_row(q, k);
+        float2 dq = make_float2(0.f, 0.f), dk = dq;
+        for (int hv = hk * rep; hv < (hk + 1) * rep; ++hv) {
+            const Rows r = nx;
+            const int nhv = hv + 1 < (hk + 1) * rep ? hv + 1 : (hk + MK_THREADS / 64) * rep;
+            if (nhv < a.Hv) nx = load(nhv);
+            const size_t gi = tok * a.Hv + hv;
+            const float d = a.gate == GATE_LOG ? expf(r.g) : r.g, e = r.beta * c;
+            const float kx = dot_row(k, r.X), qx = dot_row(q, r.X), u = dot_row(r.v, r.dy) - d * kx;
+            const float dc = r.beta * u, de = d * e;
+            dq.x += d * r.X.x + dc * k.x;
+            dq.y += d * r.X.y + dc * k.y;
+            dk.x += dc * q.x - de * r.X.x;
+            dk.y += dc * q.y - de * r.X.y;
+            store_row(a.dv, gi * a.Dv, a.Dv, l, make_float2(e * r.dy.x, e * r.dy.y), a.grad_dt);
+            if (l == 0) {
+                const float dd = qx - e * kx;
+                a.dg[gi] = a.gate == GATE_LOG ? d * dd : dd;
+                a.dbeta[gi] = c * u;
+            }
         }
+        store_row(a.dq, qb, a.Dk, l, dq, a.grad_dt);
+        store_row(a.dk, qb, a.Dk, l, dk, a.grad_dt);
     }
-}
-
-__global__ __launch_bounds__(256) void add2_kernel(float *dst, const float *x, const float *y, size_t n) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) dst[i] = x[i] + y[i];
 }
 
 int mask_max_heads() { return MK_MAX_HEADS; }
 
-void launch_mask_gates(const float *g, const float *beta, const uint8_t *mask, float *g2, float *beta2,
-                       size_t tokens, int Hv, int gate, hipStream_t st) {
-    const size_t n = tokens * Hv;
-    if (n) hipLaunchKernelGGL(mask_gates_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, g, beta, mask,
-                              g2, beta2, n, Hv, gate);
+void launch_mask_query(const MaskArgs &a, hipStream_t st) {
+    const size_t tokens = (size_t)a.B * a.T;
+    if (tokens) hipLaunchKernelGGL(mask_query_kernel, dim3((unsigned)tokens), dim3(MK_THREADS), 0, st, a);
 }
 
-void launch_mask_fix_fwd(const MaskArgs &a, size_t tokens, hipStream_t st) {
-    if (tokens) hipLaunchKernelGGL(mask_fix_fwd_kernel, dim3((unsigned)tokens), dim3(MK_THREADS), 0, st, a);
-}
-
-void launch_mask_bwd_cot(const MaskArgs &a, size_t tokens, hipStream_t st) {
-    if (tokens) hipLaunchKernelGGL(mask_bwd_cot_kernel, dim3((unsigned)tokens), dim3(MK_THREADS), 0, st, a);
-}
-
-void launch_mask_bwd_combine(const MaskArgs &a, size_t tokens, hipStream_t st) {
-    if (tokens) hipLaunchKernelGGL(mask_bwd_combine_kernel, dim3((unsigned)tokens), dim3(MK_THREADS), 0, st, a);
-}
-
-void launch_add2(float *dst, const float *x, const float *y, size_t n, hipStream_t st) {
-    if (dst && n) hipLaunchKernelGGL(add2_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, dst, x, y, n);
+void launch_mask_bwd_fix(const MaskArgs &a, hipStream_t st) {
+    const size_t tokens = (size_t)a.B * a.T;
+    if (tokens) hipLaunchKernelGGL(mask_bwd_fix_kernel, dim3((unsigned)tokens), dim3(MK_THREADS), 0, st, a);
 }
 
 }  // namespace gdn
