@@ -1256,10 +1256,17 @@ __global__ __launch_bounds__(NTB) void ck_bwd_local_bf16_kernel(Args a) {
 
 // ---------------------------------------------------------------------------------------------- ck_fwd (bf16)
 //
-// Sequential over chunks like ck_fwd_kernel, for bf16 inputs.  The A operands of every product (W, Q, P hi / lo,
+// Sequential over chunks like ck_fwd_kernel, for bf16 inputs.  The A operands of the products (W, P hi / lo,
 // (K diag(gamma_C/gamma))^T) are read as MFMA fragments straight from global memory into registers, one chunk
-// ahead (ck_prep wrote them as bf16 tiles); LDS only carries what the waves exchange each chunk: h as the
-// operand [i][j] (hi / lo) and Delta as [i][r] (hi / lo).  Two barriers per chunk.
+// ahead (ck_prep wrote them as bf16 tiles); LDS carries what the waves exchange each chunk, h as the operand [i][j]
+// (hi / lo) and Delta as [i][r] (hi / lo), and Q.  Two barriers per chunk.
+//
+// Q (and K in the backward) is read from the input, whose rows are a fragment's rows: loaded as fragments, the 16 lanes
+// that the L1 takes at a time read 16 different lines, and such a load costs 64 line accesses where a tile in fragment
+// order costs 8 (a read of 64 KiB per CU and step from L2: 1.74 against 0.61 us).  It is loaded by whole rows instead
+// (16 lanes to one) and turned into fragments through LDS, which also frees 24 registers: ck_bwd_seq_bf16 330 -> 282 us
+// (with the reading ahead that the registers leave room for), ck_fwd_bf16 350 -> 335 us at B = 4, T = 4096, Hv = 32; 152
+// -> 142 and 166 -> 142 us at B = 1, T = 4001.
 
 // Reading ahead (slices narrower than 64).  The D / VS workgroups of a head ask for the same tiles at the same time,
 // so a line that is not in L2 yet is missed by each of them, and the loads of the next chunk, issued one step ahead,
@@ -1267,14 +1274,32 @@ __global__ __launch_bounds__(NTB) void ck_bwd_local_bf16_kernel(Args a) {
 // therefore reads one 4-byte word of its own share (1 / (D / VS)) of the shared lines of the chunk kReadAhead steps on
 // (at most one load per thread and step), so each line leaves memory once and the fragment loads hit L2.  At B = 1,
 // T = 4001, Hv = 32: ck_fwd_bf16 188 -> 166 us, ck_bwd_seq_bf16 170 -> 152 us; at B = 2, T = 2048: 148 -> 129 and
-// 135 -> 125 us; three, four and six steps ahead gain less (170, 179, 184 us forward at B = 1).  At 64-wide slices the
-// kernels have no register to spare for it (forward at B = 4: 346 -> 373 us).  Args::read_ahead says whether the
+// 135 -> 125 us; three, four and six steps ahead gain less (170, 179, 184 us forward at B = 1).  At 64-wide slices
+// the backward takes it (B = 4, T = 4096: 334 -> 282 us) and the forward has no use for it (335 us with and without);
+// masked (343 -> 363 us) and per-channel launches of that width have no registers for it.  Args::read_ahead says whether the
 // launch's tiles outgrow the cache.
 constexpr int kReadAhead = 2, kLine = 128;  // bytes of an L2 line
 
-template <int DN>
+// A [C][D] bf16 tile of the input (row stride rs elements) by whole rows, two 16-byte pieces per thread; rows past n read
+// as zero.
+__device__ __forceinline__ void load_row_tile(uint4 (&x)[2], const bfr *p, unsigned rs, int n, int tid) {
+    static_assert(C * D / 8 == 2 * NTS, "two pieces per thread");
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int r = (tid + i * NTS) / (D / 8);
+        const uint4 v = *reinterpret_cast<const uint4 *>(p + (unsigned)min(r, n - 1) * rs + 8 * (tid % (D / 8)));
+        x[i] = r < n ? v : make_uint4(0u, 0u, 0u, 0u);
+    }
+}
+__device__ __forceinline__ void store_row_tile(bfr *dst, const uint4 (&x)[2], int tid) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        *reinterpret_cast<uint4 *>(dst + ((tid + i * NTS) / (D / 8)) * LA + 8 * (tid % (D / 8))) = x[i];
+}
+
+template <int DN, bool QF>
 struct FwdFrags {
-    bf8 W[4], Q[4], P[4], K[2];  // P[0..1] hi, P[2..3] lo
+    bf8 W[4], Q[QF ? 4 : 1], P[4], K[2];  // P[0..1] hi, P[2..3] lo; Q where it is read as fragments
     float U[DN][4];
     double g;
     float4 gc;  // per-channel gates: G_C of this lane's four state rows
@@ -1291,6 +1316,11 @@ __global__ __launch_bounds__(NTS) void ck_fwd_bf16_kernel(Args a) {
     __shared__ __align__(16) bfr sHl[VS * LH];
     __shared__ __align__(16) bfr sDh[VS * LDd];
     __shared__ __align__(16) bfr sDl[VS * LDd];
+    // Q staged by rows, or read as fragments: from ck_prep's tile with per-channel gates, and from the input in a
+    // forward-only launch of 16-wide slices, whose operands are still in L2 (102 against 109 us at B = 1, T = 4096);
+    // recomputed windows write no y
+    constexpr bool kQF = VG || (VS == 16 && MODE == FWD_ONLY), kRows = !kQF && kOut;
+    __shared__ __align__(16) bfr sQ[kRows ? C * LA : 8];  // Q [r][j]
     __shared__ float sGamBuf[2][C];  // by chunk parity: read after the second barrier, rewritten two chunks later
 
     const SeqBlock sb = seq_block();
@@ -1314,20 +1344,25 @@ __global__ __launch_bounds__(NTS) void ck_fwd_bf16_kernel(Args a) {
             h[t][e] = sr.s0 ? sr.s0[(head * D + i) * D + j] : 0.f;
         }
     ChunkFlags<MASK> flags;
-    auto fetch = [&](FwdFrags<DN> &f, int c) {
+    uint4 qr[2];  // this thread's pieces of the next chunk's Q
+    auto fetch = [&](FwdFrags<DN, kQF> &f, int c) {
         const size_t ci = head * a.NC + c;
-        const int t0 = c * C, n = min(C, T - t0), r = mrow + li;
+        const int t0 = c * C, n = min(C, T - t0);
         const bfr *wb = a.w.Wb + ci * C * D + frag_off<D>(mrow, 0) + 8 * l;
         const bfr *pb = a.w.Pb + ci * 2 * C * C + frag_off<C>(mrow, 0) + 8 * l;
         const bfr *kt = a.w.KTb + ci * D * C + frag_off<C>(16 * w, 0) + 8 * l;
-        // q, or a masked chunk's query rows (hi): a scalar choice of the tile's first row and of the row stride
-        const bfr *q0 = static_cast<const bfr *>(a.q) + (((size_t)b * a.Ts + t0) * a.Hk + hk) * D;
-        int q_row = a.Hk * D;
-        if (flags.nxt) {
-            q0 = static_cast<const bfr *>(a.qm) + query_row(a, b, t0, hv);
-            q_row = a.Hv * D;
+        const bfr *qf = nullptr;
+        unsigned q_row = a.Hk * D;
+        if constexpr (!VG && kOut) {
+            // q, or a masked chunk's query rows (hi): a scalar choice of the tile's first row and of the row stride
+            const bfr *q0 = static_cast<const bfr *>(a.q) + (((size_t)b * a.Ts + t0) * a.Hk + hk) * D;
+            if (flags.nxt) {
+                q0 = static_cast<const bfr *>(a.qm) + query_row(a, b, t0, hv);
+                q_row = a.Hv * D;
+            }
+            if constexpr (kRows) load_row_tile(qr, q0, q_row, n, tid);
+            qf = q0 + (unsigned)min(mrow + li, n - 1) * q_row + 8 * lg;
         }
-        const bfr *qb = q0 + (size_t)r * q_row + 8 * lg;
         const bfr *qg = VG ? a.w.QGb + ci * C * D + frag_off<D>(mrow, 0) + 8 * l : nullptr;
         // W and U in the waves that form Delta, Q and P in the waves that form y
         if (dwave) {
@@ -1338,7 +1373,7 @@ __global__ __launch_bounds__(NTS) void ck_fwd_bf16_kernel(Args a) {
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 if constexpr (VG) f.Q[k] = ld_frag(qg + FRAG_BLOCK * k);
-                else f.Q[k] = r < n ? ld_frag(qb + 32 * k) : zero_frag();
+                else if constexpr (kQF) f.Q[k] = ld_frag(qf + 32 * k);  // rows past n reach only rows of y not stored
             }
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
@@ -1382,7 +1417,7 @@ __global__ __launch_bounds__(NTS) void ck_fwd_bf16_kernel(Args a) {
     };
     // The chunk loop is unrolled by two over ping-pong fragment buffers: no register copy of the prefetched
     // fragments, so the wait for them sits at their first use, one chunk step after the loads were issued.
-    auto step = [&](const int c, FwdFrags<DN> &cur, FwdFrags<DN> &nxt) {
+    auto step = [&](const int c, FwdFrags<DN, kQF> &cur, FwdFrags<DN, kQF> &nxt) {
         const int t0 = c * C, n = min(C, T - t0);
         const size_t ci = head * a.NC + c;
         if (float *sp = snap_at<MODE>(a, c)) store_state_acc<NTN>(sp, h, head, i0, w, lg, li);
@@ -1398,6 +1433,7 @@ __global__ __launch_bounds__(NTS) void ck_fwd_bf16_kernel(Args a) {
                         (bfr)bfbits(h[t][e]);
             }
         }
+        if constexpr (kRows) store_row_tile(sQ, qr, tid);
         float *const sGam = sGamBuf[c & 1];
         if (!VG && tid < C) sGam[tid] = __builtin_amdgcn_exp2f((float)(cur.g * 1.4426950408889634));  // v_exp_f32 on log2 units
         __syncthreads();
@@ -1412,7 +1448,10 @@ __global__ __launch_bounds__(NTS) void ck_fwd_bf16_kernel(Args a) {
 #pragma unroll
         for (int t = 0; t < DN; ++t) wh[t] = zero4();
         if (dwave) mmar<D, DN>(wh, cur.W, nullptr, sHh, nullptr, LH, 16 * nt0);
-        if (ywave) mmar<D, DN, false, true>(yi, cur.Q, nullptr, sHh, sHl, LH, 16 * nt0);
+        if (ywave) {
+            if constexpr (kQF) mmar<D, DN, false, true>(yi, cur.Q, nullptr, sHh, sHl, LH, 16 * nt0);
+            else if constexpr (kRows) mmab<D, DN, false, true>(yi, sQ, nullptr, LA, mrow, sHh, sHl, LH, 16 * nt0, l);
+        }
         // a masked chunk's own loads, the lo part of its queries and its value terms, go out here, where the registers of
         // W, Q and U fall free (64-wide slices have none to spare before), and arrive during Delta's conversion
         ValueTerms<DN> vt;
@@ -1492,7 +1531,7 @@ __global__ __launch_bounds__(NTS) void ck_fwd_bf16_kernel(Args a) {
         }
         mmar<C, NTN>(h, cur.K, nullptr, sDh, nullptr, LDd, 0);
     };
-    FwdFrags<DN> fa, fb;
+    FwdFrags<DN, kQF> fa, fb;
     flags.start(a, b, cb, 1, ce);
     fetch(fa, cb);
     for (int c = cb; c < ce; c += 2) {
@@ -1819,13 +1858,13 @@ __global__ __launch_bounds__(NTP, 2) void ck_prep_bf16_kernel(Args a) {
 // exit state (this workgroup's value slice, in MFMA accumulators):
 //   dDelta = diag(rc) K dh' + P^T dY,   dh = gamma_C dh' + Q^T diag(gamma) dY - W^T dDelta,
 // and it saves TdD = T^T dDelta (fp32 [C][D]), the only form in which ck_bwd_local_bf16 needs T and dDelta.
-// The A operands (K straight from the input, P^T hi / lo, Q^T and -W^T written by ck_prep) are read as MFMA
-// fragments from global memory into registers one chunk ahead, with the chunk's dY slice; LDS carries what the
-// waves exchange: dh' as the operand [i][j] (hi / lo), dY^T, (diag(gamma) dY)^T (hi / lo) and dDelta^T (hi / lo),
-// and T^T (hi / lo, fragment order), whose 32 bytes per thread are loaded one chunk ahead and stored between the
+// The A operands P^T (hi / lo), Q^T and -W^T, written by ck_prep, are read as MFMA fragments from global memory into
+// registers one chunk ahead, with the chunk's dY slice; LDS carries what the waves exchange: dh' as the operand [i][j]
+// (hi / lo), dY^T, (diag(gamma) dY)^T (hi / lo) and dDelta^T (hi / lo), K (by rows, as the forward's Q), and T^T (hi / lo, fragment order), whose 32 bytes per thread are loaded one chunk ahead and stored between the
 // two barriers of the chunk that uses them.  Two barriers per chunk.
+template <bool VG>
 struct BwdFrags {
-    bf8 K[4], PT[4], QT[2], WT[2];  // PT[0..1] hi, PT[2..3] lo; WT = -W^T
+    bf8 K[VG ? 4 : 1], PT[4], QT[2], WT[2];  // K: per-channel gates only; PT[0..1] hi, PT[2..3] lo; WT = -W^T
     double g;
     float4 gc;  // per-channel gates: G_C of this lane's four state rows
 };
@@ -1846,6 +1885,7 @@ __global__ __launch_bounds__(NTS) void ck_bwd_seq_bf16_kernel(Args a) {
     __shared__ __align__(16) bfr sDd[VS * LDd];   // dDelta^T [i][r], hi
     __shared__ __align__(16) bfr sDdl[VS * LDd];  // dDelta^T lo
     __shared__ __align__(16) bfr sTT[2 * C * C];  // T^T hi, lo (fragment order)
+    __shared__ __align__(16) bfr sK[VG ? 8 : C * LA];  // K [r][j]
     __shared__ float sGam[C], sRc[C];
     static_assert(2 * C * C / 8 == 2 * NTS, "two 16-byte pieces of T^T per thread");
 
@@ -1881,10 +1921,11 @@ __global__ __launch_bounds__(NTS) void ck_bwd_seq_bf16_kernel(Args a) {
     };
     using YRaw = typename std::conditional<DYF32, float2, uint32_t>::type;
     ChunkFlags<MASK> flags;
-    auto fetch = [&](BwdFrags &f, YRaw (&y)[8], int c) {
+    uint4 kr[2];  // this thread's pieces of the next chunk's K
+    auto fetch = [&](BwdFrags<VG> &f, YRaw (&y)[8], int c) {
         const size_t ci = head * a.NC + c;
-        const int t0 = c * C, n = min(C, T - t0), r = mrow + li;
-        const bfr *kb = static_cast<const bfr *>(a.k) + (((size_t)b * a.Ts + t0 + r) * a.Hk + hk) * D + 8 * lg;
+        const int t0 = c * C, n = min(C, T - t0);
+        if constexpr (!VG) load_row_tile(kr, static_cast<const bfr *>(a.k) + (((size_t)b * a.Ts + t0) * a.Hk + hk) * D, a.Hk * D, n, tid);
         const bfr *kd = VG ? a.w.KDb + ci * C * D + frag_off<D>(mrow, 0) + 8 * l : nullptr;
         const bfr *pt = a.w.PTb + ci * 2 * C * C + frag_off<C>(mrow, 0) + 8 * l;
         const bfr *qt0 = a.w.QTb + (VG ? ci : ((size_t)b * a.Hk + hk) * a.NC + c) * D * C;
@@ -1896,7 +1937,6 @@ __global__ __launch_bounds__(NTS) void ck_bwd_seq_bf16_kernel(Args a) {
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 if constexpr (VG) f.K[k] = ld_frag(kd + FRAG_BLOCK * k);
-                else f.K[k] = r < n ? ld_frag(kb + 32 * k) : zero_frag();
             }
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
@@ -1924,12 +1964,13 @@ __global__ __launch_bounds__(NTS) void ck_bwd_seq_bf16_kernel(Args a) {
             }
         }
     };
+    constexpr bool RA = VS < 64 || (!VG && !MASK);  // (kReadAhead)
     uint32_t ahead = 0;
     auto read_ahead = [&](int c) {
         // threads below LPS: this slice's share of the 640 lines of P^T, Q^T, -W^T, T^T and K; threads 384..447: dY's
         // rows of the slice
         constexpr int S = D / VS, LPS = 5 * kLine / S;
-        static_assert(VS >= 64 || LPS <= 384, "the two groups of threads are apart");
+        static_assert(LPS <= 384, "the two groups of threads are apart");
         const size_t ci = head * a.NC + c;
         const char *p = nullptr;
         if (tid < LPS) {
@@ -1952,7 +1993,7 @@ __global__ __launch_bounds__(NTS) void ck_bwd_seq_bf16_kernel(Args a) {
     // unrolled by two over ping-pong fragment buffers, as in ck_fwd_bf16_kernel; both steps of a pair are
     // unconditional (a prefetch used only under a branch is sunk to its use by the compiler)
     YRaw yr[8];
-    auto step = [&](const int c, BwdFrags &cur, BwdFrags &nxt) {
+    auto step = [&](const int c, BwdFrags<VG> &cur, BwdFrags<VG> &nxt) {
         const size_t ci = head * a.NC + c;
         flags.enter(a, b, c, -1, -1);
         // dh' -> LDS as the operand [i][j] (hi / lo) and -> the saved dH ([j][i], fp32)
@@ -1964,6 +2005,7 @@ __global__ __launch_bounds__(NTS) void ck_bwd_seq_bf16_kernel(Args a) {
                 reinterpret_cast<bfr *>(a.w.dH)[ci * D * D + (size_t)(16 * w + 4 * lg + e) * D + i0 + 16 * t + li] =
                     (bfr)bfbits(dh[t][e]);
         }
+        if constexpr (!VG) store_row_tile(sK, kr, tid);
         // dY^T (exact for bf16 dY) and the gates
         float yv[8][2];
         if (ythr) {
@@ -2009,15 +2051,16 @@ __global__ __launch_bounds__(NTS) void ck_bwd_seq_bf16_kernel(Args a) {
         // first barrier of this one); the next chunk's pieces are loaded after the second barrier
         reinterpret_cast<uint4 *>(sTT)[tid] = ttr0;
         reinterpret_cast<uint4 *>(sTT)[tid + NTS] = ttr1;
-        if constexpr (VS < 64) asm volatile("" ::"v"(ahead));  // the previous step's read
+        if constexpr (RA) asm volatile("" ::"v"(ahead));  // the previous step's read
         if (c > 0) fetch(nxt, yr, c - 1);
-        if (VS < 64 && a.read_ahead && c >= kReadAhead) read_ahead(c - kReadAhead);
+        if (RA && a.read_ahead && c >= kReadAhead) read_ahead(c - kReadAhead);
         // dDelta = diag(rc) K dh' + P^T dY
         if (cwave) {
             f4 kd[DN], pd[DN];
 #pragma unroll
             for (int t = 0; t < DN; ++t) kd[t] = pd[t] = zero4();
-            mmar<D, DN, false, true>(kd, cur.K, nullptr, sHh, sHl, LH, 16 * nt0);
+            if constexpr (VG) mmar<D, DN, false, true>(kd, cur.K, nullptr, sHh, sHl, LH, 16 * nt0);
+            else mmab<D, DN, false, true>(kd, sK, nullptr, LA, mrow, sHh, sHl, LH, 16 * nt0, l);
             mmar<C, DN, true, false>(pd, cur.PT, cur.PT + 2, sY, nullptr, LDd, 16 * nt0);
 #pragma unroll
             for (int t = 0; t < DN; ++t) {
@@ -2081,7 +2124,7 @@ __global__ __launch_bounds__(NTS) void ck_bwd_seq_bf16_kernel(Args a) {
                     dh[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ql[MASK ? k : 0], frag(sYgh, LDd, 16 * t, 32 * k), dh[t], 0, 0, 0);
         }
     };
-    BwdFrags fa, fb;
+    BwdFrags<VG> fa, fb;
     flags.start(a, b, a.NC - 1, -1, -1);
     fetch(fa, yr, a.NC - 1);
     fetch_tt(a.NC - 1);

@@ -382,12 +382,14 @@ struct ValueTerms {
         const int l = opaque(threadIdx.x & 63);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int r = m0 + 4 * (l >> 4) + i, t = t0 + min(r, n - 1);
-            const size_t gi = ((size_t)b * a.Ts + t) * a.Hv + hv;
-            m[i] = r < n && a.mask[(size_t)b * a.Ts + t] == 0;
-            e[i] = a.e[gi];
+            // one 32-bit lane offset per row from uniform addresses
+            const int r = m0 + 4 * (l >> 4) + i;
+            const unsigned rc = min(r, n - 1), gi = rc * a.Hv, vi = gi * D + (l & 15);
+            m[i] = r < n && (a.mask + (size_t)b * a.Ts + t0)[rc] == 0;
+            e[i] = (a.e + ((size_t)b * a.Ts + t0) * a.Hv + hv)[gi];
+            const void *vt = elem_ptr(a.v, (((size_t)b * a.Ts + t0) * a.Hv + hv) * D + c0, dt);
 #pragma unroll
-            for (int x = 0; x < NTL; ++x) v[x][i] = load_as_f32(a.v, gi * D + c0 + 16 * x + (l & 15), dt);
+            for (int x = 0; x < NTL; ++x) v[x][i] = load_as_f32(vt, vi + 16 * x, dt);
         }
     }
     __device__ __forceinline__ void add(f4 (&y)[NTL]) const {
