@@ -146,6 +146,28 @@ int gdn_decode_step(const void *q, const void *k, const void *v, const float *g,
                     const float *state_in, float *state_out, void *y, int B, int Hk, int Hv, int Dk, int Dv,
                     int in_dtype, int out_dtype, int gate_kind, void *stream);
 
+/* One decoded token of a whole GDN block (the steps of engine/src/gdn_layer.c:18-58), batched over B sequences, in
+ * three launches: gdn_small_linears over the in-projections, gdn_block_decode, gdn_small_linears over the out-projection.
+ *
+ * gdn_small_linears: y[i] [tokens][n[i]] = x [tokens][k] * w[i]^T, w[i] [n[i]][k], for count <= 4 weights that share x;
+ * one dtype throughout, fp32 sums.  At most 16 tokens, k a multiple of 8 (else GDN_ERR_UNSUPPORTED); x and the weights
+ * 16-byte aligned.  The arrays w, y and n are read during the call.
+ *
+ * gdn_block_decode: from the projections' outputs qkv [B][2 Hk Dk + Hv Dv], z [B][Hv Dv], b and a [B][Hv] (dtype) the
+ * causal conv step + SiLU (conv_w [C][K], the last tap on the current input), the split, the q / k L2 norms (q times
+ * q_scale), the gates (decay from A_log and dt_bias [Hv], beta = sigmoid(b)), the delta rule, and the gated RMSNorm
+ * (norm_w [Dv]): out [B][Hv Dv] (dtype).  conv_in / conv_out [B][K - 1][C] fp32 (oldest first; not the same buffer) and
+ * state_in / state_out [B][Hv][Dv][Dk] fp32 (may be the same) are the caches before and after the token; conv_in and
+ * state_in may be NULL (zeros).  The parameters' dtypes are given one by one.  Dk = Dv = 128 and K = 4 (else
+ * GDN_ERR_UNSUPPORTED). */
+int gdn_small_linears(const void *x, const void *const *w, void *const *y, const int *n, int count, int tokens, int k,
+                      int dtype, void *stream);
+int gdn_block_decode(const void *qkv, const void *z, const void *b, const void *a, const void *conv_w, const void *A_log,
+                     const void *dt_bias, const void *norm_w, const float *conv_in, float *conv_out,
+                     const float *state_in, float *state_out, void *out, int B, int Hk, int Hv, int Dk, int Dv, int K,
+                     int dtype, int conv_dtype, int A_dtype, int dt_bias_dtype, int norm_dtype, float q_scale,
+                     float eps_qk, float eps_norm, void *stream);
+
 /* Device workspace gdn_bwd needs, in bytes (256-byte aligned base expected). */
 size_t gdn_bwd_workspace_bytes(int B, int T, int Hk, int Hv, int Dk, int Dv, int chunk, int gate_kind,
                                int has_mask, int form, int in_dtype);

@@ -783,6 +783,65 @@ int gdn_decode_step(const void *q, const void *k, const void *v, const float *g,
     return check_launch(st, "gdn_decode_step");
 }
 
+int gdn_small_linears(const void *x, const void *const *w, void *const *y, const int *n, int count, int tokens, int k,
+                      int dtype, void *stream) {
+    g_err[0] = 0;
+    if (count < 1 || count > 4 || tokens < 0 || k < 1 || !w || !y || !n)
+        return fail(GDN_ERR_INVALID, "one to four weights, tokens >= 0 and k > 0 are expected");
+    if (!dtype_ok(dtype)) return fail(GDN_ERR_INVALID, "unknown dtype code");
+    if (tokens > small_linears_max_tokens() || k % 8)
+        return fail(GDN_ERR_UNSUPPORTED, "at most %d tokens and k a multiple of 8", small_linears_max_tokens());
+    if (tokens == 0) return GDN_OK;
+    SmallLinears a{};
+    a.x = x;
+    a.count = count;
+    a.tokens = tokens;
+    a.k = k;
+    for (int i = 0; i < count; ++i) {
+        if (n[i] < 1 || n[i] > (1 << 28)) return fail(GDN_ERR_INVALID, "rows of weight %d: %d", i, n[i]);
+        if (!w[i] || !y[i]) return fail(GDN_ERR_INVALID, "null pointer");
+        if (misaligned16(w[i])) return fail(GDN_ERR_INVALID, "weights must be 16-byte aligned");
+        a.w[i] = w[i];
+        a.y[i] = y[i];
+        a.n[i] = n[i];
+    }
+    if (!x || misaligned16(x)) return fail(GDN_ERR_INVALID, "x must be a 16-byte aligned pointer");
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    {
+        Timed tm("small_linears", st);
+        launch_small_linears(a, dtype, st);
+    }
+    return check_launch(st, "gdn_small_linears");
+}
+
+int gdn_block_decode(const void *qkv, const void *z, const void *b, const void *a, const void *conv_w, const void *A_log,
+                     const void *dt_bias, const void *norm_w, const float *conv_in, float *conv_out,
+                     const float *state_in, float *state_out, void *out, int B, int Hk, int Hv, int Dk, int Dv, int K,
+                     int dtype, int conv_dtype, int A_dtype, int dt_bias_dtype, int norm_dtype, float q_scale,
+                     float eps_qk, float eps_norm, void *stream) {
+    g_err[0] = 0;
+    int rc = check_shape(B, 1, Hk, Hv, Dk, Dv, 1, GATE_DECAY, GDN_FORM_RECURRENT);
+    if (rc) return rc;
+    for (int dt : {dtype, conv_dtype, A_dtype, dt_bias_dtype, norm_dtype})
+        if (!dtype_ok(dt)) return fail(GDN_ERR_INVALID, "unknown dtype code");
+    if (!block_decode_supported(Dk, Dv, K))
+        return fail(GDN_ERR_UNSUPPORTED, "gdn_block_decode takes Dk = Dv = 128 and a conv of 4 taps");
+    if (B == 0) return GDN_OK;
+    if (!qkv || !z || !b || !a || !conv_w || !A_log || !dt_bias || !norm_w || !conv_out || !state_out || !out)
+        return fail(GDN_ERR_INVALID, "null input or output pointer");
+    if (conv_in == conv_out) return fail(GDN_ERR_INVALID, "conv_out may not be conv_in");
+    if (misaligned16(state_in) || misaligned16(state_out))
+        return fail(GDN_ERR_INVALID, "the states must be 16-byte aligned");
+    BlockDecode d{qkv, z, b, a, conv_w, A_log, dt_bias, norm_w, conv_in, state_in, conv_out, state_out, out,
+                  Hk, Hv, dtype, conv_dtype, A_dtype, dt_bias_dtype, norm_dtype, q_scale, eps_qk, eps_norm};
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    {
+        Timed tm("block_decode", st);
+        launch_block_decode(d, B, st);
+    }
+    return check_launch(st, "gdn_block_decode");
+}
+
 size_t gdn_bwd_workspace_bytes(int B, int T, int Hk, int Hv, int Dk, int Dv, int chunk, int gate_kind,
                                int has_mask, int form, int in_dtype) {
     if (check_shape(B, T, Hk, Hv, Dk, Dv, chunk, gate_kind, form)) return 0;

@@ -124,6 +124,26 @@ void launch_rec_bwd(const RecBwdArgs &a, hipStream_t st);
 void launch_rec_bwd_reduce(const RecBwdArgs &a, hipStream_t st);
 void launch_copy_or_zero(float *dst, const float *src, size_t n, hipStream_t st);
 
+// One decoded token of a block (gdn_decode.hip).
+struct SmallLinears {
+    const void *x, *w[4];
+    void *y[4];
+    int n[4], pad[4];  // rows of each weight; rounded up to the rows of a wave (set by the launch)
+    int count, tokens, k;
+};
+int small_linears_max_tokens();
+void launch_small_linears(const SmallLinears &a, int dt, hipStream_t st);
+struct BlockDecode {
+    const void *qkv, *z, *b, *a, *conv_w, *A_log, *dt_bias, *norm_w;
+    const float *conv_in, *state_in;
+    float *conv_out, *state_out;
+    void *out;
+    int Hk, Hv, dt, conv_dt, A_dt, dtb_dt, norm_dt;
+    float q_scale, eps_qk, eps_norm;
+};
+bool block_decode_supported(int Dk, int Dv, int K);
+void launch_block_decode(const BlockDecode &a, int B, hipStream_t st);
+
 // Block ops around the recurrence (gdn_block_ops.hip).  `vec` selects the vector-load kernels; the caller
 // checks alignment and shape for them.
 int row_lanes(int D);

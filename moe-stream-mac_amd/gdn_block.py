@@ -9,6 +9,7 @@ path.
 
 from __future__ import annotations
 
+import ctypes
 from typing import Optional
 
 import torch
@@ -312,3 +313,47 @@ def gated_rmsnorm(y: Array, z: Array, w: Array, eps: float = 1e-6) -> Array:
     """y / sqrt(mean(y^2) + eps) * w * silu(z) over the last axis (op_rmsnorm then op_silu_mul per value head,
     engine/include/ops.h:7-11, engine/src/gdn_layer.c:47-55).  Output has y's dtype."""
     return _GatedRMSNorm.apply(y, z, w, eps)
+
+
+# ------------------------------------------------------------------------------------------------ one decoded token
+
+SMALL_LINEARS_MAX_TOKENS = 16
+
+
+def small_linears_fit(tokens: int, weights) -> bool:
+    """Whether small_linears takes these weights (contiguous, 16-byte aligned rows) for this many tokens."""
+    return 0 < tokens <= SMALL_LINEARS_MAX_TOKENS and all(
+        w.shape[1] % 8 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0 for w in weights)
+
+
+def small_linears(x: Array, weights) -> list[Array]:
+    """x [tokens, k] times each weight [n, k] transposed, for a few tokens and up to four weights, in one launch (one
+    dtype, fp32 sums; forward only)."""
+    tokens, k = x.shape
+    x = _aligned16(x)
+    ys = [torch.empty((tokens, w.shape[0]), dtype=x.dtype, device=x.device) for w in weights]
+    m = len(ys)
+    ptrs = ctypes.c_void_p * m
+    L.check(L.load().gdn_small_linears(x.data_ptr(), ptrs(*[w.data_ptr() for w in weights]),
+                                       ptrs(*[y.data_ptr() for y in ys]), (ctypes.c_int * m)(*[y.shape[1] for y in ys]),
+                                       m, tokens, k, _code(x), L.stream_handle(x.device)))
+    return ys
+
+
+def block_decode(qkv: Array, z: Array, b: Array, a: Array, conv_w: Array, A_log: Array, dt_bias: Array, norm_w: Array,
+                 conv_state: Optional[Array], state: Optional[Array], Hk: int, q_scale: float, eps: float):
+    """Everything between the projections of one token of B sequences (gdn_block_decode of the C ABI): qkv [B, C], z
+    [B, Hv * 128], b and a [B, Hv] -> out [B, Hv * 128] and the conv and recurrent states after the token."""
+    B, C = qkv.shape
+    Hv = a.shape[1]
+    D = z.shape[1] // Hv
+    dev = qkv.device
+    out = torch.empty_like(z)
+    conv_out = torch.empty((B, 3, C), dtype=torch.float32, device=dev)
+    state_out = torch.empty((B, Hv, D, D), dtype=torch.float32, device=dev)
+    L.check(L.load().gdn_block_decode(
+        qkv.data_ptr(), z.data_ptr(), b.data_ptr(), a.data_ptr(), conv_w.data_ptr(), A_log.data_ptr(),
+        dt_bias.data_ptr(), norm_w.data_ptr(), L.ptr(conv_state), conv_out.data_ptr(), L.ptr(state),
+        state_out.data_ptr(), out.data_ptr(), B, Hk, Hv, D, D, 4, _code(qkv), _code(conv_w), _code(A_log),
+        _code(dt_bias), _code(norm_w), q_scale, 1e-6, eps, L.stream_handle(dev)))
+    return out, conv_out, state_out

@@ -44,6 +44,8 @@ _SIGS = {
     "gdn_gated_rmsnorm_fwd": ([_vp] * 4 + [_i64, _i, _f, _i, _i, _vp], _i),
     "gdn_gated_rmsnorm_bwd_workspace_bytes": ([_i64, _i], _sz),
     "gdn_gated_rmsnorm_bwd": ([_vp] * 8 + [_sz, _i64, _i, _f, _i, _i, _i, _vp], _i),
+    "gdn_small_linears": ([_vp] * 4 + [_i] * 4 + [_vp], _i),
+    "gdn_block_decode": ([_vp] * 13 + [_i] * 11 + [_f] * 3 + [_vp], _i),
     "gdn_version": ([], _i),
     "gdn_last_error": ([], ctypes.c_char_p),
     "gdn_num_snapshots": ([_i, _i], ctypes.c_int64),

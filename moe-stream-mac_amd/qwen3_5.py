@@ -15,14 +15,19 @@ model are outside the GDN path and are not modelled.
 from __future__ import annotations
 
 import math
+import sys
 from dataclasses import dataclass, field
 from typing import Optional
 
 import torch
+import torch.autograd.forward_ad as fwAD
 import torch.nn as nn
 import torch.nn.functional as F
+import torch.nn.modules.module as nn_module
 
+import gated_delta
 import gdn_block
+import gdn_lib as L
 from gated_delta import gated_delta_update, normalize_qk  # noqa: F401  (rebound by install())
 
 Array = torch.Tensor
@@ -89,6 +94,8 @@ class GatedDeltaNet(nn.Module):
         a prefill, then one call per decoded token."""
         B, T, _ = x.shape
         projs = (self.in_proj_qkv, self.in_proj_z, self.in_proj_b, self.in_proj_a)
+        if T == 1 and cache is not None and mask is None and not torch.is_grad_enabled() and self._decodes_fused(x, cache):
+            return self._decode_token(x, cache)
         if all(isinstance(m, LoRALinear) and m.base.bias is None for m in projs):
             qkv, z, b, a = lora_group(x, projs)  # the four adapters share one pass over x
         else:
@@ -109,6 +116,71 @@ class GatedDeltaNet(nn.Module):
             cache[0], cache[1] = conv_next[0], state_next
         out = self.norm(out.to(z.dtype), z)
         return self.out_proj(out.reshape(B, T, -1))
+
+
+    def _decodes_fused(self, x: Array, cache: "GDNCache") -> bool:
+        """Whether one token takes the fused decode (three launches): inference on plain tensors and bias-free Linear
+        layers that nothing has hooked or replaced, this package's own update, and shapes its kernels take.  Every other
+        call, wrong ones included, runs step by step."""
+        lins = (self.in_proj_qkv, self.in_proj_z, self.in_proj_b, self.in_proj_a, self.out_proj)
+        if (self.training or not x.is_cuda or type(x) is not Array or (self.Dk, self.Dv, self.K) != (128, 128, 4)
+                or x.dtype not in L.DTYPE_CODE or torch.is_autocast_enabled("cuda") or fwAD._current_level >= 0
+                or nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks
+                or nn.Linear.forward is not _LINEAR_FORWARD or RMSNormGated.forward is not _NORM_FORWARD
+                or not _own_update(globals()["gated_delta_update"])):
+            return False
+        for m in (*lins, self.norm):
+            if m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__:
+                return False
+        if type(self.norm) is not RMSNormGated or any(type(m) is not nn.Linear or m.bias is not None for m in lins):
+            return False
+        params = [m.weight for m in lins] + [self.conv1d.weight, self.A_log, self.dt_bias, self.norm.weight]
+        dev = x.device
+        if any(type(p) not in (nn.Parameter, Array) or p.device != dev or p.dtype not in L.DTYPE_CODE
+               or not p.is_contiguous() for p in params):
+            return False
+        B, h = x.shape[0], x.shape[2]
+        want = ((self.conv_dim, h), (self.value_dim, h), (self.Hv, h), (self.Hv, h), (h, self.value_dim),
+                (self.conv_dim, 1, self.K), (self.Hv,), (self.Hv,), (self.Dv,))
+        if any(p.shape != s for p, s in zip(params, want)) or any(m.weight.dtype != x.dtype for m in lins):
+            return False
+        for t, shape in ((cache[0], (B, self.K - 1, self.conv_dim)), (cache[1], (B, self.Hv, self.Dv, self.Dk))):
+            if t is not None and (type(t) is not Array or t.shape != shape or t.dtype != torch.float32
+                                  or t.device != dev or not t.is_contiguous() or t.data_ptr() % 16):
+                return False
+        return B > 0
+
+    def _decode_token(self, x: Array, cache: "GDNCache") -> Array:
+        """One token of B sequences: the in-projections, everything between the projections, the out-projection."""
+        B, _, h = x.shape
+        x2 = x.reshape(B, h)
+        lins = (self.in_proj_qkv, self.in_proj_z, self.in_proj_b, self.in_proj_a)
+        weights = [m.weight for m in lins]
+        if gdn_block.small_linears_fit(B, weights):
+            qkv, z, b, a = gdn_block.small_linears(x2, weights)
+        else:
+            qkv, z, b, a = (m(x2) for m in lins)
+        out, cache[0], cache[1] = gdn_block.block_decode(
+            qkv, z, b, a, self.conv1d.weight, self.A_log, self.dt_bias, self.norm.weight, cache[0], cache[1], self.Hk,
+            self.Dk ** -0.5, self.norm.eps)
+        if gdn_block.small_linears_fit(B, (self.out_proj.weight,)):
+            return gdn_block.small_linears(out, (self.out_proj.weight,))[0].view(B, 1, h)
+        return self.out_proj(out).view(B, 1, h)
+
+
+_LINEAR_FORWARD, _NORM_FORWARD = nn.Linear.forward, RMSNormGated.forward
+
+
+def _own_update(update) -> bool:
+    """Whether an inference call of ``update`` ends in this package's gated_delta_update: itself, or one that an
+    install() bound over it."""
+    while update is not gated_delta.gated_delta_update:
+        mod = sys.modules.get(getattr(update, "__module__", None))
+        names = {"gdn_vjp": "_vjp_update", "gdn_checkpoint": "_checkpointed_update", "frozen_gdn": "_marked_update"}
+        if mod is None or update is not getattr(mod, names.get(mod.__name__, ""), None):
+            return False
+        update = mod._ORIGINAL_UPDATE
+    return True
 
 
 class GDNCache:
