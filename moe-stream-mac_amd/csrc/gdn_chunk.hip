@@ -119,8 +119,408 @@ __global__ __launch_bounds__(NTP) void ck_prep_kernel(Args a) {
 }
 
 // ---------------------------------------------------------------------------------------------- ck_fwd
+//
+// The fp32 sequential kernels.  v_mfma_f32_16x16x4_f32 takes one A and one B element per lane (row li, k-index lg of the
+// four); since the order of a contraction is free, lane group lg takes the indices 16 s + 4 lg + i, i = 0..3, in the four
+// products of step s: an operand whose rows run along the contraction is then one 16-byte LDS read per step, and the
+// accumulators' four rows per lane are 16 contiguous bytes of the transposed tiles the next product reads.  The chunk's
+// tiles (W, Q, K, P; K, Q, W, P in the backward) are loaded by whole rows one chunk ahead and each has its own LDS space,
+// so a chunk step is one pass of stores, two of products and three barriers.  T^T, needed once, is read from memory in
+// operand form.  The first form shared the space between the tiles of the two passes (five barriers, two passes of
+// stores) and read every operand 4 bytes at a time: forward / backward at B = 1, T = 4096, Hv = 32
+// 356 / 364 -> 309 / 344 us (4.8 / 5.4 a step, of which the products take 1.5 / 1.7 at the fp32 matrix rate), at B = 2,
+// T = 1024 131 / 138 -> 106 / 126 us.
 
+// acc[t] += A * B_t over NS steps of 16 contraction indices, B_t(k, n) at b[(n0 + 16 t + n) * ldb + k]: A(m, k) from a(s),
+// four contraction indices of this lane's row.  Two accumulator sets, so that two products of a tile are in flight.
+template <int NS, int NTL, class AOp>
+__device__ __forceinline__ void mma4(f4 (&acc)[NTL], AOp a, const float *b, int ldb, int n0, int l) {
+    const float *bp = b + (n0 + (l & 15)) * ldb + 4 * (l >> 4);
+    f4 odd[NTL];
+#pragma unroll
+    for (int t = 0; t < NTL; ++t) odd[t] = zero4();
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+        const float4 x = a(s);
+        float4 y[NTL];
+#pragma unroll
+        for (int t = 0; t < NTL; ++t) y[t] = *reinterpret_cast<const float4 *>(bp + 16 * t * ldb + 16 * s);
+#pragma unroll
+        for (int t = 0; t < NTL; ++t) {
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x, y[t].x, acc[t], 0, 0, 0);
+            odd[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, y[t].y, odd[t], 0, 0, 0);
+        }
+#pragma unroll
+        for (int t = 0; t < NTL; ++t) {
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.z, y[t].z, acc[t], 0, 0, 0);
+            odd[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w, y[t].w, odd[t], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < NTL; ++t) acc[t] += odd[t];
+}
+// A operands in LDS: rows m0.. of a row-major tile (16-byte reads), or its columns m0.. (four reads of 64-byte runs).
+struct RowsA {
+    const float *p;
+    __device__ RowsA(const float *t, int ld, int m0, int l) : p(t + (m0 + (l & 15)) * ld + 4 * (l >> 4)) {}
+    __device__ __forceinline__ float4 operator()(int s) const { return *reinterpret_cast<const float4 *>(p + 16 * s); }
+};
+template <int LDT>
+struct ColsA {
+    const float *p;
+    __device__ ColsA(const float *t, int m0, int l) : p(t + 4 * (l >> 4) * LDT + m0 + (l & 15)) {}
+    __device__ __forceinline__ float4 operator()(int s) const {
+        const float *x = p + 16 * s * LDT;
+        return make_float4(x[0], x[LDT], x[2 * LDT], x[3 * LDT]);
+    }
+};
 
+// A [C][COLS] tile loaded by rows as raw 16-byte pieces, later written to LDS as fp32 (row stride ld); rows past n are
+// zero (they load row n - 1: no load under a branch).  Row stride rs in elements of dtype dt.
+template <int COLS>
+struct RowTile {
+    static constexpr int PER = C * COLS / 4 / NTS;  // pieces per thread in fp32, twice those in 16-bit dtypes
+    uint4 x[PER];
+    __device__ __forceinline__ void load(const void *p, unsigned rs, int n, int dt, int tid) {
+        const bool f32 = dt == DT_F32;
+        const int epq = f32 ? 4 : 8, vpr = COLS / epq;  // elements per piece, pieces per row
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            if (!f32 && i >= PER / 2) continue;
+            const int v = tid + i * NTS, r = v / vpr;
+            const unsigned off = ((unsigned)min(r, n - 1) * rs + epq * (v - r * vpr)) * (f32 ? 4 : 2);
+            const uint4 y = *reinterpret_cast<const uint4 *>(static_cast<const char *>(p) + off);
+            x[i] = r < n ? y : make_uint4(0u, 0u, 0u, 0u);
+        }
+    }
+    __device__ __forceinline__ void store(float *dst, int ld, int dt, int tid) const {
+        const bool f32 = dt == DT_F32;
+        const int epq = f32 ? 4 : 8, vpr = COLS / epq;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            if (!f32 && i >= PER / 2) continue;
+            const int v = tid + i * NTS, r = v / vpr;
+            float *d = dst + r * ld + epq * (v - r * vpr);
+            if (f32) {
+                *reinterpret_cast<uint4 *>(d) = x[i];
+            } else {
+                const uint32_t w[4] = {x[i].x, x[i].y, x[i].z, x[i].w};
+#pragma unroll
+                for (int k = 0; k < 4; ++k) unpack16(w[k], dt, d[2 * k], d[2 * k + 1]);
+            }
+        }
+    }
+};
+
+template <int VS, int MODE, bool AF32, bool MASK>
+__global__ __launch_bounds__(NTS) void ck_fwd_kernel(Args a) {
+    DTYPES_OF(a);
+    constexpr bool kTiles = MODE != FWD_ONLY, kOut = MODE != FWD_RECOMPUTE;
+    constexpr int NTN = VS / 16, DN = NTN >= 2 ? NTN / 2 : 1;  // value tiles of the slice / of a wave's [C][VS] products
+    __shared__ __align__(16) float sW[C * LD], sK[C * LD];
+    __shared__ __align__(16) float sQ[kOut ? C * LD : 4], sP[kOut ? C * LDC : 4];
+    __shared__ __align__(16) float sH[VS * LD];                        // h [i][j]
+    __shared__ __align__(16) float sD[kOut ? VS * LDC : 4], sDs[VS * LDC];  // Delta, diag(gamma_C / gamma) Delta [i][r]
+    __shared__ __align__(16) float sGam[C], sRc[C];
+
+    const SeqBlock sb = seq_block();
+    const SeqRange sr = seq_range<MODE>(a, sb.b);
+    const int i0 = sb.slice * VS, hv = sb.hv, b = sr.b, cb = sr.cb, ce = sr.ce;
+    const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, li = l & 15, lg = l >> 4;
+    const int T = a.T, hk = hv / (a.Hv / a.Hk);
+    const size_t head = (size_t)b * a.Hv + hv;
+    const int mrow = 16 * (w & 3);
+    // with 16-wide slices waves 0-3 form Delta and waves 4-7 form y on the same row blocks
+    const bool dwave = NTN >= 2 || w < 4, ywave = NTN >= 2 || w >= 4;
+    const int nt0 = NTN >= 2 ? (w >> 2) * DN : 0;
+
+    f4 h[NTN];  // rows j = 16 w + 4 lg + e, columns i = i0 + 16 t + li
+#pragma unroll
+    for (int t = 0; t < NTN; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int j = 16 * w + 4 * lg + e, i = i0 + 16 * t + li;
+            h[t][e] = sr.s0 ? sr.s0[(head * D + i) * D + j] : 0.f;
+        }
+    ChunkFlags<MASK> flags;
+    RowTile<D> rW, rQ, rK;
+    RowTile<C> rP;
+    float rU[DN][4];
+    double rG = 0.0;
+    auto fetch = [&](int c) {
+        const size_t ci = head * a.NC + c;
+        const int t0 = c * C, n = min(C, T - t0);
+        const size_t qk0 = (((size_t)b * a.Ts + t0) * a.Hk + hk) * D;
+        rW.load(a.w.W + ci * C * D, D, C, DT_F32, tid);
+        rK.load(elem_ptr(a.k, qk0, k_in_dt), a.Hk * D, n, k_in_dt, tid);
+        if constexpr (kOut) {
+            rP.load(a.w.P + ci * C * C, C, C, DT_F32, tid);
+            const void *q = elem_ptr(a.q, qk0, k_in_dt);
+            unsigned q_row = a.Hk * D;
+            if (AF32 && MASK && flags.nxt) {  // a masked chunk's query rows (other dtypes: after the store below)
+                q = static_cast<const float *>(a.qm) + query_row(a, b, t0, hv);
+                q_row = a.Hv * D;
+            }
+            rQ.load(q, q_row, n, k_in_dt, tid);
+        }
+        if (dwave) {
+#pragma unroll
+            for (int t = 0; t < DN; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    rU[t][e] = (a.w.U + ci * C * D + i0)[(unsigned)((mrow + 4 * lg + e) * D + 16 * (nt0 + t) + li)];
+        }
+        if (tid < C) rG = a.w.G[ci * C + tid];
+    };
+    flags.start(a, b, cb, 1, ce);
+    fetch(cb);
+    for (int c = cb; c < ce; ++c) {
+        const int t0 = c * C, n = min(C, T - t0);
+        const size_t ci = head * a.NC + c;
+        if (float *sp = snap_at<MODE>(a, c)) store_state_acc<NTN>(sp, h, head, i0, w, lg, li);
+        flags.enter(a, b, c, 1, ce);
+        __syncthreads();  // the previous step's tiles read
+        // h -> LDS as the operand [i][j]; the chunk-entry state -> saved H ([j][i])
+#pragma unroll
+        for (int t = 0; t < NTN; ++t) {
+            *reinterpret_cast<f4 *>(sH + (16 * t + li) * LD + 16 * w + 4 * lg) = h[t];
+            if constexpr (kTiles) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    (a.w.H + ci * D * D + i0)[(unsigned)((16 * w + 4 * lg + e) * D + 16 * t + li)] = h[t][e];
+            }
+        }
+        rW.store(sW, LD, DT_F32, tid);
+        if constexpr (kOut) {
+            rQ.store(sQ, LD, k_in_dt, tid);
+            if (!AF32 && flags.cur) load_queries<NTS>(sQ, LD, a, b, hv, t0, n, k_in_dt, tid);
+            rP.store(sP, LDC, DT_F32, tid);
+        }
+        rK.store(sK, LD, k_in_dt, tid);
+        if (tid < C) {
+            sGam[tid] = expf((float)rG);
+            sRc[tid] = expf((float)(readlane_f64(rG, C - 1) - rG));
+        }
+        float u[DN][4];
+#pragma unroll
+        for (int t = 0; t < DN; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) u[t][e] = rU[t][e];
+        __syncthreads();
+        if (c + 1 < ce) fetch(c + 1);
+        f4 wh[DN], yi[DN];
+#pragma unroll
+        for (int t = 0; t < DN; ++t) wh[t] = yi[t] = zero4();
+        if (dwave) {
+            // Delta = U - W h
+            mma4<D / 16>(wh, RowsA(sW, LD, mrow, l), sH, LD, 16 * nt0, l);
+            const float4 rc = *reinterpret_cast<const float4 *>(sRc + mrow + 4 * lg);
+#pragma unroll
+            for (int t = 0; t < DN; ++t) {
+                f4 dl, ds;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) dl[e] = u[t][e] - wh[t][e];
+                ds[0] = rc.x * dl[0]; ds[1] = rc.y * dl[1]; ds[2] = rc.z * dl[2]; ds[3] = rc.w * dl[3];
+                const int o = (16 * (nt0 + t) + li) * LDC + mrow + 4 * lg;
+                if constexpr (kOut) *reinterpret_cast<f4 *>(sD + o) = dl;
+                *reinterpret_cast<f4 *>(sDs + o) = ds;
+                if constexpr (kTiles) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        (a.w.Dl + ci * C * D + i0)[(unsigned)((mrow + 4 * lg + e) * D + 16 * (nt0 + t) + li)] = dl[e];
+                }
+            }
+        }
+        if (ywave && kOut) mma4<D / 16>(yi, RowsA(sQ, LD, mrow, l), sH, LD, 16 * nt0, l);
+        __syncthreads();
+        if (ywave && kOut) {
+            // Y = diag(gamma) Q h + P Delta
+            const float4 gm = *reinterpret_cast<const float4 *>(sGam + mrow + 4 * lg);
+#pragma unroll
+            for (int t = 0; t < DN; ++t) {
+                yi[t][0] *= gm.x; yi[t][1] *= gm.y; yi[t][2] *= gm.z; yi[t][3] *= gm.w;
+            }
+            ValueTerms<DN> vt;
+            if (MASK && flags.cur) vt.load(a, b, hv, t0, n, mrow, i0 + 16 * nt0, k_in_dt);
+            mma4<C / 16>(yi, RowsA(sP, LDC, mrow, l), sD, LDC, 16 * nt0, l);
+            if (MASK && flags.cur) vt.add(yi);
+            void *const yt = const_cast<void *>(elem_ptr(a.y, (((size_t)b * a.Ts + t0) * a.Hv + hv) * D + i0, k_out_dt));
+#pragma unroll
+            for (int t = 0; t < DN; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int r = mrow + 4 * lg + e;
+                    if (r < n) store_from_f32(yt, (unsigned)r * (a.Hv * D) + 16 * (nt0 + t) + li, yi[t][e], k_out_dt);
+                }
+        }
+        // h = gamma_C h + K^T diag(gamma_C / gamma) Delta
+        const float gC = sGam[C - 1];
+#pragma unroll
+        for (int t = 0; t < NTN; ++t) h[t] *= gC;
+        mma4<C / 16>(h, ColsA<LD>(sK, 16 * w, l), sDs, LDC, 0, l);
+    }
+    if (kOut && a.state_T) store_state_acc<NTN>(a.state_T, h, head, i0, w, lg, li);
+}
+
+// ---------------------------------------------------------------------------------------------- ck_bwd_seq
+
+template <int VS, bool AF32, bool MASK>
+__global__ __launch_bounds__(NTS) void ck_bwd_seq_kernel(Args a) {
+    DTYPES_OF(a);
+    constexpr int NTN = VS / 16, DN = NTN >= 2 ? NTN / 2 : 1;
+    constexpr int NY = VS / 8;  // consecutive tokens of one dY column per thread
+    static_assert(NY * NTS == C * VS, "even split");
+    __shared__ __align__(16) float sK[C * LD], sQ[C * LD], sW[C * LD], sP[C * LDC];
+    __shared__ __align__(16) float sH[VS * LD];                      // dh' [i][j]
+    __shared__ __align__(16) float sY[VS * LDC], sYg[VS * LDC];      // dY^T, (diag(gamma) dY)^T [i][s]
+    __shared__ __align__(16) float sD[VS * LDC];                     // dDelta^T [i][r]
+    __shared__ __align__(16) float sGam[C], sRc[C];
+
+    const SeqBlock sb = seq_block();
+    const int i0 = sb.slice * VS, hv = sb.hv, b = sb.b;
+    const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, li = l & 15, lg = l >> 4;
+    const int T = a.T, hk = hv / (a.Hv / a.Hk);
+    const size_t head = (size_t)b * a.Hv + hv;
+    const int mrow = 16 * (w & 3);
+    // with 16-wide slices waves 0-3 form dDelta and waves 4-7 the saved TdD
+    const bool cwave = NTN >= 2 || w < 4, twave = NTN >= 2 || w >= 4;
+    const int nt0 = NTN >= 2 ? (w >> 2) * DN : 0;
+    const int yi = tid % VS, ys = (tid / VS) * NY;  // this thread's dY column and first token
+
+    f4 dh[NTN];
+#pragma unroll
+    for (int t = 0; t < NTN; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int j = 16 * w + 4 * lg + e, i = i0 + 16 * t + li;
+            dh[t][e] = a.dstate_T ? a.dstate_T[(head * D + i) * D + j] : 0.f;
+        }
+    ChunkFlags<MASK> flags;
+    RowTile<D> rK, rQ, rW;
+    RowTile<C> rP;
+    float4 rT[C / 16];  // T^T in operand form: row s = mrow + li, indices r = 16 s' + 4 lg + i
+    float rY[NY];
+    double rG = 0.0;
+    auto fetch_t = [&](int c) {
+        if (!twave) return;
+        const unsigned off = 4 * lg * C + mrow + li;
+#pragma unroll
+        for (int s = 0; s < C / 16; ++s) {
+            const float *p = a.w.T + (head * a.NC + c) * C * C + 16 * s * C;
+            rT[s] = make_float4(p[off], (p + C)[off], (p + 2 * C)[off], (p + 3 * C)[off]);
+        }
+    };
+    auto fetch = [&](int c) {
+        const size_t ci = head * a.NC + c;
+        const int t0 = c * C, n = min(C, T - t0);
+        const size_t qk0 = (((size_t)b * a.Ts + t0) * a.Hk + hk) * D;
+        rK.load(elem_ptr(a.k, qk0, k_in_dt), a.Hk * D, n, k_in_dt, tid);
+        rP.load(a.w.P + ci * C * C, C, C, DT_F32, tid);
+        const void *q = elem_ptr(a.q, qk0, k_in_dt);
+        unsigned q_row = a.Hk * D;
+        if (AF32 && MASK && flags.nxt) {
+            q = static_cast<const float *>(a.qm) + query_row(a, b, t0, hv);
+            q_row = a.Hv * D;
+        }
+        rQ.load(q, q_row, n, k_in_dt, tid);
+        rW.load(a.w.W + ci * C * D, D, C, DT_F32, tid);
+        const void *dy = elem_ptr(a.dy, (((size_t)b * a.Ts + t0) * a.Hv + hv) * D + i0, k_dy_dt);
+#pragma unroll
+        for (int i = 0; i < NY; ++i) {
+            const float x = load_as_f32(dy, (unsigned)min(ys + i, n - 1) * (a.Hv * D) + yi, k_dy_dt);
+            rY[i] = ys + i < n ? x : 0.f;
+        }
+        if (tid < C) rG = a.w.G[ci * C + tid];
+    };
+    flags.start(a, b, a.NC - 1, -1, -1);
+    fetch(a.NC - 1);
+    fetch_t(a.NC - 1);
+    for (int c = a.NC - 1; c >= 0; --c) {
+        const size_t ci = head * a.NC + c;
+        flags.enter(a, b, c, -1, -1);
+        __syncthreads();  // the previous step's tiles read
+        // dh' -> LDS as the operand [i][j] and -> the saved dH ([j][i])
+#pragma unroll
+        for (int t = 0; t < NTN; ++t) {
+            *reinterpret_cast<f4 *>(sH + (16 * t + li) * LD + 16 * w + 4 * lg) = dh[t];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                (a.w.dH + ci * D * D + i0)[(unsigned)((16 * w + 4 * lg + e) * D + 16 * t + li)] = dh[t][e];
+        }
+        rK.store(sK, LD, k_in_dt, tid);
+        rP.store(sP, LDC, DT_F32, tid);
+        rQ.store(sQ, LD, k_in_dt, tid);
+        if (!AF32 && flags.cur) load_queries<NTS>(sQ, LD, a, b, hv, c * C, min(C, T - c * C), k_in_dt, tid);
+        rW.store(sW, LD, DT_F32, tid);
+        float y[NY];
+#pragma unroll
+        for (int i = 0; i < NY; ++i) sY[yi * LDC + ys + i] = y[i] = rY[i];
+        if (tid < C) {
+            sGam[tid] = expf((float)rG);
+            sRc[tid] = expf((float)(readlane_f64(rG, C - 1) - rG));
+        }
+        __syncthreads();
+        if (c > 0) fetch(c - 1);
+        const float gC = sGam[C - 1];
+#pragma unroll
+        for (int i = 0; i < NY; ++i) sYg[yi * LDC + ys + i] = sGam[ys + i] * y[i];
+        // dDelta = diag(gamma_C / gamma) K dh' + P^T dY
+        if (cwave) {
+            f4 dd[DN];
+#pragma unroll
+            for (int t = 0; t < DN; ++t) dd[t] = zero4();
+            mma4<D / 16>(dd, RowsA(sK, LD, mrow, l), sH, LD, 16 * nt0, l);
+            const float4 rc = *reinterpret_cast<const float4 *>(sRc + mrow + 4 * lg);
+#pragma unroll
+            for (int t = 0; t < DN; ++t) {
+                dd[t][0] *= rc.x; dd[t][1] *= rc.y; dd[t][2] *= rc.z; dd[t][3] *= rc.w;
+            }
+            mma4<C / 16>(dd, ColsA<LDC>(sP, mrow, l), sY, LDC, 16 * nt0, l);
+#pragma unroll
+            for (int t = 0; t < DN; ++t) *reinterpret_cast<f4 *>(sD + (16 * (nt0 + t) + li) * LDC + mrow + 4 * lg) = dd[t];
+        }
+        __syncthreads();
+        // saved TdD = T^T dDelta, the only form in which ck_bwd_local_kernel needs T and dDelta
+        if (twave) {
+            f4 tdd[DN];
+#pragma unroll
+            for (int t = 0; t < DN; ++t) tdd[t] = zero4();
+            mma4<C / 16>(tdd, [&](int s) { return rT[s]; }, sD, LDC, 16 * nt0, l);
+#pragma unroll
+            for (int t = 0; t < DN; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    (a.w.dDl + ci * C * D + i0)[(unsigned)((mrow + 4 * lg + e) * D + 16 * (nt0 + t) + li)] = tdd[t][e];
+        }
+        if (c > 0) fetch_t(c - 1);
+        // dh = gamma_C dh' + Q^T diag(gamma) dY - W^T dDelta
+        f4 wd[NTN];
+#pragma unroll
+        for (int t = 0; t < NTN; ++t) {
+            dh[t] *= gC;
+            wd[t] = zero4();
+        }
+        mma4<C / 16>(dh, ColsA<LD>(sQ, 16 * w, l), sYg, LDC, 0, l);
+        mma4<C / 16>(wd, ColsA<LD>(sW, 16 * w, l), sD, LDC, 0, l);
+#pragma unroll
+        for (int t = 0; t < NTN; ++t) dh[t] -= wd[t];
+    }
+    if (a.dstate0) {
+#pragma unroll
+        for (int t = 0; t < NTN; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int j = 16 * w + 4 * lg + e, i = i0 + 16 * t + li;
+                a.dstate0[(head * D + i) * D + j] = dh[t][e];
+            }
+    }
+}
+
+// ---------------------------------------------------------------------------------------------- wide slices
+//
+// The fp32 sequential kernels at 64-wide slices, for launches with heads enough to fill the chip with them: the tiles of
+// ck_fwd_kernel do not fit in LDS beside such a slice, so those of the two passes share their space.  At B = 4, T = 1024,
+// Hv = 32 the forward / backward take 221 / 233 us this way and 226 / 259 us in two rounds of 32-wide workgroups.
 // Row scalings read the chunk's cumulative log decays from LDS: gamma_r = exp(G_r), rc_r = exp(G_{C-1} - G_r).
 struct GamScale {
     const double *G;
@@ -131,8 +531,9 @@ struct RcScale {
     __device__ float operator()(int r) const { return expf((float)(G[C - 1] - G[r])); }
 };
 
-template <int VS, int MODE, bool AF32, bool MASK>
-__global__ __launch_bounds__(NTS) void ck_fwd_kernel(Args a) {
+template <int MODE, bool AF32, bool MASK>
+__global__ __launch_bounds__(NTS) void ck_fwd_wide_kernel(Args a) {
+    constexpr int VS = 64;
     DTYPES_OF(a);
     constexpr bool kTiles = MODE != FWD_ONLY, kOut = MODE != FWD_RECOMPUTE;
     constexpr int LV = VS + 4;
@@ -259,10 +660,10 @@ __global__ __launch_bounds__(NTS) void ck_fwd_kernel(Args a) {
     if (kOut && a.state_T) store_state_acc<NTN>(a.state_T, h, head, i0, w, lg, li);
 }
 
-// ---------------------------------------------------------------------------------------------- ck_bwd_seq
 
-template <int VS, bool AF32, bool MASK>
-__global__ __launch_bounds__(NTS) void ck_bwd_seq_kernel(Args a) {
+template <bool AF32, bool MASK>
+__global__ __launch_bounds__(NTS) void ck_bwd_seq_wide_kernel(Args a) {
+    constexpr int VS = 64;
     DTYPES_OF(a);
     constexpr int LV = VS + 4;
     constexpr int NTN = VS / 16;
@@ -2273,10 +2674,14 @@ static void fwd_launch(const ck::Args &a, hipStream_t st, dim3 grid) {
             constexpr bool MASK = MODE != ck::FWD_RECOMPUTE && decltype(mask)::value;
             if constexpr (MT == 1)
                 hipLaunchKernelGGL((ck::ck_fwd_bf16_kernel<VS, MODE, false, MASK>), grid, dim3(ck::NTS), 0, st, a);
-            else if (all_f32(a))
-                hipLaunchKernelGGL((ck::ck_fwd_kernel<VS, MODE, true, MASK>), grid, dim3(ck::NTS), 0, st, a);
             else
-                hipLaunchKernelGGL((ck::ck_fwd_kernel<VS, MODE, false, MASK>), grid, dim3(ck::NTS), 0, st, a);
+                with_flag(all_f32(a), [&](auto f32) {
+                    constexpr bool F32 = decltype(f32)::value;
+                    if constexpr (VS == 64)
+                        hipLaunchKernelGGL((ck::ck_fwd_wide_kernel<MODE, F32, MASK>), grid, dim3(ck::NTS), 0, st, a);
+                    else
+                        hipLaunchKernelGGL((ck::ck_fwd_kernel<VS, MODE, F32, MASK>), grid, dim3(ck::NTS), 0, st, a);
+                });
         });
     }
 }
@@ -2296,6 +2701,8 @@ static void seq_launch(const ck::Args &a, hipStream_t st, bool fwd) {
             constexpr bool F32 = decltype(f32)::value;
             if constexpr (MT >= 1)
                 hipLaunchKernelGGL((ck::ck_bwd_seq_bf16_kernel<VS, F32, MT == 2, MASK>), grid, dim3(ck::NTS), 0, st, a);
+            else if constexpr (VS == 64)
+                hipLaunchKernelGGL((ck::ck_bwd_seq_wide_kernel<F32, MASK>), grid, dim3(ck::NTS), 0, st, a);
             else
                 hipLaunchKernelGGL((ck::ck_bwd_seq_kernel<VS, F32, MASK>), grid, dim3(ck::NTS), 0, st, a);
         });
@@ -2304,7 +2711,11 @@ static void seq_launch(const ck::Args &a, hipStream_t st, bool fwd) {
 
 template <int MT>
 static void seq_dispatch(const ck::Args &a, hipStream_t st, bool fwd) {
-    switch (slice_width(seq_z(a) * a.Hv)) {
+    int vs = slice_width(seq_z(a) * a.Hv);
+    // fp32 windows recomputed side by side (no y, so no Q and P in LDS): 628 us per checkpointed T = 16384 backward at
+    // 32-wide slices, two workgroups to a CU, 668 at 64
+    if (MT == 0 && a.recompute) vs = vs > 32 ? 32 : vs;
+    switch (vs) {
         case 64: seq_launch<MT, 64>(a, st, fwd); break;
         case 32: seq_launch<MT, 32>(a, st, fwd); break;
         default: seq_launch<MT, 16>(a, st, fwd); break;
