@@ -880,11 +880,44 @@ __device__ __forceinline__ void chunk_dg_dbeta(float *sE, const float (*sRow)[2]
 // u:  dg_u = sum_{r >= u} sum_{s' < u} E[r][s'].  Summing only straddling terms (each carrying the factor
 // exp(g_u)) keeps dg accurate for tiny decays, where a reverse cumulative sum of dG would cancel.
 
+__device__ __forceinline__ float at4(const float4 &x, int i) { return i == 0 ? x.x : i == 1 ? x.y : i == 2 ? x.z : x.w; }
+
+// f(std::integral_constant<int, n>) for a wave-uniform n of 1 or 2; nothing for 0.
+template <class F>
+__device__ __forceinline__ void tiles12(int n, F f) {
+    if (n == 2) f(std::integral_constant<int, 2>{});
+    else if (n == 1) f(std::integral_constant<int, 1>{});
+}
+
+// acc[t] += A * B_t over the 16-index steps s0 <= s < s1 (wave-uniform), B_t(k, n) at b[k * LD + 16 t + n]: operands in
+// the index order of mma4, B's elements read one by one (their columns run along the contraction).
+template <class AOp>
+__device__ __forceinline__ void mma_cols(f4 (&acc)[4], int s0, int s1, AOp a, const float *b, int l) {
+    const float *bp = b + 4 * (l >> 4) * LD + (l & 15);
+    for (int s = s0; s < s1; ++s) {
+        const float4 x = a(s);
+        float y[4][4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) y[i][t] = bp[(16 * s + i) * LD + 16 * t];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(at4(x, i), y[i][t], acc[t], 0, 0, 0);
+    }
+}
+
 // One value head hv = hk * rep + rr of key head hk.  dq | dk of the key head are summed in order (rr = 0, 1, ...)
 // in the part rows of its first value head hk * rep, each thread reading back only the elements it wrote itself,
 // and the last value head writes dq and dk in the gradient dtype.  T and dDelta enter only through TdD = T^T dDelta
 // (saved by ck_bwd_seq_kernel): dv = diag(beta) TdD, dK -= diag(beta gamma) Y2 (Y2 = TdD h^T), dA = -TdD Delta^T
 // below the diagonal, dbeta += rowsum(V * TdD) - gamma s4 and dG -= beta gamma s4 (s4 = rowsum(K * Y2)).
+//
+// Bound by the fp32 matrix rate: one workgroup fills a CU's LDS, so a head takes the same time in an idle chip and in a
+// full one, half of it in products.  Taking only the blocks on and below the diagonal of dP, dA, dPG and K K^T, M + M^T
+// as one operand and the operands that run along the contraction 16 bytes at a time took a head from 42 to 32 us;
+// at B = 4, T = 1024, Hv = 32 388 -> 316 us, T = 16384 in windows of 2048 chunk-heads 1578 -> 1277 us.
 template <bool AF32, bool MASK>
 __device__ __forceinline__ void bwd_local_f32_head(const Args &a, int c, int hk, int b, int rr, int rep) {
     DTYPES_OF(a);
@@ -903,7 +936,11 @@ __device__ __forceinline__ void bwd_local_f32_head(const Args &a, int c, int hk,
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
     const int w = tid >> 6, l = tid & 63, li = l & 15, lg = l >> 4;
-    const int r0 = 16 * (w & 3), ch = w >> 2;  // this wave's rows r0..r0+15 and column half
+    // this wave's rows r0..r0+15 and column half.  Products with a lower-triangular [C][C] operand or result take the
+    // blocks on and below the diagonal only; the two halves take the strips in opposite order, so that the waves of a SIMD
+    // (w, w + 4) have a short and a long one.
+    const int ch = w >> 2, r0 = 16 * (ch ? 7 - w : w), nd = r0 / 16 + 1;  // nd: the strip's blocks up to the diagonal
+    const int ntl = min(max(nd - 2 * ch, 0), 2);                          // those in this column half
     const int T = a.T, t0 = c * C, n = min(C, T - t0);
     const size_t ci = chunk_index(a, b, hv, c);
     float *const sKm = R1;
@@ -925,6 +962,11 @@ __device__ __forceinline__ void bwd_local_f32_head(const Args &a, int c, int hk,
         sB[tid] = tid < n ? bt : 0.f;
     }
     load_tile<D, D, NTB>(R1, LD, Hc, D, D, DT_F32, nullptr, tid);
+    // dh': read once, for <dh', h> and, held in registers during phase 1, for phase 2
+    constexpr int PDH = D * D / 4 / NTB;
+    float4 dv4[PDH];
+#pragma unroll
+    for (int p = 0; p < PDH; ++p) dv4[p] = reinterpret_cast<const float4 *>(dHc)[tid + p * NTB];
     load_tile<C, D, NTB>(R2, LD, elem_ptr(a.dy, v0, k_dy_dt), v_row, n, k_dy_dt, nullptr, tid);
     {
         constexpr int PER = C * D / 4 / NTB;  // float4 pieces per thread; 32 consecutive threads hold one row
@@ -977,42 +1019,42 @@ __device__ __forceinline__ void bwd_local_f32_head(const Args &a, int c, int hk,
         sGam[tid] = expf((float)sG[tid]);
         sRc[tid] = expf((float)(sG[C - 1] - sG[tid]));
     }
+    // phase 2's Delta: in flight during phase 1
+    RowTile<D> tDl;
+    tDl.load(Dc, D, C, DT_F32, tid);
     float lastp = 0.f;  // pair (C-1, chunk start): gamma_C <dh', h>
-    {
-        constexpr int PER = D * D / 4 / NTB;
-        float4 dv4[PER];
 #pragma unroll
-        for (int p = 0; p < PER; ++p) dv4[p] = reinterpret_cast<const float4 *>(dHc)[tid + p * NTB];
-#pragma unroll
-        for (int p = 0; p < PER; ++p) {
-            const int v = tid + p * NTB, i = v / (D / 4), j = (v - i * (D / 4)) * 4;
-            const float *hh = R1 + i * LD + j;
-            lastp += dv4[p].x * hh[0] + dv4[p].y * hh[1] + dv4[p].z * hh[2] + dv4[p].w * hh[3];
-        }
+    for (int p = 0; p < PDH; ++p) {
+        const int v = tid + p * NTB, i = v / (D / 4), j = (v - i * (D / 4)) * 4;
+        const float4 hh = *reinterpret_cast<const float4 *>(R1 + i * LD + j);
+        lastp += dv4[p].x * hh.x + dv4[p].y * hh.y + dv4[p].z * hh.z + dv4[p].w * hh.w;
     }
     float bnd[4] = {0.f, 0.f, 0.f, 0.f};   // pair terms (r, chunk start) of rows r0+4lg+e, this lane's columns
     float rowB[4] = {0.f, 0.f, 0.f, 0.f};  // dbeta partials
     float tl[4] = {0.f, 0.f, 0.f, 0.f};    // pair terms (C-1, r)
 
     // ---- phase 1: dQ = diag(gamma) dY h^T ; Y2 = TdD h^T.  This lane's A values of TdD (row r0 + li, columns
-    // 4 k + lg) stay in registers for dA = TdD Delta^T in phase 2.
+    // 16 s + 4 lg + i) stay in registers for dA = TdD Delta^T in phase 2.
     f4 dQ[4], dK[4], Y2[4];
-    float tdA[D / 4];
+    float4 tdA[D / 16];
     {
 #pragma unroll
         for (int t = 0; t < 4; ++t) dQ[t] = Y2[t] = zero4();
-        const float *ay = R2 + (r0 + li) * LD + lg, *at = RX + (r0 + li) * LD + lg;
-        const float *bh = R1 + (64 * ch + li) * LD + lg;
-#pragma unroll 8
-        for (int k = 0; k < D / 4; ++k) {
-            const float yv = ay[4 * k], tv = at[4 * k];
-            tdA[k] = tv;
+        const RowsA ay(R2, LD, r0, l), at(RX, LD, r0, l);
+        const float *bh = R1 + (64 * ch + li) * LD + 4 * lg;
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const float bv = bh[16 * t * LD + 4 * k];
-                dQ[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(yv, bv, dQ[t], 0, 0, 0);
-                Y2[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(tv, bv, Y2[t], 0, 0, 0);
-            }
+        for (int s = 0; s < D / 16; ++s) {
+            const float4 yv = ay(s), tv = tdA[s] = at(s);
+            float4 hb[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) hb[t] = *reinterpret_cast<const float4 *>(bh + 16 * t * LD + 16 * s);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    dQ[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(at4(yv, i), at4(hb[t], i), dQ[t], 0, 0, 0);
+                    Y2[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(at4(tv, i), at4(hb[t], i), Y2[t], 0, 0, 0);
+                }
         }
     }
     __syncthreads();  // sGam / sRc ready; phase 1's tiles read
@@ -1024,12 +1066,19 @@ __device__ __forceinline__ void bwd_local_f32_head(const Args &a, int c, int hk,
 #pragma unroll
         for (int e = 0; e < 4; ++e) dQ[t][e] *= sGam[r0 + 4 * lg + e];
     // ---- phase 2: dK = diag(gamma_C/gamma) Delta dh'^T ; dP = lower(dY Delta^T) ; dA = -TdD Delta^T
-    load_tile<D, D, NTB>(R1, LD, dHc, D, D, DT_F32, nullptr, tid);
-    load_tile<C, D, NTB>(RX, LD, Dc, D, C, DT_F32, nullptr, tid);  // Delta in place of TdD (phase 1 is done)
+#pragma unroll
+    for (int p = 0; p < PDH; ++p) {
+        const int v = tid + p * NTB, i = v / (D / 4), j = (v - i * (D / 4)) * 4;
+        *reinterpret_cast<float4 *>(R1 + i * LD + j) = dv4[p];
+    }
+    tDl.store(RX, LD, DT_F32, tid);  // Delta in place of TdD (phase 1 is done)
     __syncthreads();
+    RowTile<D> tK, tQ;  // phase 3's K and Q: in flight during phase 2
+    tK.load(elem_ptr(a.k, qk0, k_in_dt), (unsigned)qk_row, n, k_in_dt, tid);
+    tQ.load(elem_ptr(a.q, qk0, k_in_dt), (unsigned)qk_row, n, k_in_dt, tid);
 #pragma unroll
     for (int t = 0; t < 4; ++t) dK[t] = zero4();
-    mma_strip<D, 4>(dK, RX + r0 * LD, LD, 1, R1 + 64 * ch * LD, 1, LD, 16 * LD, l);
+    mma4<D / 16>(dK, RowsA(RX, LD, r0, l), R1, LD, 64 * ch, l);
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -1045,13 +1094,25 @@ __device__ __forceinline__ void bwd_local_f32_head(const Args &a, int c, int hk,
                 pw[t][e] = a.w.P[ci * C * C + (r0 + 4 * lg + e) * C + 32 * ch + 16 * t + li];
         f4 dp[2] = {zero4(), zero4()};
         dA[0] = dA[1] = zero4();
-        mma_strip<D, 2>(dp, R2 + r0 * LD, LD, 1, RX + 32 * ch * LD, 1, LD, 16 * LD, l);
-        const float *bd = RX + (32 * ch + li) * LD + lg;
-#pragma unroll 8
-        for (int k = 0; k < D / 4; ++k)
+        const RowsA ay(R2, LD, r0, l);
+        const float *bd = RX + (32 * ch + li) * LD + 4 * lg;
+        tiles12(ntl, [&](auto nt) {
+            constexpr int NT = decltype(nt)::value;
 #pragma unroll
-            for (int t = 0; t < 2; ++t)
-                dA[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(tdA[k], bd[16 * t * LD + 4 * k], dA[t], 0, 0, 0);
+            for (int s = 0; s < D / 16; ++s) {
+                const float4 yv = ay(s);
+                float4 db[NT];
+#pragma unroll
+                for (int t = 0; t < NT; ++t) db[t] = *reinterpret_cast<const float4 *>(bd + 16 * t * LD + 16 * s);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) {
+                        dp[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(at4(yv, i), at4(db[t], i), dp[t], 0, 0, 0);
+                        dA[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(at4(tdA[s], i), at4(db[t], i), dA[t], 0, 0, 0);
+                    }
+            }
+        });
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -1064,8 +1125,8 @@ __device__ __forceinline__ void bwd_local_f32_head(const Args &a, int c, int hk,
     }
     __syncthreads();
     // ---- phase 3: dQ += dPG K ; dK += dPG^T Q ; K K^T
-    load_tile<C, D, NTB>(sKm, LD, elem_ptr(a.k, qk0, k_in_dt), qk_row, n, k_in_dt, nullptr, tid);
-    load_tile<C, D, NTB>(sQm, LD, elem_ptr(a.q, qk0, k_in_dt), qk_row, n, k_in_dt, nullptr, tid);
+    tK.store(sKm, LD, k_in_dt, tid);
+    tQ.store(sQm, LD, k_in_dt, tid);
     const bool mk = MASK && flag_set(chunk_flag(a, b, c));
     if (mk) load_queries<NTB>(sQm, LD, a, b, hv, t0, n, k_in_dt, tid);
 #pragma unroll
@@ -1088,12 +1149,20 @@ __device__ __forceinline__ void bwd_local_f32_head(const Args &a, int c, int hk,
             bnd[e] -= bg * s4;
             dK[t][e] -= bg * Y2[t][e];
         }
-    mma_strip<C, 4>(dQ, R4 + r0 * LDC, LDC, 1, sKm + 64 * ch, LD, 1, 16, l);
-    mma_strip<C, 4>(dK, R4 + r0, 1, LDC, sQm + 64 * ch, LD, 1, 16, l);
+    // dPG is lower triangular: row strip r0 of it ends, column strip r0 begins, at the diagonal block
+    mma_cols(dQ, 0, nd, RowsA(R4, LDC, r0, l), sKm + 64 * ch, l);
+    mma_cols(dK, nd - 1, C / 16, ColsA<LDC>(R4, r0, l), sQm + 64 * ch, l);
     f4 Mt[2];
     {
         f4 kk[2] = {zero4(), zero4()};
-        mma_strip<D, 2>(kk, sKm + r0 * LD, LD, 1, sKm + 32 * ch * LD, 1, LD, 16 * LD, l);
+        tiles12(ntl, [&](auto nt) {
+            f4 x[decltype(nt)::value];
+#pragma unroll
+            for (int t = 0; t < decltype(nt)::value; ++t) x[t] = zero4();
+            mma4<D / 16>(x, RowsA(sKm, LD, r0, l), sKm, LD, 32 * ch, l);
+#pragma unroll
+            for (int t = 0; t < decltype(nt)::value; ++t) kk[t] = x[t];
+        });
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -1108,14 +1177,16 @@ __device__ __forceinline__ void bwd_local_f32_head(const Args &a, int c, int hk,
             }
     }
     __syncthreads();
-    // ---- phase 4: dK += (M + M^T) K
+    // ---- phase 4: dK += (M + M^T) K, with M + M^T (M strictly lower triangular) as one operand
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) R4[(r0 + 4 * lg + e) * LDC + 32 * ch + 16 * t + li] = Mt[t][e];
+        for (int e = 0; e < 4; ++e) {
+            const int r = r0 + 4 * lg + e, s2 = 32 * ch + 16 * t + li;
+            if (s2 <= r) R4[r * LDC + s2] = R4[s2 * LDC + r] = Mt[t][e];
+        }
     __syncthreads();
-    mma_strip<C, 4>(dK, R4 + r0 * LDC, LDC, 1, sKm + 64 * ch, LD, 1, 16, l);
-    mma_strip<C, 4>(dK, R4 + r0, 1, LDC, sKm + 64 * ch, LD, 1, 16, l);
+    mma_cols(dK, 0, C / 16, RowsA(R4, LDC, r0, l), sKm + 64 * ch, l);
     // ---- phase 6: straddle sums for dg, dbeta, outputs.  R2 (dY) is free: E goes there.
     float *const sE = R2;
 #pragma unroll

@@ -22,6 +22,7 @@ NAMES = ("y", "S_T", "dq", "dk", "dv", "dg", "dbeta", "dS0")
     (2, 16, 32, 66, 64), (4, 16, 16, 127, 64),                                                         # 32 wide
     (4, 16, 32, 65, 64), (8, 16, 16, 129, 64),                                                         # 64 wide
     (1, 2, 4, 385, 128), (2, 16, 32, 200, 128), (4, 16, 32, 140, 128),   # windows recomputed side by side
+    (1, 1, 4, 100, 64), (4, 16, 32, 200, 64), (3, 16, 32, 400, 64),      # 4, 256 and 336 (chunk, key head) pairs
 ])
 def test_slice_widths(B, Hk, Hv, T, chunk, dtype):
     if not torch.cuda.is_available():
