@@ -919,7 +919,8 @@ __device__ __forceinline__ void mma_cols(f4 (&acc)[4], int s0, int s1, AOp a, co
 // as one operand and the operands that run along the contraction 16 bytes at a time took a head from 42 to 32 us;
 // at B = 4, T = 1024, Hv = 32 388 -> 316 us, T = 16384 in windows of 2048 chunk-heads 1578 -> 1277 us.
 template <bool AF32, bool MASK>
-__device__ __forceinline__ void bwd_local_f32_head(const Args &a, int c, int hk, int b, int rr, int rep) {
+__device__ __forceinline__ void bwd_local_f32_head(const Args &a, int c, int hk, int b, int rr, int rep,
+                                                   bool split) {
     DTYPES_OF(a);
     __shared__ __align__(16) float R1[D * LD];       // h, then dh' ([j][i]); then K at R1, Q at R1 + C*LD
     __shared__ __align__(16) float R2[C * LD];       // dY, then the pair matrix E
@@ -929,7 +930,7 @@ __device__ __forceinline__ void bwd_local_f32_head(const Args &a, int c, int hk,
     __shared__ float sRow[3][2][C];                  // per column half: chunk-start pair terms, t2 terms, dbeta
     __shared__ float sLast[8];
 
-    const bool first = rr == 0, last = rr == rep - 1;
+    const bool first = split || rr == 0, last = !split && rr == rep - 1;
     const int hv = hk * rep + rr;
     // an opaque thread index per value head: the lane-dependent addresses are formed inside the head instead of
     // being hoisted out of the caller's loop and held in registers across the whole head
@@ -1213,7 +1214,7 @@ __device__ __forceinline__ void bwd_local_f32_head(const Args &a, int c, int hk,
     constexpr int LQ = 64 + 4;
     static_assert(8 * 16 * LQ <= D * LD, "staging fits R1");
     float *const stg = R1 + w * 16 * LQ;
-    float *const sum_row = a.w.part + ((size_t)b * T + t0) * a.Hv * 2 * D + (size_t)hk * rep * 2 * D;
+    float *const sum_row = a.w.part + ((size_t)b * T + t0) * a.Hv * 2 * D + (size_t)(split ? hv : hk * rep) * 2 * D;
     float4 prq[4], prk[4];
     if (!first) {
 #pragma unroll
@@ -1260,16 +1261,44 @@ __device__ __forceinline__ void bwd_local_f32_head(const Args &a, int c, int hk,
     __syncthreads();  // the pair matrix read: the next value head's tiles reuse its space
 }
 
-// One workgroup of 8 waves per (chunk, key head), walking the key head's value heads in order.
+// One workgroup of 8 waves per (chunk, key head), walking the key head's value heads in order; or (grid.y = Hv, see
+// local_split) per (chunk, value head), each leaving its dq | dk in its own part rows for ck_local_sum_kernel.
 template <bool AF32, bool MASK>
 __global__ __launch_bounds__(NTB) void ck_bwd_local_kernel(Args a) {
     typedef const __attribute__((address_space(4))) Args *KArgs;  // the kernel arguments (constant memory)
     const int rep = a.Hv / a.Hk;
-    for (int rr = 0; rr < rep; ++rr) {
+    const bool split = (int)gridDim.y != a.Hk;
+    const int hk = split ? blockIdx.y / rep : blockIdx.y, rr0 = split ? blockIdx.y - hk * rep : 0;
+    for (int rr = rr0; rr < (split ? rr0 + 1 : rep); ++rr) {
         // the arguments are read anew for each value head instead of being held in scalar registers across it
         KArgs ap = (KArgs)__builtin_amdgcn_kernarg_segment_ptr();
         asm volatile("" : "+s"(ap));
-        bwd_local_f32_head<AF32, MASK>(*(const Args *)ap, blockIdx.x, blockIdx.y, blockIdx.z, rr, rep);
+        bwd_local_f32_head<AF32, MASK>(*(const Args *)ap, blockIdx.x, hk, blockIdx.z, rr, rep, split);
+    }
+}
+
+// dq and dk of each (token, key head) from its value heads' part rows, summed in the order of the walk: the same bits.
+// A wave per row pair: lane l holds elements 4 l .. 4 l + 3 of dq | dk.
+__global__ __launch_bounds__(256) void ck_local_sum_kernel(Args a) {
+    const int l = threadIdx.x & 63, rep = a.Hv / a.Hk;
+    const size_t rows = (size_t)a.B * a.T * a.Hk, row = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const float *p = a.w.part + row * rep * 2 * D + 4 * l;
+    float4 v = *reinterpret_cast<const float4 *>(p);
+    for (int rr = 1; rr < rep; ++rr) {
+        const float4 x = *reinterpret_cast<const float4 *>(p + (size_t)rr * 2 * D);
+        v = make_float4(v.x + x.x, v.y + x.y, v.z + x.z, v.w + x.w);
+    }
+    const size_t tok = row / a.Hk, b = tok / a.T, t = tok - b * a.T;
+    const size_t o = ((b * a.Ts + t) * a.Hk + (row - tok * a.Hk)) * D + 4 * (l & 31);
+    void *const dst = l < 32 ? a.dq : a.dk;
+    if (a.grad_dt == DT_F32) {
+        *reinterpret_cast<float4 *>(static_cast<float *>(dst) + o) = v;
+    } else {
+        store_from_f32(dst, o, v.x, a.grad_dt);
+        store_from_f32(dst, o + 1, v.y, a.grad_dt);
+        store_from_f32(dst, o + 2, v.z, a.grad_dt);
+        store_from_f32(dst, o + 3, v.w, a.grad_dt);
     }
 }
 
@@ -2810,6 +2839,15 @@ static void ck_fwd_launch(const ck::Args &a, hipStream_t st, const char *stage) 
     }
 }
 
+// fp32 set: a workgroup per value head instead of per key head, where that takes fewer rounds of workgroups (one to a CU; a
+// head takes the same time in each): with the sum of the heads' dq | dk 65 -> 37 us for one 64-token chunk of 16 key and
+// 32 value heads, 148 -> 129 us at T = 1280 (320 key-head workgroups).  In equal rounds the walk saves the sum: T = 768 76 us
+// either way.  The bf16 set's head is a third of that, memory-bound in a full chip, and keeps the walk.
+static bool local_split(const ck::Args &a) {
+    const size_t cus = 256, wgs = (size_t)a.NC * a.Hk * a.B, rep = a.Hv / a.Hk;
+    return (wgs * rep + cus - 1) / cus < (wgs + cus - 1) / cus * rep;
+}
+
 template <int MT>
 static void ck_bwd_launch(const ck::Args &a, hipStream_t st, const char *stage) {
     if (stage[0] == 's') {
@@ -2818,7 +2856,8 @@ static void ck_bwd_launch(const ck::Args &a, hipStream_t st, const char *stage) 
         if (stage[0] == 'd') ck::launch_vg_dg(a, st);
         else ck::launch_vg_local(a, st);
     } else {
-        const dim3 grid(a.NC, a.Hk, a.B);
+        const bool split = MT == 0 && local_split(a);
+        const dim3 grid(a.NC, split ? a.Hv : a.Hk, a.B);
         with_flag(a.mask != nullptr, [&](auto mask) {
             constexpr bool MASK = decltype(mask)::value;
             with_flag(MT == 0 ? all_f32(a) : a.dy_dt == DT_F32, [&](auto f32) {
@@ -2827,6 +2866,10 @@ static void ck_bwd_launch(const ck::Args &a, hipStream_t st, const char *stage) 
                 else hipLaunchKernelGGL((ck::ck_bwd_local_kernel<F32, MASK>), grid, dim3(ck::NTB), 0, st, a);
             });
         });
+        if (split) {
+            const size_t rows = (size_t)a.B * a.T * a.Hk;
+            hipLaunchKernelGGL(ck::ck_local_sum_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, a);
+        }
     }
 }
 
