@@ -41,24 +41,16 @@ def normalize_qk(q: Array, k: Array, inv_scale: float, eps: float = 1e-6) -> tup
     return gdn_block.normalize_qk(q, k, inv_scale, eps)
 
 
-def _default_state(q: Array, v: Array, state: Optional[Array]) -> Array:
-    if state is not None:
-        return state
-    B, _, _, Dk = q.shape
-    Hv, Dv = v.shape[-2:]
-    return torch.zeros((B, Hv, Dv, Dk), dtype=torch.float32, device=q.device)
-
-
 def gated_delta_ops(q: Array, k: Array, v: Array, g: Array, beta: Array, state: Optional[Array] = None,
                     mask: Optional[Array] = None) -> tuple[Array, Array]:
     """Differentiable recurrence over the whole sequence (the ops loop the reference tests compare with)."""
-    return gdn_engine.recurrence(q, k, v, g, beta, _default_state(q, v, state), mask, chunk=64)
+    return gdn_engine.recurrence(q, k, v, g, beta, state, mask, chunk=64)
 
 
 def gated_delta_kernel(q: Array, k: Array, v: Array, g: Array, beta: Array, state: Optional[Array] = None,
                        mask: Optional[Array] = None) -> tuple[Array, Array]:
     """Forward-only recurrence (inference kernel; used for frozen layers, tools/frozen_gdn.py:19-25)."""
-    return gdn_engine.recurrence(q, k, v, g, beta, _default_state(q, v, state), mask, chunk=64,
+    return gdn_engine.recurrence(q, k, v, g, beta, state, mask, chunk=64,
                                  need_grad=False)
 
 

@@ -41,10 +41,6 @@ def gated_delta_ops_checkpointed(
     """
     if chunk <= 0:
         raise ValueError("chunk must be a positive integer")
-    batch, timesteps, key_heads, key_dim = q.shape
-    value_heads, value_dim = v.shape[-2:]
-    if state is None:
-        state = torch.zeros((batch, value_heads, value_dim, key_dim), dtype=torch.float32, device=q.device)
     return gdn_engine.recurrence(q, k, v, g, beta, state, mask, chunk)
 
 
@@ -72,10 +68,6 @@ def _checkpointed_update(
             use_kernel=use_kernel, lower_bound=lower_bound, allow_neg_eigval=allow_neg_eigval,
         )
     g, beta = gated_delta.gates(a, b, A_log, dt_bias, allow_neg_eigval, lower_bound)
-    if state is None:
-        batch, _, _, key_dim = q.shape
-        value_heads, value_dim = v.shape[-2:]
-        state = torch.zeros((batch, value_heads, value_dim, key_dim), dtype=torch.float32, device=q.device)
     return gated_delta_ops_checkpointed(q, k, v, g, beta, state, mask)
 
 

@@ -10,6 +10,7 @@ chunk from its boundary, like ``_chunk_vjp`` (``:273-320``) and ``mx.checkpoint`
 
 from __future__ import annotations
 
+import functools
 import os
 from typing import Optional
 
@@ -36,8 +37,23 @@ def gate_kind_for(g: torch.Tensor, log_gate: bool) -> int:
     raise ValueError(f"Unsupported gating shape {tuple(g.shape)}")
 
 
-def _saved_bytes(lib, B, T, Hk, Hv, Dk, Dv, chunk, gate, has_mask, form, in_code) -> int:
-    return int(lib.gdn_saved_bytes(B, T, Hk, Hv, Dk, Dv, chunk, gate, has_mask, form, in_code))
+# The library's answers to the size queries, which depend on these numbers alone: a query through ctypes takes 2 us, and a
+# training call asks four.
+@functools.lru_cache(maxsize=256)
+def _fwd_sizes(need_saved, B, T, Hk, Hv, Dk, Dv, chunk, gate, has_mask, form, in_code) -> tuple[int, int]:
+    """(saved bytes, workspace bytes) of a forward; raises where no form takes it."""
+    lib = L.load()
+    resolved = int(lib.gdn_select_form(Hv, Dk, Dv, has_mask, gate, form, in_code))
+    if resolved < 0:
+        L.check(resolved)
+    shape = (B, T, Hk, Hv, Dk, Dv, chunk, gate, has_mask, form, in_code)
+    return (int(lib.gdn_saved_bytes(*shape)) if need_saved else 0,
+            int(lib.gdn_fwd_workspace_bytes(*shape, int(need_saved))))
+
+
+@functools.lru_cache(maxsize=256)
+def _bwd_workspace_bytes(B, T, Hk, Hv, Dk, Dv, chunk, gate, has_mask, form, in_code) -> int:
+    return int(L.load().gdn_bwd_workspace_bytes(B, T, Hk, Hv, Dk, Dv, chunk, gate, has_mask, form, in_code))
 
 
 class _GDNRecurrence(torch.autograd.Function):
@@ -47,25 +63,20 @@ class _GDNRecurrence(torch.autograd.Function):
         # an output that the loss does not use reaches backward as None instead of a zero tensor filled for it
         # (the library takes a NULL exit-state cotangent as zero)
         ctx.set_materialize_grads(False)
-        dev = _require_device(q, k, v, g, beta, state)
+        dev = q.device
         B, T, Hk, Dk = q.shape
         Hv, Dv = v.shape[2], v.shape[3]
         in_dtype = q.dtype
         gate = gate_kind_for(g, log_gate)
         lib = L.load()
         has_mask = int(mask is not None)
-        resolved = int(lib.gdn_select_form(Hv, Dk, Dv, has_mask, gate, form, L.DTYPE_CODE[in_dtype]))
-        if resolved < 0:
-            L.check(resolved)
+        in_code = L.DTYPE_CODE[in_dtype]
+        n_saved, n_ws = _fwd_sizes(need_saved, B, T, Hk, Hv, Dk, Dv, chunk, gate, has_mask, form, in_code)
         y = torch.empty((B, T, Hv, Dv), device=dev, dtype=out_dtype)
         state_T = torch.empty((B, Hv, Dv, Dk), device=dev, dtype=torch.float32)
-        in_code = L.DTYPE_CODE[in_dtype]
-        n_saved = _saved_bytes(lib, B, T, Hk, Hv, Dk, Dv, chunk, gate, has_mask, form, in_code) if need_saved else 0
         # a forward-only call keeps nothing (saved = NULL); the saved buffer of a training call may still be empty
         # (T <= chunk), which is passed as a real pointer so that the library sees a training call
         saved = torch.empty((max(n_saved, 1) if need_saved else 0,), device=dev, dtype=torch.uint8)
-        n_ws = int(lib.gdn_fwd_workspace_bytes(B, T, Hk, Hv, Dk, Dv, chunk, gate, has_mask, form, in_code,
-                                               int(need_saved)))
         ws = torch.empty((n_ws,), device=dev, dtype=torch.uint8) if n_ws else None
         L.check(lib.gdn_fwd(L.ptr(q), L.ptr(k), L.ptr(v), L.ptr(g), L.ptr(beta), L.ptr(state),
                             L.ptr(mask), L.ptr(y), L.ptr(state_T), L.ptr(saved) if need_saved else None, n_saved,
@@ -102,9 +113,8 @@ class _GDNRecurrence(torch.autograd.Function):
         dv = torch.empty((B, T, Hv, Dv), device=dev, dtype=grad_dtype)
         dg = torch.empty(g.shape, device=dev, dtype=torch.float32)
         dbeta = torch.empty((B, T, Hv), device=dev, dtype=torch.float32)
-        dS0 = torch.empty((B, Hv, Dv, Dk), device=dev, dtype=torch.float32)
-        ws_bytes = int(lib.gdn_bwd_workspace_bytes(B, T, Hk, Hv, Dk, Dv, chunk, gate, has_mask, form,
-                                                   L.DTYPE_CODE[q.dtype]))
+        dS0 = torch.empty((B, Hv, Dv, Dk), device=dev, dtype=torch.float32) if ctx.needs_input_grad[5] else None
+        ws_bytes = _bwd_workspace_bytes(B, T, Hk, Hv, Dk, Dv, chunk, gate, has_mask, form, L.DTYPE_CODE[q.dtype])
         ws = torch.empty((max(ws_bytes, 1),), device=dev, dtype=torch.uint8)
         L.check(lib.gdn_bwd(L.ptr(q), L.ptr(k), L.ptr(v), L.ptr(g), L.ptr(beta), L.ptr(state), L.ptr(mask),
                             L.ptr(saved), saved.numel(), L.ptr(dy),
@@ -127,7 +137,8 @@ def _prep(q, k, v, g, beta, state, mask):
     q, k, v = (_aligned(x.to(common).contiguous()) for x in (q, k, v))
     g = g.to(torch.float32).contiguous()
     beta = beta.to(torch.float32).contiguous()
-    state = state.to(torch.float32).contiguous()
+    if state is not None:
+        state = state.to(torch.float32).contiguous()
     if mask is not None:
         mask = mask.to(device=q.device, dtype=torch.uint8).contiguous()
     return q, k, v, g, beta, state, mask
@@ -150,7 +161,7 @@ def check_shapes(q, k, v, g, beta, state, mask) -> None:
         raise ValueError(f"Unsupported gating shape {tuple(g.shape)}")
     if tuple(beta.shape) != (B, T, Hv):
         raise ValueError("beta must be [B, T, Hv]")
-    if tuple(state.shape) != (B, Hv, Dv, Dk):
+    if state is not None and tuple(state.shape) != (B, Hv, Dv, Dk):
         raise ValueError("state must be [B, Hv, Dv, Dk]")
     if mask is not None and tuple(mask.shape) != (B, T):
         raise ValueError("mask must be [B, T]")
@@ -173,7 +184,8 @@ def recurrence(q, k, v, g, beta, state, mask=None, chunk: int = 64, log_gate: bo
     ``y`` defaults to the dtype the reference's arithmetic promotes to (fp32 with an fp32 state).
     ``need_grad=False`` runs the forward-only path (no autograd graph).  ``form`` is "auto" (default, or the
     GDN_FORM environment variable), "recurrent" or "chunk".  ``backward_error``, when given, is raised as a
-    ``ValueError`` by the backward (the forward runs).
+    ``ValueError`` by the backward (the forward runs).  ``state`` may be None: zeros in fp32, without a tensor filled
+    with them.
     """
     if chunk <= 0:
         raise ValueError("chunk must be a positive integer")
@@ -182,12 +194,13 @@ def recurrence(q, k, v, g, beta, state, mask=None, chunk: int = 64, log_gate: bo
     out_dtype = output_dtype
     if out_dtype is None:
         out_dtype = q.dtype
-        for t in (k, v, g, beta, state):
+        for t in (k, v, g, beta):
             out_dtype = torch.promote_types(out_dtype, t.dtype)
+        out_dtype = torch.promote_types(out_dtype, torch.float32 if state is None else state.dtype)
         if out_dtype not in L.DTYPE_CODE:
             out_dtype = torch.float32
     grads_wanted = torch.is_grad_enabled() and any(
-        t.requires_grad for t in (q, k, v, g, beta, state))
+        t is not None and t.requires_grad for t in (q, k, v, g, beta, state))
     if need_grad is None:
         need_grad = grads_wanted
     form_code = default_form() if form is None else L.FORMS[form]
@@ -195,7 +208,7 @@ def recurrence(q, k, v, g, beta, state, mask=None, chunk: int = 64, log_gate: bo
     if not (need_grad and grads_wanted) and q.shape[1] == 1 and pm is None:
         # one token, no gradient: the decode step (gdn_recurrent_step's counterpart)
         with torch.no_grad():
-            state_T = torch.empty_like(ps)
+            state_T = torch.empty((q.shape[0], v.shape[2], v.shape[3], q.shape[3]), device=q.device, dtype=torch.float32)
             y = decode_step(pq[:, 0], pk[:, 0], pv[:, 0], pg[:, 0], pb[:, 0], ps, state_T, log_gate, out_dtype)
         return y[:, None], state_T
     if not (need_grad and grads_wanted):

@@ -129,4 +129,7 @@ def profile_collect() -> dict[str, tuple[float, int]]:
 
 
 def stream_handle(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    if device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    # without a Stream object around it (3 us each)
+    return torch._C._cuda_getCurrentRawStream(device.index)

@@ -62,10 +62,6 @@ def gated_delta_chunked(
             backward_error = "impl='kernel' requires key_dim divisible by 32"
         elif q.dtype != k.dtype or q.dtype != v.dtype:
             backward_error = "impl='kernel' requires q, k, and v to share a dtype"
-    batch, _, _, key_dim = q.shape
-    value_heads, value_dim = v.shape[-2:]
-    if state is None:
-        state = torch.zeros((batch, value_heads, value_dim, key_dim), dtype=torch.float32, device=q.device)
     return gdn_engine.recurrence(q, k, v, g, beta, state, mask, chunk, output_dtype=output_dtype,
                                  backward_error=backward_error)
 
