@@ -31,105 +31,53 @@ namespace ck {
               k_out_dt = AF32 ? (int)DT_F32 : (args).out_dt, k_grad_dt = AF32 ? (int)DT_F32 : (args).grad_dt; \
     (void)k_in_dt; (void)k_dy_dt; (void)k_out_dt; (void)k_grad_dt
 
-template <bool AF32, bool MASK>
-__global__ __launch_bounds__(NTP) void ck_prep_kernel(Args a) {
-    DTYPES_OF(a);
-    __shared__ __align__(16) float sK[C * LD];
-    __shared__ __align__(16) float sX[C * LD];
-    __shared__ __align__(16) float sA[C * LDC];
-    __shared__ __align__(16) float sT[C * LDC];
-    __shared__ float scratch[3 * 256];
-    __shared__ double sG[C];
-    __shared__ float sB[C], sGam[C], sRc[C];
-
-    const int c = blockIdx.x, hv = blockIdx.y, b = blockIdx.z;
-    const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, li = l & 15, lg = l >> 4;
-    const int T = a.T, hk = hv / (a.Hv / a.Hk), t0 = c * C, n = min(C, T - t0);
-    const size_t ci = chunk_index(a, b, hv, c);
-    const size_t qk0 = (((size_t)b * a.Ts + t0) * a.Hk + hk) * D, qk_row = (size_t)a.Hk * D;
-    const size_t v0 = (((size_t)b * a.Ts + t0) * a.Hv + hv) * D, v_row = (size_t)a.Hv * D;
-
-    TileRegs<C, D, NTP> rV;  // V is needed only after the inverse: fetch it now, store it later
-    tile_fetch(rV, elem_ptr(a.v, v0, k_in_dt), v_row, n, k_in_dt);
-    load_tile<C, D, NTP>(sK, LD, elem_ptr(a.k, qk0, k_in_dt), qk_row, n, k_in_dt);
-    load_tile<C, D, NTP>(sX, LD, elem_ptr(a.q, qk0, k_in_dt), qk_row, n, k_in_dt);
-    if (MASK && flag_set(chunk_flag(a, b, c))) load_queries<NTP>(sX, LD, a, b, hv, t0, n, k_in_dt, tid);
-    if (tid < C) {
-        // inclusive prefix sum of the log decays in fp64 across wave 0
-        float bt = 0.f, gl = 0.f;
-        if (tid < n) {
-            const size_t gi = ((size_t)b * a.Ts + t0 + tid) * a.Hv + hv;
-            bt = a.beta[gi];
-            gl = gate_log(a.g[gi], a.gate);
+// A [C][COLS] tile loaded by rows as raw 16-byte pieces, later written to LDS as fp32 (row stride ld); rows past n are
+// zero (they load row n - 1: no load under a branch).  Row stride rs in elements of dtype dt.
+template <int COLS>
+struct RowTile {
+    static constexpr int PER = C * COLS / 4 / NTS;  // pieces per thread in fp32, twice those in 16-bit dtypes
+    uint4 x[PER];
+    __device__ __forceinline__ void load(const void *p, unsigned rs, int n, int dt, int tid) {
+        const bool f32 = dt == DT_F32;
+        const int epq = f32 ? 4 : 8, vpr = COLS / epq;  // elements per piece, pieces per row
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            if (!f32 && i >= PER / 2) continue;
+            const int v = tid + i * NTS, r = v / vpr;
+            const unsigned off = ((unsigned)min(r, n - 1) * rs + epq * (v - r * vpr)) * (f32 ? 4 : 2);
+            const uint4 y = *reinterpret_cast<const uint4 *>(static_cast<const char *>(p) + off);
+            x[i] = r < n ? y : make_uint4(0u, 0u, 0u, 0u);
         }
-        const double x = wave_prefix_sum((double)gl);
-        sB[tid] = bt;
-        sG[tid] = x;
-        sGam[tid] = expf((float)x);
-        sRc[tid] = expf((float)(readlane_f64(x, 63) - x));  // gamma_C / gamma_r
     }
-    __syncthreads();
-    // K K^T (waves 0-3) and Q K^T (waves 4-7): each wave a 16-row strip of 4 tiles
-    {
-        const int r0 = 16 * (w & 3);
-        const bool isq = w >= 4;
-        f4 acc[4];
+    // with scale: row r times scale[r]
+    __device__ __forceinline__ void store(float *dst, int ld, int dt, int tid, const float *scale = nullptr) const {
+        const bool f32 = dt == DT_F32;
+        const int epq = f32 ? 4 : 8, vpr = COLS / epq;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) acc[t] = zero4();
-        mma_strip<D, 4>(acc, (isq ? sX : sK) + r0 * LD, LD, 1, sK, 1, LD, 16 * LD);
+        for (int i = 0; i < PER; ++i) {
+            if (!f32 && i >= PER / 2) continue;
+            const int v = tid + i * NTS, r = v / vpr;
+            float *d = dst + r * ld + epq * (v - r * vpr);
+            const float sc = scale ? scale[r] : 1.f;
+            if (f32 && !scale) {
+                *reinterpret_cast<uint4 *>(d) = x[i];
+            } else if (f32) {
+                *reinterpret_cast<float4 *>(d) = make_float4(sc * __uint_as_float(x[i].x), sc * __uint_as_float(x[i].y),
+                                                             sc * __uint_as_float(x[i].z), sc * __uint_as_float(x[i].w));
+            } else {
+                const uint32_t w[4] = {x[i].x, x[i].y, x[i].z, x[i].w};
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int r = r0 + 4 * lg + e, s2 = 16 * t + li;
-                const float gam = s2 <= r ? expf((float)(sG[r] - sG[s2])) : 0.f;
-                if (isq) a.w.P[ci * C * C + r * C + s2] = acc[t][e] * gam;
-                else sA[r * LDC + s2] = s2 < r ? sB[r] * acc[t][e] * gam : 0.f;
+                for (int k = 0; k < 4; ++k) {
+                    unpack16(w[k], dt, d[2 * k], d[2 * k + 1]);
+                    if (scale) d[2 * k] *= sc, d[2 * k + 1] *= sc;
+                }
             }
+        }
     }
-    __syncthreads();
-    unit_lower_inverse<NTP>(sA, sT, scratch);
-    for (int i = tid; i < C * D; i += NTP) {
-        const int r = i / D, j = i - r * D;
-        sK[r * LD + j] *= sB[r] * sGam[r];
-    }
-    {
-        const float *bp = sB;
-        tile_store(sX, LD, rV, k_in_dt, [bp](int r) { return bp[r]; });
-    }
-    __syncthreads();
-    // W = T diag(beta gamma) K (waves 0-3) and U = T diag(beta) V (waves 4-7), 16-row strips of 8 tiles
-    {
-        const int r0 = 16 * (w & 3);
-        const bool isu = w >= 4;
-        f4 acc[8];
-#pragma unroll
-        for (int t = 0; t < 8; ++t) acc[t] = zero4();
-        if (isu) mma_strip<C, 8>(acc, sT + r0 * LDC, LDC, 1, sX, LD, 1, 16);
-        else mma_strip<C, 8>(acc, sT + r0 * LDC, LDC, 1, sK, LD, 1, 16);
-        float *out = isu ? a.w.U : a.w.W;
-#pragma unroll
-        for (int t = 0; t < 8; ++t)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) out[ci * C * D + (r0 + 4 * lg + e) * D + 16 * t + li] = acc[t][e];
-    }
-    if (!a.fwd_only)
-        for (int i = tid; i < C * C; i += NTP) a.w.T[ci * C * C + i] = sT[(i / C) * LDC + (i % C)];
-    if (tid < C) a.w.G[ci * C + tid] = sG[tid];
-}
+};
 
-// ---------------------------------------------------------------------------------------------- ck_fwd
-//
-// The fp32 sequential kernels.  v_mfma_f32_16x16x4_f32 takes one A and one B element per lane (row li, k-index lg of the
-// four); since the order of a contraction is free, lane group lg takes the indices 16 s + 4 lg + i, i = 0..3, in the four
-// products of step s: an operand whose rows run along the contraction is then one 16-byte LDS read per step, and the
-// accumulators' four rows per lane are 16 contiguous bytes of the transposed tiles the next product reads.  The chunk's
-// tiles (W, Q, K, P; K, Q, W, P in the backward) are loaded by whole rows one chunk ahead and each has its own LDS space,
-// so a chunk step is one pass of stores, two of products and three barriers.  T^T, needed once, is read from memory in
-// operand form.  The first form shared the space between the tiles of the two passes (five barriers, two passes of
-// stores) and read every operand 4 bytes at a time: forward / backward at B = 1, T = 4096, Hv = 32
-// 356 / 364 -> 309 / 344 us (4.8 / 5.4 a step, of which the products take 1.5 / 1.7 at the fp32 matrix rate), at B = 2,
-// T = 1024 131 / 138 -> 106 / 126 us.
+
+__device__ __forceinline__ float at4(const float4 &x, int i) { return i == 0 ? x.x : i == 1 ? x.y : i == 2 ? x.z : x.w; }
 
 // acc[t] += A * B_t over NS steps of 16 contraction indices, B_t(k, n) at b[(n0 + 16 t + n) * ldb + k]: A(m, k) from a(s),
 // four contraction indices of this lane's row.  Two accumulator sets, so that two products of a tile are in flight.
@@ -175,42 +123,133 @@ struct ColsA {
     }
 };
 
-// A [C][COLS] tile loaded by rows as raw 16-byte pieces, later written to LDS as fp32 (row stride ld); rows past n are
-// zero (they load row n - 1: no load under a branch).  Row stride rs in elements of dtype dt.
-template <int COLS>
-struct RowTile {
-    static constexpr int PER = C * COLS / 4 / NTS;  // pieces per thread in fp32, twice those in 16-bit dtypes
-    uint4 x[PER];
-    __device__ __forceinline__ void load(const void *p, unsigned rs, int n, int dt, int tid) {
-        const bool f32 = dt == DT_F32;
-        const int epq = f32 ? 4 : 8, vpr = COLS / epq;  // elements per piece, pieces per row
+// acc[t] += A * B_t over the 16-index steps s0 <= s < s1 (wave-uniform), B_t(k, n) at b[k * LDB + 16 t + n]: operands in
+// the index order of mma4, B's elements read one by one (their columns run along the contraction).
+template <int LDB, class AOp>
+__device__ __forceinline__ void mma_cols(f4 (&acc)[4], int s0, int s1, AOp a, const float *b, int l) {
+    const float *bp = b + 4 * (l >> 4) * LDB + (l & 15);
+    for (int s = s0; s < s1; ++s) {
+        const float4 x = a(s);
+        float y[4][4];
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            if (!f32 && i >= PER / 2) continue;
-            const int v = tid + i * NTS, r = v / vpr;
-            const unsigned off = ((unsigned)min(r, n - 1) * rs + epq * (v - r * vpr)) * (f32 ? 4 : 2);
-            const uint4 y = *reinterpret_cast<const uint4 *>(static_cast<const char *>(p) + off);
-            x[i] = r < n ? y : make_uint4(0u, 0u, 0u, 0u);
-        }
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) y[i][t] = bp[(16 * s + i) * LDB + 16 * t];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(at4(x, i), y[i][t], acc[t], 0, 0, 0);
     }
-    __device__ __forceinline__ void store(float *dst, int ld, int dt, int tid) const {
-        const bool f32 = dt == DT_F32;
-        const int epq = f32 ? 4 : 8, vpr = COLS / epq;
+}
+
+// Bound by the latency of its phases (loads, K K^T | Q K^T, the inverse, W | U), so two workgroups share a CU: A, T and
+// the column halves of V take Q's place in LDS one after the other, 73 KiB instead of 107, within 128 VGPRs.  Products take
+// the blocks on and below the diagonal only.  At B = 4, T = 1024, Hv = 32 172 -> 107 us, T = 16384 in windows (the forward's
+// and the backward's launches) 1365 -> 851 us, one 64-token chunk 22 -> 20 us.
+template <bool AF32, bool MASK>
+__global__ __launch_bounds__(NTP, 4) void ck_prep_kernel(Args a) {
+    DTYPES_OF(a);
+    __shared__ __align__(16) float sK[C * LD];
+    __shared__ __align__(16) float sX[2 * C * LDC];  // Q; then A, half of diag(beta) V after the inverse | T
+    static_assert(C * LD <= 2 * C * LDC && D == 2 * C, "Q fits sX, half of V fits A");
+    float *const sA = sX, *const sT = sX + C * LDC;
+    __shared__ float scratch[3 * 256];
+    __shared__ double sG[C];
+    __shared__ float sB[C], sGam[C], sRc[C];
+
+    const int c = blockIdx.x, hv = blockIdx.y, b = blockIdx.z;
+    const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, li = l & 15, lg = l >> 4;
+    const int T = a.T, hk = hv / (a.Hv / a.Hk), t0 = c * C, n = min(C, T - t0);
+    const size_t ci = chunk_index(a, b, hv, c);
+    const size_t qk0 = (((size_t)b * a.Ts + t0) * a.Hk + hk) * D, qk_row = (size_t)a.Hk * D;
+    const size_t v0 = (((size_t)b * a.Ts + t0) * a.Hv + hv) * D, v_row = (size_t)a.Hv * D;
+
+    RowTile<D / 2> rV[2];  // the column halves of V, needed only after the inverse: fetch them now, store them later
+    for (int i = 0; i < 2; ++i) rV[i].load(elem_ptr(a.v, v0 + i * (D / 2), k_in_dt), (unsigned)v_row, n, k_in_dt, tid);
+    load_tile<C, D, NTP>(sK, LD, elem_ptr(a.k, qk0, k_in_dt), qk_row, n, k_in_dt);
+    load_tile<C, D, NTP>(sX, LD, elem_ptr(a.q, qk0, k_in_dt), qk_row, n, k_in_dt);
+    if (MASK && flag_set(chunk_flag(a, b, c))) load_queries<NTP>(sX, LD, a, b, hv, t0, n, k_in_dt, tid);
+    if (tid < C) {
+        // inclusive prefix sum of the log decays in fp64 across wave 0
+        float bt = 0.f, gl = 0.f;
+        if (tid < n) {
+            const size_t gi = ((size_t)b * a.Ts + t0 + tid) * a.Hv + hv;
+            bt = a.beta[gi];
+            gl = gate_log(a.g[gi], a.gate);
+        }
+        const double x = wave_prefix_sum((double)gl);
+        sB[tid] = bt;
+        sG[tid] = x;
+        sGam[tid] = expf((float)x);
+        sRc[tid] = expf((float)(readlane_f64(x, 63) - x));  // gamma_C / gamma_r
+    }
+    __syncthreads();
+    // K K^T (waves 0-3) and Q K^T (waves 4-7): each wave a 16-row strip of 4 tiles, those on and below the diagonal in
+    // pairs.  The two take the strips in opposite order, so that the waves of a SIMD (w, w + 4) have a short and a long one.
+    const bool hi = w >= 4;
+    const int r0 = 16 * (hi ? 7 - w : w);
+    {
+        f4 acc[2][2];
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            if (!f32 && i >= PER / 2) continue;
-            const int v = tid + i * NTS, r = v / vpr;
-            float *d = dst + r * ld + epq * (v - r * vpr);
-            if (f32) {
-                *reinterpret_cast<uint4 *>(d) = x[i];
-            } else {
-                const uint32_t w[4] = {x[i].x, x[i].y, x[i].z, x[i].w};
+        for (int t = 0; t < 2; ++t) acc[t][0] = acc[t][1] = zero4();
+        const RowsA x(hi ? sX : sK, LD, r0, l);
+        mma4<D / 16>(acc[0], x, sK, LD, 0, l);
+        if (r0 >= 32) mma4<D / 16>(acc[1], x, sK, LD, 32, l);
+        __syncthreads();  // Q read: A takes its place
 #pragma unroll
-                for (int k = 0; k < 4; ++k) unpack16(w[k], dt, d[2 * k], d[2 * k + 1]);
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int r = r0 + 4 * lg + e, s2 = 16 * t + li;
+                const float gam = s2 <= r ? expf((float)(sG[r] - sG[s2])) : 0.f, y = acc[t >> 1][t & 1][e];
+                if (hi) a.w.P[ci * C * C + r * C + s2] = y * gam;
+                else sA[r * LDC + s2] = s2 < r ? sB[r] * y * gam : 0.f;
             }
-        }
     }
-};
+    __syncthreads();
+    unit_lower_inverse<NTP>(sA, sT, scratch);
+    for (int i = tid; i < C * D / 4; i += NTP) {
+        const int r = i / (D / 4);
+        float4 *x = reinterpret_cast<float4 *>(sK + r * LD + 4 * (i - r * (D / 4)));
+        const float f = sB[r] * sGam[r];
+        *x = make_float4(x->x * f, x->y * f, x->z * f, x->w * f);
+    }
+    // W = T diag(beta gamma) K (waves 0-3) and U = T diag(beta) V (waves 4-7), 16-row strips by column halves; T is lower
+    // triangular
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        __syncthreads();  // A, or the first half of V, read
+        rV[h].store(sA, LDC, k_in_dt, tid, sB);
+        __syncthreads();
+        f4 acc[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc[t] = zero4();
+        const RowsA x(sT, LDC, r0, l);
+        if (hi) mma_cols<LDC>(acc, 0, r0 / 16 + 1, x, sA, l);
+        else mma_cols<LD>(acc, 0, r0 / 16 + 1, x, sK + h * (D / 2), l);
+        float *out = hi ? a.w.U : a.w.W;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) out[ci * C * D + (r0 + 4 * lg + e) * D + h * (D / 2) + 16 * t + li] = acc[t][e];
+    }
+    if (!a.fwd_only)
+        for (int i = tid; i < C * C; i += NTP) a.w.T[ci * C * C + i] = sT[(i / C) * LDC + (i % C)];
+    if (tid < C) a.w.G[ci * C + tid] = sG[tid];
+}
+
+// ---------------------------------------------------------------------------------------------- ck_fwd
+//
+// The fp32 sequential kernels.  v_mfma_f32_16x16x4_f32 takes one A and one B element per lane (row li, k-index lg of the
+// four); since the order of a contraction is free, lane group lg takes the indices 16 s + 4 lg + i, i = 0..3, in the four
+// products of step s: an operand whose rows run along the contraction is then one 16-byte LDS read per step, and the
+// accumulators' four rows per lane are 16 contiguous bytes of the transposed tiles the next product reads.  The chunk's
+// tiles (W, Q, K, P; K, Q, W, P in the backward) are loaded by whole rows one chunk ahead and each has its own LDS space,
+// so a chunk step is one pass of stores, two of products and three barriers.  T^T, needed once, is read from memory in
+// operand form.  The first form shared the space between the tiles of the two passes (five barriers, two passes of
+// stores) and read every operand 4 bytes at a time: forward / backward at B = 1, T = 4096, Hv = 32
+// 356 / 364 -> 309 / 344 us (4.8 / 5.4 a step, of which the products take 1.5 / 1.7 at the fp32 matrix rate), at B = 2,
+// T = 1024 131 / 138 -> 106 / 126 us.
 
 template <int VS, int MODE, bool AF32, bool MASK>
 __global__ __launch_bounds__(NTS) void ck_fwd_kernel(Args a) {
@@ -880,32 +919,11 @@ __device__ __forceinline__ void chunk_dg_dbeta(float *sE, const float (*sRow)[2]
 // u:  dg_u = sum_{r >= u} sum_{s' < u} E[r][s'].  Summing only straddling terms (each carrying the factor
 // exp(g_u)) keeps dg accurate for tiny decays, where a reverse cumulative sum of dG would cancel.
 
-__device__ __forceinline__ float at4(const float4 &x, int i) { return i == 0 ? x.x : i == 1 ? x.y : i == 2 ? x.z : x.w; }
-
 // f(std::integral_constant<int, n>) for a wave-uniform n of 1 or 2; nothing for 0.
 template <class F>
 __device__ __forceinline__ void tiles12(int n, F f) {
     if (n == 2) f(std::integral_constant<int, 2>{});
     else if (n == 1) f(std::integral_constant<int, 1>{});
-}
-
-// acc[t] += A * B_t over the 16-index steps s0 <= s < s1 (wave-uniform), B_t(k, n) at b[k * LD + 16 t + n]: operands in
-// the index order of mma4, B's elements read one by one (their columns run along the contraction).
-template <class AOp>
-__device__ __forceinline__ void mma_cols(f4 (&acc)[4], int s0, int s1, AOp a, const float *b, int l) {
-    const float *bp = b + 4 * (l >> 4) * LD + (l & 15);
-    for (int s = s0; s < s1; ++s) {
-        const float4 x = a(s);
-        float y[4][4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) y[i][t] = bp[(16 * s + i) * LD + 16 * t];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(at4(x, i), y[i][t], acc[t], 0, 0, 0);
-    }
 }
 
 // One value head hv = hk * rep + rr of key head hk.  dq | dk of the key head are summed in order (rr = 0, 1, ...)
@@ -1151,8 +1169,8 @@ __device__ __forceinline__ void bwd_local_f32_head(const Args &a, int c, int hk,
             dK[t][e] -= bg * Y2[t][e];
         }
     // dPG is lower triangular: row strip r0 of it ends, column strip r0 begins, at the diagonal block
-    mma_cols(dQ, 0, nd, RowsA(R4, LDC, r0, l), sKm + 64 * ch, l);
-    mma_cols(dK, nd - 1, C / 16, ColsA<LDC>(R4, r0, l), sQm + 64 * ch, l);
+    mma_cols<LD>(dQ, 0, nd, RowsA(R4, LDC, r0, l), sKm + 64 * ch, l);
+    mma_cols<LD>(dK, nd - 1, C / 16, ColsA<LDC>(R4, r0, l), sQm + 64 * ch, l);
     f4 Mt[2];
     {
         f4 kk[2] = {zero4(), zero4()};
@@ -1187,7 +1205,7 @@ __device__ __forceinline__ void bwd_local_f32_head(const Args &a, int c, int hk,
             if (s2 <= r) R4[r * LDC + s2] = R4[s2 * LDC + r] = Mt[t][e];
         }
     __syncthreads();
-    mma_cols(dK, 0, C / 16, RowsA(R4, LDC, r0, l), sKm + 64 * ch, l);
+    mma_cols<LD>(dK, 0, C / 16, RowsA(R4, LDC, r0, l), sKm + 64 * ch, l);
     // ---- phase 6: straddle sums for dg, dbeta, outputs.  R2 (dY) is free: E goes there.
     float *const sE = R2;
 #pragma unroll
@@ -1818,7 +1836,7 @@ __global__ __launch_bounds__(NTS) void ck_fwd_bf16_kernel(Args a) {
     __shared__ __align__(16) bfr sDh[VS * LDd];
     __shared__ __align__(16) bfr sDl[VS * LDd];
     // Q staged by rows, or read as fragments: from ck_prep's tile with per-channel gates, and from the input in a
-    // forward-only launch of 16-wide slices, whose operands are still in L2 (102 against 109 us at B = 1, T = 4096);
+    // forward-only launch of 16-wide slices, whose operands are still in L2 (107 against 114 us at B = 1, T = 4096);
     // recomputed windows write no y
     constexpr bool kQF = VG || (VS == 16 && MODE == FWD_ONLY), kRows = !kQF && kOut;
     __shared__ __align__(16) bfr sQ[kRows ? C * LA : 8];  // Q [r][j]
