@@ -13,8 +13,8 @@ Workloads (one GPU; the default is the T=4096 configuration the metric is quoted
   fp32_b1_t2048   B=1, T=2048, fp32, S0 ~ N(0, 0.02), full dS0
   ckpt_b1_t16384  B=1, T=16384, fp32, snapshots every 256 tokens, peak HBM reported
   masked_bf16_b4_t4096
-                  bf16_b4_t4096 with a mask (each sequence's last 10% masked, padding): two chunked
-                  passes plus the masked tokens' fix-up
+                  bf16_b4_t4096 with a mask (each sequence's last 10% masked, padding): one chunked
+                  pass with the masked tokens' own query rows, and their gradients' kernel
   vgate_bf16_b4_t4096
                   bf16_b4_t4096 with one log decay per key channel (g [B, T, Hv, D], the headline's gate
                   distribution per channel, taken as log decays as the headline takes its per-head gates); the
@@ -134,6 +134,7 @@ def kernel_model(name, B, T, Hk, Hv, D, in_b, fwd_only=False):
                        + cd * 2 * kv + cd * 4)
             # a forward-only call writes none of the backward's tiles: T, P^T, -W^T, Q^T
             return f, by - (ch * (cc * 4 + 2 * cc * 2 + cd * 2 + cd * 2 * kv) if fwd_only else 0)
+        f = f * 10 // 16  # the 16 x 16 blocks of the triangular operands and results
         return f, ch * (3 * cd * in_b + 2 * C * 4 + 2 * cd * 4 + 2 * cc * 4 + C * 8) - (ch * cc * 4 if fwd_only else 0)
     if name in ("ck_fwd", "ck_bwd_seq"):
         f = ch * (3 * 2 * cd * D + 2 * cc * D)
@@ -157,6 +158,7 @@ def kernel_model(name, B, T, Hk, Hv, D, in_b, fwd_only=False):
             kv = Hk / Hv  # key-head rows per value head
             return f, ch * (2 * dd * 2 + 2 * cd * 4 + 2 * cc * 2 + C * 8 + 2 * cd * 2 + 2 * cd * 2 * kv
                             + C * 4 + 2 * cd * 2 * kv + cd * 2 + 2 * C * 4)
+        f -= ch * 5 * 2 * cc * D * 6 // 16  # all but (M + M^T) K: the blocks on and below the diagonal
         by = ch * (2 * dd * 4 + 2 * cd * 4 + cc * 4 + C * 8 + 4 * cd * in_b + C * 4
                    + 2 * cd * 4 + cd * in_b + 2 * C * 4)
         return f, by
@@ -495,8 +497,8 @@ def main():
         if rec:
             traffic = rec["read_bytes"] + rec["write_bytes"]
     # the implementation model of a chunk kernel covers the whole batch once; a call that runs group-wise launches
-    # it several times per step, each launch over its share (a masked call's two passes each cover the whole batch)
-    per_step = lambda n: kt[n][1] / args.steps / (2 if w.get("masked_tail") else 1) if n.startswith("ck_") else 1
+    # it several times per step, each launch over its share
+    per_step = lambda n: kt[n][1] / args.steps if n.startswith("ck_") else 1
     i_flops, i_bytes = (int(x / per_step(dom)) for x in km(dom))
     roofline.update({
         "traffic": traffic, "traffic_source": "profiles/traffic.json (rocprofv3 FETCH_SIZE + WRITE_SIZE)"
