@@ -101,8 +101,10 @@ int gdn_select_form(int Hv, int Dk, int Dv, int has_mask, int gate_kind, int for
 
 /* Masks on the chunked form.  A masked step keeps the state but its output reads the candidate state.  The chunked
  * form runs the recurrence once, with decay 1 and beta 0 at masked tokens (the same states); a masked token's query is
- * decay (q - beta (k . q) k), one per value head, and beta (k . q) v is added to its y.  Needs Hv <= 256; the saved
- * buffer also holds the effective gates and those queries (4 bytes per (token, value head, key channel)). */
+ * decay (q - beta (k . q) k), one per value head, and beta (k . q) v is added to its y.  Needs Hv <= 256.  The saved
+ * buffer also holds the effective gates, the factors beta (k . q), a flag per 64-token chunk and those queries (4 bytes per
+ * (token, value head, key channel)); with bf16 inputs and chunk <= 64 also the queries transposed and what rounding the
+ * chunk-entry states to bf16 leaves of them (4 bytes each; with larger chunks the workspace holds these). */
 
 /* Size of the buffer gdn_fwd fills for gdn_bwd (the "saved" activations) for inputs of in_dtype. */
 size_t gdn_saved_bytes(int B, int T, int Hk, int Hv, int Dk, int Dv, int chunk, int gate_kind, int has_mask,

@@ -1549,6 +1549,47 @@ __device__ __forceinline__ void bwd_local_bf16_head(const Args &a, int c, int hk
                 dA[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at, xl, dA[t], 0, 0, 0);
             }
         }
+        if (mk) {
+            // A masked token's dg and dbeta follow from dQ alone (mask_bwd_fix_kernel), so a chunk that holds one adds
+            // what the bf16 tiles leave of the state and of an fp32 dY: dQ += dY hlo^T + dYlo h^T, dp += dYlo Delta^T
+            // (both lo parts straight from memory).  Without, dg of the masked tokens was off
+            // by 1.7e-3 of its norm, with 1e-4 (B = 2, T = 512, one token in five masked, fp32 dY).
+            const int x = opaque(l);
+            const bfr *hl = a.w.HLb + ci * D * D + frag_off<D>(64 * ch, 0) + 8 * x;
+            const float *ys = static_cast<const float *>(a.dy) + v0 + (size_t)min(r0 + (x & 15), n - 1) * v_row + 8 * (x >> 4);
+            bf8 hb[D / 32][4];
+            float4 y[DYF32 ? D / 32 : 1][2];
+#pragma unroll
+            for (int k = 0; k < D / 32; ++k) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) hb[k][t] = ld_frag(hl + frag_off<D>(16 * t, 32 * k));
+                if constexpr (DYF32) {
+                    y[k][0] = *reinterpret_cast<const float4 *>(ys + 32 * k);
+                    y[k][1] = *reinterpret_cast<const float4 *>(ys + 32 * k + 4);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < D / 32; ++k) {
+                const bf8 ay = frag(tY, LA, r0, 32 * k, l);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) dQ[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ay, hb[k][t], dQ[t], 0, 0, 0);
+                if constexpr (DYF32) {
+                    const float4 y0 = y[k][0], y1 = y[k][1];
+                    uint4 yh, yl;
+                    pk2(y0.x, y0.y, yh.x, yl.x);
+                    pk2(y0.z, y0.w, yh.y, yl.y);
+                    pk2(y1.x, y1.y, yh.z, yl.z);
+                    pk2(y1.z, y1.w, yh.w, yl.w);
+                    const bf8 al = r0 + li < n ? __builtin_bit_cast(bf8, yl) : zero_frag();
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                        dQ[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, frag(tH, LA, 64 * ch + 16 * t, 32 * k, l), dQ[t], 0, 0, 0);
+#pragma unroll
+                    for (int t = 0; t < 2; ++t)
+                        dp[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, frag(tLh, LA, 32 * ch + 16 * t, 32 * k, l), dp[t], 0, 0, 0);
+                }
+            }
+        }
         __syncthreads();  // sGam / sRc ready; the S1 tiles read
 #pragma unroll
         for (int t = 0; t < 4; ++t)
@@ -1952,6 +1993,16 @@ __global__ __launch_bounds__(NTS) void ck_fwd_bf16_kernel(Args a) {
                         (bfr)bfbits(h[t][e]);
             }
         }
+        if (MASK && kTiles && flags.cur) {  // ... and what that leaves of it
+            const int x = opaque(l);
+            bfr *const hl = a.w.HLb + ci * D * D + 16 * w * D;
+            const unsigned o = frag_off<D>(4 * (x >> 4), i0 + (x & 15));
+#pragma unroll
+            for (int t = 0; t < NTN; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    hl[o + frag_off<D>(e, 16 * t)] = (bfr)bfbits(h[t][e] - bf2f(bfbits(h[t][e])));  // i0 % 32 = 0 where t > 0
+        }
         if constexpr (kRows) store_row_tile(sQ, qr, tid);
         float *const sGam = sGamBuf[c & 1];
         if (!VG && tid < C) sGam[tid] = __builtin_amdgcn_exp2f((float)(cur.g * 1.4426950408889634));  // v_exp_f32 on log2 units
@@ -1975,7 +2026,7 @@ __global__ __launch_bounds__(NTS) void ck_fwd_bf16_kernel(Args a) {
         // W, Q and U fall free (64-wide slices have none to spare before), and arrive during Delta's conversion
         ValueTerms<DN> vt;
         bf8 ql[MASK ? 4 : 1];
-        if (MASK && flags.cur && ywave) {
+        if (MASK && kOut && flags.cur && ywave) {
             const int x = opaque(l), r = min(mrow + (x & 15), n - 1);
             const bfr *p = static_cast<const bfr *>(a.qm) + a.qm_lo + query_row(a, b, t0, hv) + (size_t)r * a.Hv * D + 8 * (x >> 4);
 #pragma unroll
@@ -1996,7 +2047,7 @@ __global__ __launch_bounds__(NTS) void ck_fwd_bf16_kernel(Args a) {
                 }
             }
         }
-        if (MASK && flags.cur && ywave) {
+        if (MASK && kOut && flags.cur && ywave) {
 #pragma unroll
             for (int k = 0; k < 4; ++k)
 #pragma unroll
@@ -2703,6 +2754,7 @@ ChunkSizes chunk_sizes(int B, int T, int Hk, int Hv, bool bf16, bool bwd, int vg
     put(s.QGb, vg ? n * cd * 2 : 0);
     put(s.KDb, vg && bwd ? n * cd * 2 : 0);
     put(s.QMb, bf16 && bwd && masked ? n * 2 * cd * 2 : 0);
+    put(s.HLb, bf16 && bwd && masked ? n * dd * 2 : 0);
     s.saved = off;
     off = 0;
     put(s.dH, n * dd * (bf16 ? 2 : 4));
@@ -2747,6 +2799,7 @@ static ck::Args make_args(const ChunkCall &cc) {
     a.w.QGb = static_cast<unsigned short *>(at(s.QGb));
     a.w.KDb = static_cast<unsigned short *>(at(s.KDb));
     a.w.QMb = static_cast<unsigned short *>(at(s.QMb));
+    a.w.HLb = static_cast<unsigned short *>(at(s.HLb));
     if (cc.work) {
         char *wk = static_cast<char *>(cc.work);
         a.w.dH = reinterpret_cast<float *>(wk + s.dH.off);
@@ -2787,9 +2840,10 @@ static void fwd_launch(const ck::Args &a, hipStream_t st, dim3 grid) {
     if constexpr (MT == 2) {
         hipLaunchKernelGGL((ck::ck_fwd_bf16_kernel<VS, MODE, true, false>), grid, dim3(ck::NTS), 0, st, a);
     } else {
-        // recomputed windows write no y: they need no query
-        with_flag(MODE != ck::FWD_RECOMPUTE && a.mask != nullptr, [&](auto mask) {
-            constexpr bool MASK = MODE != ck::FWD_RECOMPUTE && decltype(mask)::value;
+        // recomputed windows write no y and need no query; the bf16 set's still write the lo part of masked chunks' states
+        constexpr bool masks = MT == 1 || MODE != ck::FWD_RECOMPUTE;
+        with_flag(masks && a.mask != nullptr, [&](auto mask) {
+            constexpr bool MASK = masks && decltype(mask)::value;
             if constexpr (MT == 1)
                 hipLaunchKernelGGL((ck::ck_fwd_bf16_kernel<VS, MODE, false, MASK>), grid, dim3(ck::NTS), 0, st, a);
             else

@@ -261,6 +261,7 @@ struct Bufs {
     unsigned short *KDb;  // [B][Hv][NC][C][D]     K * exp(G_C - G), fragment order (ck_bwd_seq's A operand of dDelta)
     // masked calls: the chunks that hold a masked token keep the transposed queries per value head, hi and lo
     unsigned short *QMb;  // [B][Hv][NC][2][D][C]  Q~^T hi, lo (fragment order; in the place of Q^T)
+    unsigned short *HLb;  // [B][Hv][NC][D][D]     what H leaves of the chunk-entry state, h - H (fragment order): dL/dq~ needs it
     // per-channel decays (not log decays): what ck_bwd_local_vg leaves for ck_vg_dg, VGD_FLOATS per chunk-head
     float *vgd;
 };

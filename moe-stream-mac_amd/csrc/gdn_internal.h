@@ -49,7 +49,7 @@ struct ChunkSizes {
     Buf H, G, T, P, W, U, Dl;         // tile set
     Buf Wb, KTb, Pb, PTb, QTb, nWTb;  // bf16 operand tiles of the bf16 set
     Buf Gv, QGb, KDb;                 // per-channel gates (bf16 set)
-    Buf QMb;                          // masked calls (bf16 set)
+    Buf QMb, HLb;                     // masked calls (bf16 set)
     size_t saved;                     // size of the tile set
     Buf dH, dDl, part, vgd;           // backward workspace
     size_t work;                      // its size

@@ -14,11 +14,13 @@
 // (mask_bwd_fix_kernel):
 //   dv = e dy,   dc = beta (v . dy - d k . X),   dbeta = c (v . dy - d k . X),   dd = q . X - beta c k . X,
 //   dq = sum over the key head's value heads of d X + dc k,   dk = ... of dc q - d beta c X.
+// With no other use of the state behind them, dc, dbeta and dd are as exact as X: in the bf16 set a flagged chunk's dQ
+// therefore takes in the lo parts of the entry state and of an fp32 dY too (ck_bwd_local_bf16), which costs 70 us below.
 //
 // The first form of this path ran the recurrence twice, the second time with k as the query, around fp32 copies of
 // every output, cotangent and gradient: at B = 4, T = 4096, Hv = 32, bf16, a fifth of the tokens masked, 3.78 ms per
-// forward + VJP, with the query rows 1.82 ms (1.42 ms without a mask).  Both kernels here are bound by the rows of the
-// masked tokens: 43 us (forward) and 80 us (backward) of that.
+// forward + VJP, with the query rows 1.91 ms (1.42 ms without a mask).  Both kernels here are bound by the rows of the
+// masked tokens: 43 us (forward) and 81 us (backward) of that.
 #include "gdn_common.h"
 #include "gdn_internal.h"
 
