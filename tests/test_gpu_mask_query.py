@@ -66,6 +66,33 @@ def test_masked_chunks_of_every_kind(dev, dtype, y_dtype, rep, log_gate, T):
         assert np.abs(a - b).max() <= bar * np.abs(b).max(), name
 
 
+@pytest.mark.parametrize("dtype,y_dtype,log_gate", [("fp32", "fp32", False), ("fp16", "fp32", True), ("bf16", "bf16", True)])
+def test_masked_chunks_of_every_kind_at_wide_slices(dev, dtype, y_dtype, log_gate):
+    """128 heads take 64-wide slices in the sequential kernels: training, checkpointed and forward-only calls."""
+    import gdn_engine
+    B, T, Hk, Hv = 4, 200, 16, 32
+    rng = np.random.default_rng(T)
+    d = O.make_inputs(B, T, Hk, Hv, D, seed=T, s0_std=0.05)
+    rnd = lambda x, dt: torch.tensor(x).to(DT[dt]).float().numpy()
+    d = dict(d, mask=_mask(B, T, rng), dS_T=(0.1 * rng.standard_normal(d["state"].shape)).astype(np.float32),
+             q=rnd(d["q"], dtype), k=rnd(d["k"], dtype), v=rnd(d["v"], dtype), dy=rnd(d["dy"], y_dtype))
+    (wy, wS), wg = O.gated_delta_chunked_vjp(d["q"], d["k"], d["v"], d["decay"], d["beta"], d["state"], d["mask"], d["dy"],
+                                             d["dS_T"], chunk=64, dtype=np.float64)
+    if log_gate:
+        wg = (*wg[:3], wg[3] * d["decay"], *wg[4:])
+    want = (wy, wS, *wg)
+    with torch.no_grad():
+        t = lambda x, dt=torch.float32: torch.tensor(x, device=dev, dtype=dt)
+        fwd = gdn_engine.recurrence(*(t(d[n], DT[dtype]) for n in "qkv"), t(d["g_log" if log_gate else "decay"]), t(d["beta"]),
+                                    t(d["state"]), t(d["mask"], torch.bool), log_gate=log_gate, output_dtype=DT[y_dtype],
+                                    need_grad=False)
+    for got in (_run(d, dev, dtype, log_gate, DT[y_dtype]), _run(d, dev, dtype, log_gate, DT[y_dtype], chunk=128),
+                [x.double().cpu().numpy() for x in fwd]):
+        for name, a, b in zip(NAMES, got, want):
+            bar = 1e-2 if dtype == "bf16" else 1e-3 if dtype == "fp16" and name in ("dq", "dk", "dv") else 1e-4
+            assert np.abs(a - b).max() <= bar * np.abs(b).max(), name
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "fp32"])
 def test_masked_groups_equal_whole_calls(dev, dtype):
     """Groups of 2048 chunk-heads: 64 heads x 2200 tokens take two groups, forward-only and checkpointed."""
