@@ -173,11 +173,11 @@ _LINEAR_FORWARD, _NORM_FORWARD = nn.Linear.forward, RMSNormGated.forward
 
 def _own_update(update) -> bool:
     """Whether an inference call of ``update`` ends in this package's gated_delta_update: itself, or one that an
-    install() bound over it."""
+    install() bound over it.  Installs that alternate can leave two modules calling each other: that ends nowhere."""
+    names = {"gdn_vjp": "_vjp_update", "gdn_checkpoint": "_checkpointed_update", "frozen_gdn": "_marked_update"}
     while update is not gated_delta.gated_delta_update:
         mod = sys.modules.get(getattr(update, "__module__", None))
-        names = {"gdn_vjp": "_vjp_update", "gdn_checkpoint": "_checkpointed_update", "frozen_gdn": "_marked_update"}
-        if mod is None or update is not getattr(mod, names.get(mod.__name__, ""), None):
+        if mod is None or update is not getattr(mod, names.pop(mod.__name__, ""), None):  # each module once
             return False
         update = mod._ORIGINAL_UPDATE
     return True
