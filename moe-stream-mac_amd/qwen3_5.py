@@ -27,6 +27,7 @@ import torch.nn.modules.module as nn_module
 
 import gated_delta
 import gdn_block
+import gdn_engine
 import gdn_lib as L
 from gated_delta import gated_delta_update, normalize_qk  # noqa: F401  (rebound by install())
 
@@ -152,6 +153,7 @@ class GatedDeltaNet(nn.Module):
 
     def _decode_token(self, x: Array, cache: "GDNCache") -> Array:
         """One token of B sequences: the in-projections, everything between the projections, the out-projection."""
+        gdn_engine.default_form()  # raises on an unknown GDN_FORM, as the update does
         B, _, h = x.shape
         x2 = x.reshape(B, h)
         lins = (self.in_proj_qkv, self.in_proj_z, self.in_proj_b, self.in_proj_a)

@@ -115,3 +115,15 @@ def test_calls_that_run_step_by_step(dev):
         Q.gated_delta_update = keep
     blk.out_proj = torch.nn.Linear(2 * D, 64, bias=True, device=dev)
     assert not blk._decodes_fused(x, c)
+
+
+def test_unknown_form_is_refused(dev, monkeypatch):
+    """GDN_FORM names no form: the fused token raises what the step-by-step one does, and leaves the cache alone."""
+    import qwen3_5 as Q
+    blk = Q.GatedDeltaNet(Q.ModelArgs(hidden_size=64, linear_num_key_heads=1, linear_num_value_heads=2,
+                                      linear_key_head_dim=D, linear_value_head_dim=D)).to(dev).eval()
+    x, c = torch.randn(2, 1, 64, device=dev), Q.GDNCache()
+    monkeypatch.setenv("GDN_FORM", "chunked")
+    with torch.no_grad(), pytest.raises(ValueError, match="GDN_FORM"):
+        blk(x, cache=c)
+    assert c[0] is None and c[1] is None
