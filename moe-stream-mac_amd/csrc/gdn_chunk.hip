@@ -574,7 +574,8 @@ template <int MODE, bool AF32, bool MASK>
 __global__ __launch_bounds__(NTS) void ck_fwd_wide_kernel(Args a) {
     constexpr int VS = 64;
     DTYPES_OF(a);
-    constexpr bool kTiles = MODE != FWD_ONLY, kOut = MODE != FWD_RECOMPUTE;
+    static_assert(MODE != FWD_RECOMPUTE, "recomputed windows take narrower slices");
+    constexpr bool kTiles = MODE != FWD_ONLY;
     constexpr int LV = VS + 4;
     constexpr int NTN = VS / 16;                 // value tiles of the slice
     constexpr int DN = NTN >= 2 ? NTN / 2 : 1;   // value tiles per wave for [C][VS] products
@@ -668,7 +669,7 @@ __global__ __launch_bounds__(NTS) void ck_fwd_wide_kernel(Args a) {
         tile_store(sQ, LD, rK, k_in_dt, RcScale{sG});
         __syncthreads();
         if (c + 1 < ce) fetchB(c + 1);
-        if (cwave && kOut) {
+        if (cwave) {
             // Y = diag(gamma) Q h + P Delta
 #pragma unroll
             for (int t = 0; t < DN; ++t)
@@ -696,7 +697,7 @@ __global__ __launch_bounds__(NTS) void ck_fwd_wide_kernel(Args a) {
         for (int t = 0; t < NTN; ++t) h[t] *= gC;
         mma_strip<C, NTN>(h, sQ + 16 * w, 1, LD, sD, LV, 1, 16);
     }
-    if (kOut && a.state_T) store_state_acc<NTN>(a.state_T, h, head, i0, w, lg, li);
+    if (a.state_T) store_state_acc<NTN>(a.state_T, h, head, i0, w, lg, li);
 }
 
 
@@ -2861,9 +2862,15 @@ static void fwd_launch(const ck::Args &a, hipStream_t st, dim3 grid) {
 template <int MT, int VS>
 static void seq_launch(const ck::Args &a, hipStream_t st, bool fwd) {
     const dim3 grid(CK_D / VS, a.Hv, seq_z(a));
+    if (fwd && a.recompute) {
+        // fp32 windows recomputed side by side (no y, so no Q and P in LDS) take 32-wide slices at most: 628 us per
+        // checkpointed T = 16384 backward, two workgroups to a CU, 668 at 64
+        constexpr int RVS = MT == 0 && VS > 32 ? 32 : VS;
+        fwd_launch<MT, RVS, ck::FWD_RECOMPUTE>(a, st, dim3(CK_D / RVS, a.Hv, seq_z(a)));
+        return;
+    }
     if (fwd) {
-        if (a.recompute) fwd_launch<MT, VS, ck::FWD_RECOMPUTE>(a, st, grid);
-        else if (a.fwd_only) fwd_launch<MT, VS, ck::FWD_ONLY>(a, st, grid);
+        if (a.fwd_only) fwd_launch<MT, VS, ck::FWD_ONLY>(a, st, grid);
         else fwd_launch<MT, VS, ck::FWD_TRAIN>(a, st, grid);
         return;
     }
@@ -2883,11 +2890,7 @@ static void seq_launch(const ck::Args &a, hipStream_t st, bool fwd) {
 
 template <int MT>
 static void seq_dispatch(const ck::Args &a, hipStream_t st, bool fwd) {
-    int vs = slice_width(seq_z(a) * a.Hv);
-    // fp32 windows recomputed side by side (no y, so no Q and P in LDS): 628 us per checkpointed T = 16384 backward at
-    // 32-wide slices, two workgroups to a CU, 668 at 64
-    if (MT == 0 && a.recompute) vs = vs > 32 ? 32 : vs;
-    switch (vs) {
+    switch (slice_width(seq_z(a) * a.Hv)) {
         case 64: seq_launch<MT, 64>(a, st, fwd); break;
         case 32: seq_launch<MT, 32>(a, st, fwd); break;
         default: seq_launch<MT, 16>(a, st, fwd); break;
