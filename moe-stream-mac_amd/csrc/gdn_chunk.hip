@@ -1956,20 +1956,21 @@ __global__ __launch_bounds__(NTS) void ck_fwd_bf16_kernel(Args a) {
     };
     uint32_t ahead = 0;
     auto read_ahead = [&](int c) {
-        // threads below LPS: this slice's share of the 512 lines of W, (K diag(gamma_C / gamma))^T, P and Q; threads
+        // threads below LPS: this slice's share of the 512 lines of W, (K diag(gamma_C / gamma))^T, P and Q (the first two
+        // where no y is written; a masked chunk's query rows (hi) in the place of Q, by the flag of the chunk before); threads
         // 256..: the slice's own blocks of U (accumulator order: VS / 16 blocks of 1 KiB per 16-row strip)
-        constexpr int S = D / VS, LPS = 4 * kLine / S, ULN = VS / 2;
+        constexpr int S = D / VS, LPS = (kOut ? 4 : 2) * kLine / S, ULN = VS / 2;
         const size_t ci = head * a.NC + c;
         const char *p = nullptr;
         if (tid < LPS) {
             const int i = sb.slice * LPS + tid, tile = i / kLine, ln = i % kLine;  // each tile is 128 lines
+            const size_t row = (size_t)b * a.Ts + min(c * C + ln / 2, T - 1);
             if (tile == 0) p = reinterpret_cast<const char *>(a.w.Wb + ci * C * D) + kLine * ln;
             else if (tile == 1) p = reinterpret_cast<const char *>(a.w.KTb + ci * D * C) + kLine * ln;
             else if (tile == 2) p = reinterpret_cast<const char *>(a.w.Pb + ci * 2 * C * C) + kLine * ln;
             else if (VG) p = reinterpret_cast<const char *>(a.w.QGb + ci * C * D) + kLine * ln;
-            else p = reinterpret_cast<const char *>(static_cast<const bfr *>(a.q) +
-                                                    (((size_t)b * a.Ts + min(c * C + ln / 2, T - 1)) * a.Hk + hk) * D) +
-                     kLine * (ln & 1);
+            else if (MASK && flags.nxt) p = reinterpret_cast<const char *>(static_cast<const bfr *>(a.qm) + (row * a.Hv + hv) * D) + kLine * (ln & 1);
+            else p = reinterpret_cast<const char *>(static_cast<const bfr *>(a.q) + (row * a.Hk + hk) * D) + kLine * (ln & 1);
         } else if (tid >= 256 && tid < 256 + 4 * ULN) {
             const int i = tid - 256, m = i / ULN;
             p = reinterpret_cast<const char *>(a.w.U + ci * C * D + acc_off(16 * m, i0)) + kLine * (i - m * ULN);
@@ -2548,7 +2549,8 @@ __global__ __launch_bounds__(NTS) void ck_bwd_seq_bf16_kernel(Args a) {
             const int i = sb.slice * LPS + tid, tile = i / kLine, ln = i % kLine;  // each tile is 128 lines
             if (tile == 0) p = reinterpret_cast<const char *>(a.w.PTb + ci * 2 * C * C) + kLine * ln;
             else if (tile == 1)
-                p = reinterpret_cast<const char *>(a.w.QTb + (VG ? ci : ((size_t)b * a.Hk + hk) * a.NC + c) * D * C) + kLine * ln;
+                p = reinterpret_cast<const char *>(MASK && flags.nxt ? a.w.QMb + ci * 2 * D * C  // by the flag of the chunk after
+                                                   : a.w.QTb + (VG ? ci : ((size_t)b * a.Hk + hk) * a.NC + c) * D * C) + kLine * ln;
             else if (tile == 2) p = reinterpret_cast<const char *>(a.w.nWTb + ci * D * C) + kLine * ln;
             else if (tile == 3) p = reinterpret_cast<const char *>(reinterpret_cast<const bfr *>(a.w.T) + ci * 2 * C * C) + kLine * ln;
             else if (VG) p = reinterpret_cast<const char *>(a.w.KDb + ci * C * D) + kLine * ln;
