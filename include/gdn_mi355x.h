@@ -149,7 +149,8 @@ int gdn_decode_step(const void *q, const void *k, const void *v, const float *g,
                     int in_dtype, int out_dtype, int gate_kind, void *stream);
 
 /* One decoded token of a whole GDN block (the steps of engine/src/gdn_layer.c:18-58), batched over B sequences, in
- * three launches: gdn_small_linears over the in-projections, gdn_block_decode, gdn_small_linears over the out-projection.
+ * three calls: gdn_small_linears over the in-projections, gdn_block_decode, gdn_small_linears over the out-projection
+ * (three launches up to 8 sequences; gdn_small_linears takes one per 8).
  *
  * gdn_small_linears: y[i] [tokens][n[i]] = x [tokens][k] * w[i]^T, w[i] [n[i]][k], for count <= 4 weights that share x;
  * one dtype throughout, fp32 sums.  At most 16 tokens, k a multiple of 8 (else GDN_ERR_UNSUPPORTED); x and the weights

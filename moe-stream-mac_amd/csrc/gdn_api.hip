@@ -104,8 +104,8 @@ static int check_shape(int B, int T, int Hk, int Hv, int Dk, int Dv, int chunk, 
     return GDN_OK;
 }
 
-// Masked calls run on the chunked form (gdn_mask.hip) up to mask_max_heads() value heads.  Per-channel gates run on the chunked form with bf16 inputs and no mask
-// (gdn_chunk_vg.hip).
+// Masked calls run on the chunked form (gdn_mask.hip) up to mask_max_heads() value heads.  Per-channel gates run on the
+// chunked form with bf16 inputs and no mask (gdn_chunk_vg.hip).
 static bool chunk_eligible(int Hv, int Dk, int Dv, int has_mask, int gate, int in_dt) {
     if (Dk != 128 || Dv != 128) return false;
     if (gate_vec(gate)) return !has_mask && chunk_vg_supported(in_dt);

@@ -15,7 +15,8 @@
 //   ck_fwd[_bf16]        grid (D/VS, Hv, B): sequential over chunks; one value slice of h lives in accumulators.
 //   ck_bwd_seq[_bf16]    grid (D/VS, Hv, B): reverse over chunks; the state adjoint dh and dDelta.
 //   ck_bwd_local[_bf16]  grid (NC, Hk, B): dv, dbeta, dg of one chunk for each value head of a key head in turn,
-//                        and the key head's dq, dk (the value heads' parts summed in order).
+//                        and the key head's dq, dk (the value heads' parts summed in order).  fp32 set on small grids:
+//                        (NC, Hv, B), one value head each, the parts summed by ck_local_sum (local_split).
 #include "gdn_chunk_common.h"
 
 namespace gdn {
@@ -1829,16 +1830,15 @@ __global__ __launch_bounds__(NTB) void ck_bwd_local_bf16_kernel(Args a) {
 // (with the reading ahead that the registers leave room for), ck_fwd_bf16 350 -> 335 us at B = 4, T = 4096, Hv = 32; 152
 // -> 142 and 166 -> 142 us at B = 1, T = 4001.
 
-// Reading ahead (slices narrower than 64).  The D / VS workgroups of a head ask for the same tiles at the same time,
+// Reading ahead.  The D / VS workgroups of a head ask for the same tiles at the same time,
 // so a line that is not in L2 yet is missed by each of them, and the loads of the next chunk, issued one step ahead,
 // come back late: with tiles that outgrow the Infinity Cache a step took 3.0 us against 1.7 us within it.  Each slice
 // therefore reads one 4-byte word of its own share (1 / (D / VS)) of the shared lines of the chunk kReadAhead steps on
-// (at most one load per thread and step), so each line leaves memory once and the fragment loads hit L2.  At B = 1,
-// T = 4001, Hv = 32: ck_fwd_bf16 188 -> 166 us, ck_bwd_seq_bf16 170 -> 152 us; at B = 2, T = 2048: 148 -> 129 and
-// 135 -> 125 us; three, four and six steps ahead gain less (170, 179, 184 us forward at B = 1).  At 64-wide slices
-// the backward takes it (B = 4, T = 4096: 334 -> 282 us) and the forward has no use for it (335 us with and without);
-// masked (343 -> 363 us) and per-channel launches of that width have no registers for it.  Args::read_ahead says whether the
-// launch's tiles outgrow the cache.
+// (at most one load per thread and step), so each line leaves memory once and the fragment loads hit L2 (the figures are
+// at kReadAheadBytes); three, four and six steps ahead gain less (170, 179, 184 us against 166 in the forward at B = 1,
+// T = 4001).  At 64-wide slices the backward takes it and the forward has no use for it (335 us with and without at B = 4,
+// T = 4096); masked (343 -> 363 us) and per-channel launches of that width have no registers for it.  Args::read_ahead says
+// whether the launch's tiles outgrow the cache.
 constexpr int kReadAhead = 2, kLine = 128;  // bytes of an L2 line
 
 // A [C][D] bf16 tile of the input (row stride rs elements) by whole rows, two 16-byte pieces per thread; rows past n read
@@ -2432,8 +2432,9 @@ __global__ __launch_bounds__(NTP, 2) void ck_prep_bf16_kernel(Args a) {
 // and it saves TdD = T^T dDelta (fp32 [C][D]), the only form in which ck_bwd_local_bf16 needs T and dDelta.
 // The A operands P^T (hi / lo), Q^T and -W^T, written by ck_prep, are read as MFMA fragments from global memory into
 // registers one chunk ahead, with the chunk's dY slice; LDS carries what the waves exchange: dh' as the operand [i][j]
-// (hi / lo), dY^T, (diag(gamma) dY)^T (hi / lo) and dDelta^T (hi / lo), K (by rows, as the forward's Q), and T^T (hi / lo, fragment order), whose 32 bytes per thread are loaded one chunk ahead and stored between the
-// two barriers of the chunk that uses them.  Two barriers per chunk.
+// (hi / lo), dY^T, (diag(gamma) dY)^T (hi / lo) and dDelta^T (hi / lo), K (by rows, as the forward's Q), and T^T
+// (hi / lo, fragment order), whose 32 bytes per thread are loaded one chunk ahead and stored between the two barriers of
+// the chunk that uses them.  Two barriers per chunk.
 template <bool VG>
 struct BwdFrags {
     bf8 K[VG ? 4 : 1], PT[4], QT[2], WT[2];  // K: per-channel gates only; PT[0..1] hi, PT[2..3] lo; WT = -W^T
@@ -2770,9 +2771,17 @@ ChunkSizes chunk_sizes(int B, int T, int Hk, int Hv, bool bf16, bool bwd, int vg
 }
 
 // The tile set of a launch from which the sequential kernels read ahead (kReadAhead): tiles that ck_prep has just left
-// in the 256 MiB Infinity Cache come fast enough without, and the extra loads cost.  Whole passes with / without, at
-// Hv = 32: tile set 150 MiB (T = 1536) 200 / 201 us, 175 MiB (T = 1792) 234 / 249 us, 200 MiB (T = 2048) 262 / 286 us;
-// a forward-only group (161 MiB) 178 / 172 us at B = 1.
+// in the 256 MiB Infinity Cache come fast enough without, and the extra loads cost.  ck_fwd and ck_bwd_seq with / without,
+// in us at Hv = 32 (Hv = 16 alike), the line between the second and the third column of each row:
+//   16 wide (B = 1)   100 MiB 31.9 / 32.3, 38.0 / 36.5   150: 45.7 / 45.5, 54.4 / 52.1   175: 55.6 / 59.2, 64.4 / 68.4
+//                     200: 64.5 / 74.1, 76.8 / 86.5      400: 141 / 177, 144 / 171
+//   32 wide (B = 2)   100 MiB 27.1 / 27.1, 26.5 / 26.5   150: 36.5 / 37.2, 37.3 / 37.8   200: 62.8 / 64.9, 57.3 / 65.7
+//                     400: 124 / 140, 101 / 125          800: 209 / 248, 187 / 235
+//   64 wide (B = 4)   backward only                      150: 32.7 / 31.4               200: 44.3 / 51.5
+//                     400: 81.1 / 92.3                   1600: 285 / 333
+//   masked (B = 1)    100 MiB 42.2 / 42.2, 40.7 / 39.4                                   200: 86.1 / 97.0, 85.5 / 99.6
+//   per channel (1)   136 MiB 32.4 / 31.7, 36.6 / 35.2                                   204: 55.6 / 60.0, 60.3 / 68.8
+//   forward only       84 MiB (B = 1) 57.0 / 53.3        165 (1): 105 / 107              169 (2): 166 / 180
 constexpr size_t kReadAheadBytes = (size_t)168 << 20;
 
 static ck::Args make_args(const ChunkCall &cc) {

@@ -242,9 +242,9 @@ struct Bufs {
     float *dH;   // [B][Hv][NC][D][D]  adjoint of each chunk's exit state, [j][i] like H (bf16 in the bf16 path)
     float *dDl;  // [B][Hv][NC][C][D]  dDelta (bf16 path: TdD = T^T dDelta, fp32)
     float *part; // [B][T][Hv][2][D]   ck_bwd_local scratch: the running dq | dk sum of a key head (per-channel
-                 // gates: in the rows [B][T][Hk][2][D]; fp32 set: in the slot of the key head's first value head, the
-                 // other slots parking each value head's dW; the bf16 set with one gate per head keeps the sum in
-                 // registers and has no part buffer)
+                 // gates: in the rows [B][T][Hk][2][D]; fp32 set: in the slot of the key head's first value head, or, one
+                 // workgroup per value head, each head's own dq | dk in its slot; the bf16 set with one gate per head
+                 // keeps the sum in registers and has no part buffer)
     // bf16 operand tiles written by ck_prep for the bf16 sequential kernels (raw bf16 bits), each [M][K] tile in
     // fragment order (frag_off<K>); the bf16 set keeps U in accumulator order (acc_off)
     unsigned short *Wb;   // [B][Hv][NC][C][D]     W
@@ -513,7 +513,8 @@ __device__ __forceinline__ void unit_lower_inverse(const float *sA, float *sT, f
 // Threads per workgroup: ck_prep, the sequential kernels and ck_bwd_local all run 8 waves.
 constexpr int NTP = 512;  // ck_prep: 8 waves
 constexpr int NTS = 512;  // sequential kernels: 8 waves
-constexpr int NTB = 512;  // ck_bwd_local: 8 waves; waves w and w+4 share the 16-row strip w%4 (column halves)
+constexpr int NTB = 512;  // ck_bwd_local: 8 waves, four 16-row strips by two column halves (w / 4): strip w % 4, in the
+                          // fp32 set 3 - w % 4 in the upper half (its triangular products differ in length by strip)
 
 // Sum over the wave, the same in every lane: DPP row sums, then the four row totals read as scalars.
 __device__ __forceinline__ float wave_sum(float x) {

@@ -1,5 +1,5 @@
-// One decoded token of a whole GDN block (engine/src/gdn_layer.c:18-58 at one token) in three launches: the
-// in-projections, everything between the projections, and the out-projection.
+// One decoded token of a whole GDN block (engine/src/gdn_layer.c:18-58 at one token) in three launches (five for 9 to 16
+// sequences): the in-projections, everything between the projections, and the out-projection.
 //
 // As separate calls the token takes five library GEMMs, the conv, its state, the gates, the recurrence, the norm and the
 // parameters' conversions to fp32, 16 launches that each cost more on the host than on the device: 248 us at B = 1,
@@ -53,10 +53,10 @@ struct Piece8 {
     }
 };
 
-// y_i = x W_i^T for a few tokens and up to four weights that share x.  A wave takes ROWS rows (of one weight) for all
-// tokens, its lanes 8 consecutive inputs each: the weights are read once, in 1 KiB runs, and bound the kernel.  ROWS rows
-// in flight per wave keep 12 to 24 KiB in flight per wave; more tokens take more rows, so that the inputs, re-read by
-// every wave from L1, stay below the weights' bytes.
+// y_i = x W_i^T for up to 8 tokens and up to four weights that share x.  A wave takes ROWS rows (of one weight) for all
+// tokens, its lanes 8 consecutive inputs each: the weights are read once, in runs of 1 KiB (fp32: 2), and bound the
+// kernel.  ROWS runs by an unroll of two are 8 KiB of weights in flight per wave at 4 rows, 16 at 8; more tokens take more
+// rows, so that the inputs, re-read by every wave from L1, stay below the weights' bytes.
 template <int DT, int NT, int ROWS>
 __global__ __launch_bounds__(256) void small_linears_kernel(SmallLinears a) {
     const int l = threadIdx.x & 63;

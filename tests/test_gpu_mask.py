@@ -1,5 +1,5 @@
-"""GPU parity of masked calls on the chunked form (two chunked passes over the effective gates plus the masked
-tokens' fix-up, gdn_mask.hip), against the fp64 oracle's masked recurrence (tools/gdn_vjp.py:3-6, :247-256):
+"""GPU parity of masked calls on the chunked form (one chunked pass over the effective gates with the masked tokens'
+query rows, gdn_mask.hip), against the fp64 oracle's masked recurrence (tools/gdn_vjp.py:3-6, :247-256):
 the reference's sequence lengths T in {1, 63, 64, 65, 200} at Dk = Dv = 128, fp32 (1e-4) and bf16 q/k/v/dO (1e-2),
 checkpointed (chunk 256) and forward-only calls, and the measured head layout at T = 4096 against the recurrent
 form.
@@ -98,8 +98,8 @@ def test_masked_calls_select_the_chunked_form(dev):
 
 
 def test_masked_call_above_256_value_heads_runs_recurrent(dev):
-    """Hv = 260 with a mask: AUTO resolves to the recurrent form (the fix-up kernels of the chunked form hold at most
-    256 heads of a token), and the result matches the oracle on two key-head groups."""
+    """Hv = 260 with a mask: AUTO resolves to the recurrent form (mask_query_kernel has a thread per value head, at
+    most 256), and the result matches the oracle on two key-head groups."""
     import gdn_lib as L
     lib = L.load()
     assert lib.gdn_select_form(260, 128, 128, 1, L.GATE_LOG, L.FORM_AUTO, L.F32) == L.FORM_RECURRENT
@@ -129,7 +129,7 @@ def test_masked_chunked_decay_gate_and_null_cotangent(dev, log_gate):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_masked_checkpointed_against_oracle(dev, dtype):
-    """chunk = 256: the forward keeps pass 1's window states only; the backward rebuilds both passes from them."""
+    """chunk = 256: the forward keeps the window states and the query rows; the backward rebuilds the tiles from them."""
     bf = dtype == torch.bfloat16
     d = _inputs(2, 600, 2, 4, seed=55, bf16=bf)
     got = _gpu(d, dev, chunk=256, dtype=dtype)

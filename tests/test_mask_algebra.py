@@ -1,7 +1,7 @@
-"""The decomposition the chunked form uses for masked steps, checked on the CPU against the oracle's masked
-recurrence (tools/gdn_vjp.py:3-6, _step_parts :238-256): two unmasked passes over the effective gates
-(decay 1 and beta 0 where the mask is 0), the second with k as the query, an elementwise fix-up of y at masked
-tokens, and the fix-up's VJP feeding the two passes' backwards (gdn_mask.hip states the formulas).  Float64,
+"""A second derivation of the oracle's masked recurrence (tools/gdn_vjp.py:3-6, _step_parts :238-256), on the CPU: two
+unmasked passes over the effective gates (decay 1 and beta 0 where the mask is 0), the second with k as the query, an
+elementwise fix-up of y at masked tokens, and the fix-up's VJP feeding the two passes' backwards.  It pins the oracle that
+the masked kernels are compared with; the kernels' own form, one pass with query rows, is in test_mask_query.py.  Float64,
 every output of forward and VJP, scalar decay and log-decay gates, GQA 2:1, with and without an initial state.
 """
 
