@@ -489,7 +489,13 @@ def main():
     if "ops" in w:
         # streaming kernels: the bytes the launch must read and write, against the HBM roof
         a_bytes, a_flops = km(dom)[1] / tokens, {"none": 0}
-    roofline = roof(a_bytes * launch_tokens, sum(a_flops.values()) * launch_tokens, a_peak, avg_ms * 1e-3)
+    # a kernel of the recurrence is charged with its own share of the step's algorithmic work, split in proportion to the
+    # implementation model of the step's kernels (the step as a whole: `step`)
+    models = {n: km(n) for n in kt if n.startswith(("ck_", "rec_"))}
+    f_share, b_share = ((models[dom][i] / sum(m[i] for m in models.values()) if models.get(dom, (0, 0))[i] else 1.0)
+                        for i in (0, 1))
+    own_bytes, own_flops = a_bytes * launch_tokens * b_share, sum(a_flops.values()) * launch_tokens * f_share
+    roofline = roof(own_bytes, own_flops, a_peak, avg_ms * 1e-3)
     traffic = None
     tj = ROOT / "profiles" / "traffic.json"
     if tj.exists():
@@ -504,8 +510,7 @@ def main():
         "traffic": traffic, "traffic_source": "profiles/traffic.json (rocprofv3 FETCH_SIZE + WRITE_SIZE)"
         if traffic else None, "kernel": dom, "avg_launch_ms": round(avg_ms, 4),
         "algo_bytes_per_token": a_bytes, "algo_flops_per_token": a_flops, "tokens_per_launch": launch_tokens,
-        "algo_bytes_per_launch": a_bytes * launch_tokens,
-        "algo_flops_per_launch": sum(a_flops.values()) * launch_tokens,
+        "algo_bytes_per_launch": own_bytes, "algo_flops_per_launch": own_flops,
         # the whole step against the same roofline (a block step also runs the projections: no step roof there)
         "step": None if ("block" in w or "ops" in w) else dict(roof(a_bytes * tokens, sum(a_flops.values()) * tokens, a_peak,
                                                      step_s), ms=round(step_s * 1e3, 4)),
@@ -515,9 +520,7 @@ def main():
         # every kernel's modelled bytes per launch over its own average launch time
         "kernels_gbs": {n: round(km(n)[1] / per_step(n) / (v[0] / v[1] * 1e-3) / 1e9, 1)
                         for n, v in kt.items() if km(n)[1]}})
-    # each kernel's own share of the step's algorithmic flops (split in proportion to the implementation model's
-    # flops of the kernels) over that kernel's own time, against the same flop peak; `frac` above charges the
-    # whole step's work to the dominant kernel alone
+    # each kernel's own share of the step's algorithmic flops over that kernel's own time, against the same flop peak
     kf = {n: km(n)[0] for n in kt}
     kf_sum = sum(kf.values())
     if kf_sum and "block" not in w and "ops" not in w:
