@@ -19,7 +19,7 @@
 //
 // The first form of this path ran the recurrence twice, the second time with k as the query, around fp32 copies of
 // every output, cotangent and gradient: at B = 4, T = 4096, Hv = 32, bf16, a fifth of the tokens masked, 3.78 ms per
-// forward + VJP, with the query rows 1.91 ms (1.42 ms without a mask).  Both kernels here are bound by the rows of the
+// forward + VJP, with the query rows 1.89 ms (1.42 ms without a mask).  Both kernels here are bound by the rows of the
 // masked tokens: 43 us (forward) and 81 us (backward) of that.
 #include "gdn_common.h"
 #include "gdn_internal.h"
