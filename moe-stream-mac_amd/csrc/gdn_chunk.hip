@@ -1554,8 +1554,8 @@ __device__ __forceinline__ void bwd_local_bf16_head(const Args &a, int c, int hk
         if (mk) {
             // A masked token's dg and dbeta follow from dQ alone (mask_bwd_fix_kernel), so a chunk that holds one adds
             // what the bf16 tiles leave of the state and of an fp32 dY: dQ += dY hlo^T + dYlo h^T, dp += dYlo Delta^T
-            // (both lo parts straight from memory).  Without, dg of the masked tokens was off
-            // by 1.7e-3 of its norm, with 1e-4 (B = 2, T = 512, one token in five masked, fp32 dY).
+            // (both lo parts straight from memory).  Without, dg of the masked tokens was off by 1.7e-3 of its norm, with
+            // 2e-4 (B = 2, T = 512, one token in five masked, fp32 dY).
             const int x = opaque(l);
             const bfr *hl = a.w.HLb + ci * D * D + frag_off<D>(64 * ch, 0) + 8 * x;
             const float *ys = static_cast<const float *>(a.dy) + v0 + (size_t)min(r0 + (x & 15), n - 1) * v_row + 8 * (x >> 4);
@@ -1830,15 +1830,15 @@ __global__ __launch_bounds__(NTB) void ck_bwd_local_bf16_kernel(Args a) {
 // (with the reading ahead that the registers leave room for), ck_fwd_bf16 350 -> 335 us at B = 4, T = 4096, Hv = 32; 152
 // -> 142 and 166 -> 142 us at B = 1, T = 4001.
 
-// Reading ahead.  The D / VS workgroups of a head ask for the same tiles at the same time,
-// so a line that is not in L2 yet is missed by each of them, and the loads of the next chunk, issued one step ahead,
-// come back late: with tiles that outgrow the Infinity Cache a step took 3.0 us against 1.7 us within it.  Each slice
-// therefore reads one 4-byte word of its own share (1 / (D / VS)) of the shared lines of the chunk kReadAhead steps on
-// (at most one load per thread and step), so each line leaves memory once and the fragment loads hit L2 (the figures are
-// at kReadAheadBytes); three, four and six steps ahead gain less (170, 179, 184 us against 166 in the forward at B = 1,
-// T = 4001).  At 64-wide slices the backward takes it and the forward has no use for it (335 us with and without at B = 4,
-// T = 4096); masked (343 -> 363 us) and per-channel launches of that width have no registers for it.  Args::read_ahead says
-// whether the launch's tiles outgrow the cache.
+// Reading ahead.  The D / VS workgroups of a head ask for the same tiles at the same time, so a line that is not in L2
+// yet is missed by each of them, and the loads of the next chunk, issued one step ahead, come back late: with tiles that
+// outgrow the Infinity Cache a step took 3.0 us against 1.7 us within it.  Each slice therefore reads one 4-byte word
+// of its own share (1 / (D / VS)) of the shared lines of the chunk kReadAhead steps on (at most one load per thread and
+// step), so each line leaves memory once and the fragment loads hit L2 (the figures are at kReadAheadBytes); three, four
+// and six steps ahead gain less (170, 179, 184 us against 166 in the forward at B = 1, T = 4001).  At 64-wide slices the
+// backward takes it and the forward has no use for it (335 us with and without at B = 4, T = 4096); masked (343 -> 363 us)
+// and per-channel launches of that width have no registers for it.  Args::read_ahead says whether the launch's tiles
+// outgrow the cache.
 constexpr int kReadAhead = 2, kLine = 128;  // bytes of an L2 line
 
 // A [C][D] bf16 tile of the input (row stride rs elements) by whole rows, two 16-byte pieces per thread; rows past n read
@@ -2777,9 +2777,10 @@ ChunkSizes chunk_sizes(int B, int T, int Hk, int Hv, bool bf16, bool bwd, int vg
 //                     200: 64.5 / 74.1, 76.8 / 86.5      400: 141 / 177, 144 / 171
 //   32 wide (B = 2)   100 MiB 27.1 / 27.1, 26.5 / 26.5   150: 36.5 / 37.2, 37.3 / 37.8   200: 62.8 / 64.9, 57.3 / 65.7
 //                     400: 124 / 140, 101 / 125          800: 209 / 248, 187 / 235
-//   64 wide (B = 4)   backward only                      150: 32.7 / 31.4               200: 44.3 / 51.5
+//   64 wide (B = 4)   backward only                      150: 32.7 / 31.4                200: 44.3 / 51.5
 //                     400: 81.1 / 92.3                   1600: 285 / 333
-//   masked (B = 1)    100 MiB 42.2 / 42.2, 40.7 / 39.4                                   200: 86.1 / 97.0, 85.5 / 99.6
+//   masked (B = 1)    132 MiB 42.0 / 42.1, 41.0 / 39.4   165: 51.3 / 51.3, 50.6 / 48.6   198: 61.0 / 63.5, 60.4 / 63.0
+//                     264: 86.1 / 97.0, 85.5 / 99.6
 //   per channel (1)   136 MiB 32.4 / 31.7, 36.6 / 35.2                                   204: 55.6 / 60.0, 60.3 / 68.8
 //   forward only       84 MiB (B = 1) 57.0 / 53.3        165 (1): 105 / 107              169 (2): 166 / 180
 constexpr size_t kReadAheadBytes = (size_t)168 << 20;
